@@ -377,11 +377,28 @@ int noise_rank1_expand(const noise_population_t *pop, const float *base, int64_t
 /* lowrank (eggroll.py:56-58) for any shape, in autocast's form: y[m, t, o] = bf16(x[m, t, :] . w[o, :]) +
  * sign[m] * bf16(x[m, t, :] . bf16(b[m/dir_div, :])) * a[m/dir_div, o], fp32 accumulation, y fp32
  * [members][tokens][n_out]. x bf16 through the strided view (element (m, t, k) at x + m*sm + t*st + k),
- * w bf16 [n_out][n_in]. Serves the call sites whose shapes the MFMA tiles of noise_pop_linear do not take,
- * e.g. the value-embedding gate linear('attn.ve_gate.weight', h[..., :32]) (eggroll.py:88 via :80): w [8, 32]
- * on a 32-wide slice of a 512-wide row. One thread per output element. */
+ * w bf16 [n_out][n_in]. One launch with no workspace, on the vector units: for a few outputs, e.g. the
+ * value-embedding gate linear('attn.ve_gate.weight', h[..., :32]) (eggroll.py:88 via :80). */
 int noise_lowrank_rows(const noise_population_t *pop, noise_view_t x, int64_t n_in, const void *w, int64_t n_out,
                        const noise_rank1_t *r1, float *y, noise_stream_t stream);
+
+/* As noise_lowrank_rows with x and w each fp32 (x_fp32 / w_fp32 != 0, rounded to bf16 as they are read) or bf16. */
+int noise_lowrank_narrow(const noise_population_t *pop, noise_view_t x, int x_fp32, int64_t n_in, const void *w,
+                         int w_fp32, int64_t n_out, const noise_rank1_t *r1, float *y, noise_stream_t stream);
+
+/* The matrix-core form of lowrank in two calls. noise_lowrank_operands: xb [members * tokens][k_pad] and wb
+ * [n_out + b_rows][k_pad] as bf16 rows, zeros past n_in (k_pad: n_in in whole 64s), from x (fp32 or bf16, strided
+ * view) and w (fp32 or bf16 [n_out][n_in]); dots[m*tokens + t] = x[m, t] . bf16(b[m/dir_div]) when dots is given;
+ * b's first b_rows rows follow w's. xb NULL: x is left as it is.
+ * noise_lowrank_product: the products of rows x [rows][ldx] with w [N][K], each rounded to bf16 and stored fp32:
+ * features < split to y [rows][split], the others to y2 [rows][ld2]; with r1 (rows = members * tokens, split = N)
+ * plus sign[m] * bf16(dots) * a. pop gives the members of the rows (tokens, dir_div, sign). */
+int noise_lowrank_operands(const noise_population_t *pop, noise_view_t x, int x_fp32, int64_t n_in, const void *w,
+                           int w_fp32, int64_t n_out, const float *b, int64_t b_stride, int64_t b_rows, int64_t k_pad,
+                           void *xb, void *wb, float *dots, noise_stream_t stream);
+int noise_lowrank_product(const noise_population_t *pop, const void *x, int64_t ldx, int64_t rows, const void *w,
+                          int64_t K, int64_t N, const noise_rank1_t *r1, const float *dots, float *y, int64_t split,
+                          float *y2, int64_t ld2, noise_stream_t stream);
 
 /* ---- DUST --------------------------------------------------------------------------------------------- */
 

@@ -457,36 +457,6 @@ __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y,
     }
 }
 
-// lowrank (eggroll.py:56-58) for shapes the MFMA tiles do not take, such as the value-embedding gate's
-// [8, 32] weight applied to h[..., :32] (eggroll.py:88):
-//   y[m, t, o] = bf16(x[m, t] . W[o]) + sign[m] * bf16(x[m, t] . bf16(b[dir])) * a[dir, o]
-// with fp32 accumulation and the two products rounded to bf16 as autocast's matmuls return them (b enters
-// the matmul rounded, a multiplies in fp32); y fp32 [m][T][out]. One thread per output element.
-__global__ __launch_bounds__(256) void lowrank_rows_kernel(int tokens, int n_in, int n_out, int dir_div,
-                                                           const __bf16 *x, int64_t xs_m, int64_t xs_t,
-                                                           const __bf16 *w, const float *a, const float *b,
-                                                           int64_t a_stride, int64_t b_stride, const float *sign,
-                                                           float *y, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) return;
-    const int64_t row = i / n_out;
-    const int o = (int)(i - row * n_out);
-    const int m = (int)(row / tokens), t = (int)(row - (int64_t)m * tokens);
-    const int dir = m / dir_div;
-    const __bf16 *xr = x + m * xs_m + (int64_t)t * xs_t;
-    const __bf16 *wr = w + (int64_t)o * n_in;
-    const float *br = a ? b + dir * b_stride : nullptr;
-    float prod = 0.f, dot = 0.f;
-    for (int k = 0; k < n_in; ++k) {
-        const float xv = (float)xr[k];
-        prod += xv * (float)wr[k];
-        if (br) dot += xv * bfr(br[k]);
-    }
-    float v = bfr(prod);
-    if (a) v += sign[m] * bfr(dot) * a[dir * a_stride + o];
-    y[i] = v;
-}
-
 }  // namespace
 }  // namespace noise
 
@@ -598,23 +568,6 @@ extern "C" int noise_pop_gate(const noise_population_t *pop, noise_view_t x, con
                        pop->sign, noisy ? gate_noise->a : nullptr, noisy ? gate_noise->b : nullptr,
                        noisy ? gate_noise->a_stride : 0, noisy ? gate_noise->b_stride : 0, gates,
                        (int)(pop->rounding == NOISE_ROUNDING_EAGER));
-    return launch_status(fn);
-}
-
-extern "C" int noise_lowrank_rows(const noise_population_t *pop, noise_view_t x, int64_t n_in, const void *w,
-                                  int64_t n_out, const noise_rank1_t *r1, float *y, noise_stream_t stream) {
-    clear_error();
-    const char *fn = "noise_lowrank_rows";
-    NOISE_CHECK_ARG(pop && pop->members > 0 && pop->tokens > 0 && pop->dir_div >= 1, "%s: bad population", fn);
-    NOISE_CHECK_ARG(x.ptr && w && y && n_in > 0 && n_out > 0, "%s: NULL pointer or empty shape", fn);
-    NOISE_CHECK_ARG(pop->members * pop->tokens * n_out < (1ll << 38), "%s: output too large", fn);
-    const bool noisy = r1 && r1->a;
-    NOISE_CHECK_ARG(!noisy || (pop->sign && r1->b), "%s: noise needs sign and b rows", fn);
-    const int64_t total = pop->members * pop->tokens * n_out;
-    hipLaunchKernelGGL(lowrank_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       (int)pop->tokens, (int)n_in, (int)n_out, (int)pop->dir_div, (const __bf16 *)x.ptr, x.sm, x.st,
-                       (const __bf16 *)w, noisy ? r1->a : nullptr, noisy ? r1->b : nullptr,
-                       noisy ? r1->a_stride : 0, noisy ? r1->b_stride : 0, pop->sign, y, total);
     return launch_status(fn);
 }
 

@@ -57,10 +57,11 @@ struct Mma {
     __device__ static int swz(int r, int c) { return c ^ ((r / RPB) % CPR); }
 
     // W: BN rows of stride ldw; X: BM rows of stride ldx (elements, multiples of 8; 16 B aligned bases);
-    // K a multiple of BK
-    template <class Tail = NoTail>
+    // K a multiple of BK. CLAMP: rows past wlast / xlast read that last row instead (a ragged edge's tile)
+    template <bool CLAMP = false, class Tail = NoTail>
     __device__ static void run(const __bf16 *W, int64_t ldw, const __bf16 *X, int64_t ldx, int K, void *lds_v,
-                               f32x16 (&acc)[4][2], int tid, int wn, int wm, Tail tail = Tail{}) {
+                               f32x16 (&acc)[4][2], int tid, int wn, int wm, Tail tail = Tail{}, int wlast = BN - 1,
+                               int xlast = BM - 1) {
         constexpr bool kTail = !__is_same(Tail, NoTail);
         char *lds = static_cast<char *>(lds_v);
         const int lane = tid & 63, j = lane & 31, hf = lane >> 5;
@@ -79,6 +80,16 @@ struct Mma {
         const int rl = wave * RPI + lane / CPR;
         const int cl = swz(rl, lane % CPR);
         const unsigned offw = (unsigned)(rl * ldw * 2 + cl * 16), offx = (unsigned)(rl * ldx * 2 + cl * 16);
+        // CLAMP: the copies' row steps are no longer uniform, so each keeps its own lane offset
+        unsigned offc[CLAMP ? NI : 1];
+        if constexpr (CLAMP) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int r = (i < IW ? i : i - IW) * STEP + rl;
+                offc[i] = i < IW ? (unsigned)((r < wlast ? r : wlast) * (int)ldw * 2 + cl * 16)
+                                 : (unsigned)((r < xlast ? r : xlast) * (int)ldx * 2 + cl * 16);
+            }
+        }
         // fragment rows wn + 32 fb + j and BN + wm + 32 tb + j share the swizzle of row j
         static_assert(32 % (RPB * CPR) == 0 && BN % (RPB * CPR) == 0, "fragment swizzle depends on j only");
         int lo[SPK];
@@ -89,7 +100,9 @@ struct Mma {
             const unsigned st = lbase + (p % NS) * STAGE + wave * 1024;
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                if (i < IW)
+                if constexpr (CLAMP)
+                    lds_dma16_at((i < IW ? W : X) + p * BK, offc[i], st + i * NW * 1024);
+                else if (i < IW)
                     lds_dma16_at(W + (int64_t)(i * STEP) * ldw + p * BK, offw, st + i * NW * 1024);
                 else
                     lds_dma16_at(X + (int64_t)((i - IW) * STEP) * ldx + p * BK, offx, st + i * NW * 1024);

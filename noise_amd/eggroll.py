@@ -577,10 +577,11 @@ def lowrank_eager(x, weight, a, b, sign, dir_div=1):
 
     a [dirs, out], b [dirs, in] fp32 rows, member m uses row m // dir_div; sign [m]. Returns fp32
     [m, T, out] in autocast's form (the reference calls it under torch.autocast, eggroll.py:144): the
-    product x W^T and the dot x . b are bf16, the rank-1 term is added in fp32. Any shape is served: in a
-    multiple of 512 with out and T multiples of 256 run on the MFMA tiles (x broadcast over members, stride 0
-    in dim 0, is multiplied once and the rank-1 terms streamed out); other shapes, such as the value-embedding
-    gate's [8, 32] weight on h[..., :32] (eggroll.py:88), on noise_lowrank_rows. x may be a strided view."""
+    product x W^T and the dot x . b are bf16, the rank-1 term is added in fp32. Any shape and strides are
+    served. A few outputs of a short contraction (the value-embedding gate's [8, 32] weight on h[..., :32],
+    eggroll.py:88) are one launch on the tensors as they are; otherwise one pass makes the bf16 operands (and
+    the dots) and one runs the MFMA tiles. With x broadcast over members (stride 0 in dim 0) x W^T and the
+    directions' dots are one product over the shared rows, and the members' outputs are streamed from it."""
     m, T, n_in = x.shape
     n_out = weight.shape[0]
     dev = x.device
@@ -590,51 +591,62 @@ def lowrank_eager(x, weight, a, b, sign, dir_div=1):
     if a.shape[0] * dir_div < m or b.shape[0] * dir_div < m:
         raise ValueError(f'lowrank: {a.shape[0]} noise rows cannot serve {m} members at dir_div {dir_div}')
     sign = sign.to(device=dev, dtype=F32).contiguous()
-    ok = lambda t: t.dtype == F32 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.stride(0) % 4 == 0
-    a = a if ok(a) else a.float().contiguous()
-    b = b.to(BF16).to(F32).contiguous()   # autocast rounds b to bf16 for the x . b matmul
-    r1 = _rank1((a, b))
-    stream = _lib.stream_ptr(dev)
-    w = weight.to(device=dev, dtype=BF16).contiguous()
+    if a.dtype != F32 or a.stride(-1) != 1:
+        a = a.float().contiguous()
+    if b.dtype != F32:
+        b = b.to(BF16).to(F32)   # autocast rounds b to bf16 for the x . b matmul; the kernels round fp32 rows
+    if b.stride(-1) != 1:
+        b = b.contiguous()
+    w = weight.to(device=dev)
+    if w.dtype not in (F32, BF16):
+        w = w.to(BF16)
+    w = w.contiguous()
     shared = x.stride(0) == 0
-    xb = (x[:1] if shared else x).to(BF16)
-    pop = _pop(m, T, sign, dir_div)
-    y = torch.empty(m, T, n_out, dtype=F32, device=dev)
-    if n_in % 512 or n_out % 256 or T % 256:
-        # shapes outside the MFMA tiles: one thread per output element
-        if xb.stride(-1) != 1:
-            xb = xb.contiguous()
-        _lib.call('noise_lowrank_rows', ctypes.byref(pop), _lib.View(xb.data_ptr(), 0 if shared else xb.stride(0),
-                                                                      xb.stride(1)),
-                  n_in, w.data_ptr(), n_out, ctypes.byref(r1), y.data_ptr(), stream)
-        return y
-    if xb.stride(-1) != 1 or xb.stride(1) % 8 or xb.data_ptr() % 16 or (not shared and xb.stride(0) % 8):
+    xb = x[:1] if shared else x
+    if xb.dtype not in (F32, BF16):
+        xb = xb.to(BF16)
+    if xb.stride(-1) != 1:
         xb = xb.contiguous()
-    if shared:
-        # x is the same for every member, so x W^T and the dots x . b (one per direction) are computed once,
-        # as two products over the shared rows (the b rows as a bf16 weight, padded to the 256-row tile); the
-        # members' outputs are then a rank-1 expansion
-        xv = _lib.View(xb.data_ptr(), 0, xb.stride(1))
-        one = _pop(1, T, None, 1)
-        base = torch.empty(1, T, n_out, dtype=F32, device=dev)
-        _lib.call('noise_pop_linear', ctypes.byref(one), xv, w.data_ptr(), n_in, n_out, None, None, base.data_ptr(),
-                  _lib.LINEAR_AUTOCAST, T * n_out, n_out, stream)
-        dirs = -(-m // dir_div)
-        dpad = -(-dirs // 256) * 256
-        bw = torch.zeros(dpad, n_in, dtype=BF16, device=dev)
-        bw[:dirs] = b[:dirs]  # b holds bf16 values already: exact
-        dots = torch.empty(T, dpad, dtype=F32, device=dev)
-        _lib.call('noise_pop_linear', ctypes.byref(one), xv, bw.data_ptr(), n_in, dpad, None, None, dots.data_ptr(),
-                  _lib.LINEAR_AUTOCAST, T * dpad, dpad, stream)
-        _lib.call('noise_rank1_expand', ctypes.byref(pop), base.data_ptr(), n_out, dots.data_ptr(), dpad,
-                  ctypes.byref(r1), y.data_ptr(), _lib.LINEAR_AUTOCAST, stream)
+    stream = _lib.stream_ptr(dev)
+    pop = _pop(m, T, sign, dir_div)
+    x_fp32, w_fp32 = int(xb.dtype == F32), int(w.dtype == F32)
+    xv = _lib.View(xb.data_ptr(), 0 if shared else xb.stride(0), xb.stride(1))
+    y = torch.empty(m, T, n_out, dtype=F32, device=dev)
+    if n_out <= 16 and n_in <= 256 or n_in > 1 << 21:
+        # one launch: two (operands, product) cost more than the products of so few outputs (and the product's copies
+        # address rows of up to 2^21 elements)
+        r1 = _lib.Rank1(a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0))
+        _lib.call('noise_lowrank_narrow', ctypes.byref(pop), xv, x_fp32, n_in, w.data_ptr(), w_fp32, n_out,
+                  ctypes.byref(r1), y.data_ptr(), stream)
         return y
-    dots = torch.empty(m * T, dtype=F32, device=dev)
-    _lib.call('noise_member_dots', ctypes.byref(pop), _lib.View(xb.data_ptr(), xb.stride(0), xb.stride(1)), n_in,
-              ctypes.byref(r1), 1, dots.data_ptr(), stream)
-    _lib.call('noise_pop_linear', ctypes.byref(pop), _lib.View(xb.data_ptr(), xb.stride(0), xb.stride(1)), w.data_ptr(),
-              n_in, n_out, ctypes.byref(r1), dots.data_ptr(), y.data_ptr(), _lib.LINEAR_AUTOCAST, T * n_out,
-              n_out, stream)
+    if shared and n_out % 4 == 0:
+        if a.data_ptr() % 16 or a.stride(0) % 4:
+            a = torch.empty(a.shape, dtype=F32, device=a.device).copy_(a)
+        dirs = -(-m // dir_div)
+        one, rows, extra = _pop(1, T, None, 1), T, dirs
+    else:
+        one, rows, extra = pop, m * T, 0
+    kp = -(-n_in // 64) * 64
+    flat = extra or m == 1 or (not shared and xb.stride(0) == T * xb.stride(1))
+    direct = (not x_fp32 and kp == n_in and flat and xb.stride(1) % 8 == 0 and xb.stride(1) <= 1 << 21
+              and xb.data_ptr() % 16 == 0)
+    xo = None if direct else torch.empty(rows, kp, dtype=BF16, device=dev)
+    wo = torch.empty(n_out + extra, kp, dtype=BF16, device=dev)
+    dots = torch.empty(rows, -(-extra // 4) * 4 if extra else 1, dtype=F32, device=dev)
+    _lib.call('noise_lowrank_operands', ctypes.byref(one), xv, x_fp32, n_in, w.data_ptr(), w_fp32, n_out, b.data_ptr(),
+              b.stride(0), extra, kp, _lib.ptr(xo), wo.data_ptr(), None if extra else dots.data_ptr(), stream)
+    xp, ldx = (xb.data_ptr(), xb.stride(1)) if direct else (xo.data_ptr(), kp)
+    r1 = _lib.Rank1(a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0))
+    if not extra:
+        _lib.call('noise_lowrank_product', ctypes.byref(pop), xp, ldx, rows, wo.data_ptr(), kp, n_out,
+                  ctypes.byref(r1), dots.data_ptr(), y.data_ptr(), n_out, None, 0, stream)
+        return y
+    base = torch.empty(T, n_out, dtype=F32, device=dev)
+    pad = dots.shape[1]
+    _lib.call('noise_lowrank_product', ctypes.byref(one), xp, ldx, T, wo.data_ptr(), kp, n_out + extra, None, None,
+              base.data_ptr(), n_out, dots.data_ptr(), pad, stream)
+    _lib.call('noise_rank1_expand', ctypes.byref(pop), base.data_ptr(), n_out, dots.data_ptr(), pad, ctypes.byref(r1),
+              y.data_ptr(), _lib.LINEAR_AUTOCAST, stream)
     return y
 
 

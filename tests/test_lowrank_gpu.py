@@ -1,0 +1,71 @@
+"""lowrank (eggroll.py:56-58) at the edges of its kernels: tile remainders of rows, outputs and contraction, the
+one-launch form for few outputs, the tile sizes' rule, and the strides, dtypes and alignments the operands pass
+reads. Against the formula in fp32 on bf16 operands; a product's or dot's bf16 rounding may go the other way where two
+fp32 sums straddle a boundary, so the bound is one bf16 ulp of each plus the sums' order error (2^-20 of the terms)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device('cuda', 0)
+
+
+def check(x, w, a, b, sign, div):
+    from noise_amd.eggroll import lowrank
+    m = x.shape[0]
+    got = lowrank(x, w, a, b, sign, dir_div=div)
+    bf = lambda t: t.bfloat16().float()
+    d = torch.arange(m, device=DEV) // div
+    xr, wr, br, ar = bf(x), bf(w), bf(b)[d], a.float()[d]
+    prod = torch.stack([xr[i] @ wr.t() for i in range(m)])
+    dot = (xr * br[:, None, :]).sum(-1, keepdim=True)
+    s = sign[:, None, None]
+    ref = bf(prod) + s * bf(dot) * ar[:, None, :]
+    size = torch.stack([xr[i].abs() @ wr.abs().t() for i in range(m)])
+    dsize = (xr * br[:, None, :]).abs().sum(-1, keepdim=True)
+    bound = (prod.abs() * 2.0 ** -7 + size * 2.0 ** -20
+             + (s * ar[:, None, :]).abs() * (dot.abs() * 2.0 ** -7 + dsize * 2.0 ** -20) + 1e-30)
+    assert got.shape == ref.shape and got.dtype == torch.float32
+    assert ((got - ref).abs() <= bound).all()
+
+
+def inputs(m, T, n_in, n_out, div, dtype, seed):
+    g = torch.Generator(DEV).manual_seed(seed)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    dirs = -(-m // div)
+    return r(m, T, n_in).to(dtype), r(n_out, n_in) * 0.2, r(dirs, n_out), r(dirs, n_in), r(m) * 0.3
+
+
+@pytest.mark.parametrize('m,T,n_in,n_out', [
+    (1, 1, 1, 1), (3, 5, 33, 7), (2, 33, 256, 16), (2, 17, 257, 16), (5, 51, 64, 17), (1, 127, 65, 20),
+    (1, 128, 63, 128), (3, 43, 512, 129), (2, 129, 192, 260), (4, 256, 512, 256), (9, 911, 128, 2049),
+    (16, 256, 320, 4096)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_lowrank_edges(m, T, n_in, n_out, dtype):
+    print(m, T, n_in, n_out, dtype, flush=True)
+    x, w, a, b, sign = inputs(m, T, n_in, n_out, 2, dtype, m + T)
+    check(x, w, a, b, sign, 2)
+    check(x, w.bfloat16(), a, b, sign, 2)
+    check(x[:1].expand(m, T, n_in), w, a, b, sign, 2)  # shared over the members
+
+
+def test_lowrank_views():
+    x, w, a, b, sign = inputs(6, 40, 512, 96, 1, torch.float32, 3)
+    bf = x.bfloat16()
+    wide = torch.randn(6, 40, 1031, device=DEV)
+    cases = dict(columns=x[..., 64:192], odd_columns=wide[..., 3:131], every_other=bf[:, ::2], transposed=bf.transpose(0, 1),
+                 inner=x.transpose(1, 2), tokens_expanded=bf[:, :1].expand(6, 40, 512), misaligned=wide.bfloat16()[..., 1:513],
+                 members_reversed=bf.flip(0)[::2], half=x.half())
+    for name, v in cases.items():
+        print(name, tuple(v.shape), v.stride(), flush=True)
+        m, T, n_in = v.shape
+        for div in (1, 3):
+            s = torch.randn(m, device=DEV) * 0.3
+            aa, bb = torch.randn(m, 96, device=DEV), torch.randn(m, n_in, device=DEV)
+            check(v, torch.randn(96, n_in, device=DEV) * 0.2, aa, bb, s, div)
+    rows = torch.randn(6, 96 + 512 + 3, device=DEV)
+    check(x, w, rows[:, :96], rows[:, 96:608], sign, 1)        # noise as column views of one table
+    check(x, w, rows[:, 1:97], rows[:, 98:610], sign, 1)       # off the 16 B alignment
+    check(x[:1].expand(6, 40, 512), w, rows[:, 1:97], rows[:, 98:610], sign, 1)
+    check(x, w.t().contiguous().t(), a.bfloat16(), b.half(), sign, 1)
+    check(x.transpose(1, 2)[:1].expand(6, 512, 40), torch.randn(18, 40, device=DEV), torch.randn(6, 18, device=DEV),
+          torch.randn(6, 40, device=DEV), sign, 1)             # shared, no unit inner stride, outputs off the groups of 4
