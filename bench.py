@@ -53,7 +53,7 @@ def kernel_flops_per_launch(name, label, members, T):
         return 2 * (512 * 512 + 2 * 512 * 2048) * rows
     if name == 'noise_pop_block_qkv':
         return 2 * (512 * 512 + 2 * 512 * 2048 + 512 * 1536) * rows
-    if name == 'noise_pop_head_ce':
+    if name in ('noise_pop_head_ce', 'noise_head_ce'):
         return 2 * 512 * 4096 * rows
     if name == 'noise_attention_fwd':
         window = int(label.split()[-1])

@@ -255,6 +255,15 @@ int noise_pop_head_ce(const noise_population_t *pop, noise_view_t x, const void 
                       const noise_rank1_t *r1, const float *dots, const int64_t *targets, int64_t targets_sm,
                       float *token_loss, noise_stream_t stream);
 
+/* The same for K = 512 or 1536 and any number of tokens, with a workspace: where the token tiles leave CUs idle, the
+ * vocabulary of a tile is shared out over several workgroups, whose sums meet in the workspace in a fixed order.
+ * x_fp32 (K = 1536, unperturbed): x is fp32 [T][512] rows, split as they are read and normed in the logits.
+ * noise_head_ce_workspace_bytes: the bytes to give (0: none; workspace NULL always runs unsplit; negative: invalid). */
+int64_t noise_head_ce_workspace_bytes(int64_t members, int64_t tokens, int64_t K, int64_t vocab);
+int noise_head_ce(const noise_population_t *pop, noise_view_t x, int x_fp32, const void *w, int64_t K, int64_t vocab,
+                  const noise_rank1_t *r1, const float *dots, const int64_t *targets, int64_t targets_sm,
+                  float *token_loss, void *workspace, int64_t workspace_bytes, noise_stream_t stream);
+
 /* The block's whole MLP with its residual writer (eggroll.py:93, then the next block's mixing, eggroll.py:77-79,
  * and what noise_pop_residual derives from the new residual): with x = h (bf16, the norm of the block's mid
  * residual) and per member m,

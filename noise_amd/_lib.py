@@ -44,3 +44,11 @@ def stream_ptr(device=None):
 def ptr(t):
     """Device address of a tensor (None -> NULL)."""
     return None if t is None else t.data_ptr()
+
+
+def head_workspace(members, tokens, K, vocab, device):
+    """(tensor or None, bytes) of noise_head_ce's workspace for these sizes."""
+    need = lib().noise_head_ce_workspace_bytes(members, tokens, K, vocab)
+    if need < 0:
+        raise RuntimeError(lib().noise_last_error().decode(errors='replace'))
+    return (torch.empty(need, dtype=torch.uint8, device=device) if need else None), need

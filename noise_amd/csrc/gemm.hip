@@ -810,7 +810,46 @@ struct HeadArgs {
     const int64_t *targets;   // [T] shared by all members, or [m][T] when targets_sm != 0
     int64_t targets_sm;
     float *loss;              // [m][T] per-token CE (0 where target == -1, NaN for targets outside [0, vocab))
+    int parts;                // workgroups that share a token tile's vocabulary
+    float2 *partial;          // parts > 1: [vocab / 128][m T] (sum of e^(z - 15), target's logit or 0)
 };
+
+// A token's sum of e^(z - 15) is formed per segment of 128 vocabulary rows and the segments' sums are added in order,
+// in one workgroup or over several: a loss has the same bits whatever number of workgroups shares its tile.
+constexpr int kHeadSegment = 128;
+
+// the segments of part `part`: as even as whole segments allow
+struct HeadSpan {
+    int first, end;
+};
+__device__ __forceinline__ HeadSpan head_span(int segments, int parts, int part) {
+    return {segments * part / parts, segments * (part + 1) / parts};
+}
+
+// the loss of a token from its sum of e^(z - 15) and its target's logit: ignore_index -1 contributes 0, any other
+// id outside [0, vocab) is an error, reported as NaN
+__device__ __forceinline__ float head_token_loss(float sum, float zl, int64_t tgt, int vocab) {
+    const float k1 = (2.0f / 15.0f) * kLog2e;
+    const float z = 15.0f - 30.0f / (exp2_fast(zl * k1) + 1.0f);
+    const float ce = 15.0f + __logf(sum) - z;
+    return tgt == -1 ? 0.f : (tgt < 0 || tgt >= vocab ? __builtin_nanf("") : ce);
+}
+
+// The split head's end: a token's segments summed in order. The shift of the exponents is fixed, so the sums add.
+// One wave per workgroup and many loads in flight: a few thousand rows are all latency.
+__global__ __launch_bounds__(64) void head_combine_kernel(HeadArgs p, int64_t rows) {
+    const int64_t row = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (row >= rows) return;
+    float sum = 0.f, zl = 0.f;
+#pragma unroll 16
+    for (int i = 0; i < p.vocab / kHeadSegment; ++i) {
+        const float2 v = p.partial[i * rows + row];
+        sum += v.x;
+        zl += v.y;
+    }
+    const int64_t m = row / p.pop.tokens, t = row - m * p.pop.tokens;
+    p.loss[row] = head_token_loss(sum, zl, p.targets[m * p.targets_sm + t], p.vocab);
+}
 
 // EAGER: logits rounded to bf16 before the soft cap (the autocast head's bf16 output; unperturbed calls only)
 template <bool EAGER = false>
@@ -899,11 +938,13 @@ constexpr int kHxStepBytes = kHxRows * 512 * 2;  // [8 k-tiles][64 rows][128 B]
 template <bool EAGER, bool PERT>
 __global__ __launch_bounds__(kHxThreads, 1) void head_x_kernel(HeadArgs p) {
     __shared__ __attribute__((aligned(16))) char lds[2 * kHxStepBytes];
-    const int T = p.pop.tokens, tiles_t = T / kHxTok;
-    const int m = blockIdx.x / tiles_t, t0 = (blockIdx.x % tiles_t) * kHxTok;
+    const int T = p.pop.tokens, tiles_t = (T + kHxTok - 1) / kHxTok;
+    const int tile = blockIdx.x / p.parts, part = blockIdx.x % p.parts;
+    const int m = tile / tiles_t, t0 = (tile % tiles_t) * kHxTok;
     const int tid = threadIdx.x, lane = tid & 63, jl = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tok = t0 + 32 * wave + jl;
+    const bool live = t0 + 32 * wave + jl < T;  // a ragged last tile repeats the last token, unstored
+    const int tok = live ? t0 + 32 * wave + jl : T - 1;
     const int64_t row = (int64_t)m * T + tok;
     const int dir = m / p.pop.dir_div;
     const unsigned lbase = lds_addr(lds);
@@ -919,7 +960,10 @@ __global__ __launch_bounds__(kHxThreads, 1) void head_x_kernel(HeadArgs p) {
                          dst + ci * 1024);
         }
     };
-    issue(0);
+    constexpr int kPer = kHeadSegment / kHxRows;  // steps of a segment
+    const HeadSpan span = head_span(p.vocab / kHeadSegment, p.parts, part);
+    const int js0 = span.first * kPer, js1 = span.end * kPer;
+    issue(js0);
     // this lane's token row: xf[s] = x[tok][16 s + 8 hf .. + 8], the B operand of k-step s
     bf16x8 xf[32];
     {
@@ -932,14 +976,13 @@ __global__ __launch_bounds__(kHxThreads, 1) void head_x_kernel(HeadArgs p) {
     const float *arow = PERT ? p.r1.a + dir * p.r1.a_stride + 4 * hf : nullptr;
     const float k1 = (2.0f / 15.0f) * kLog2e;     // u = 2^(k1 l) = e^(2 l / 15)
     const float c2 = 1.0f / (-30.0f * kLog2e);    // rcp(c2 (1 + u)) = -30 log2(e) / (1 + u) = log2 e^(z - 15)
-    float sum = 0.f, zl = 0.f;                    // sum of e^(z - 15) over this lane's rows; the target's logit
+    float sum = 0.f, zl = 0.f, total = 0.f;       // e^(z - 15) over this lane's rows of a segment; the target's logit
     vm_wait<0>();
     __syncthreads();
-    const int nsteps = p.vocab / kHxRows;
     f32x16 acc[2];
 #pragma unroll 1
-    for (int js = 0; js < nsteps; ++js) {
-        if (js + 1 < nsteps) issue(js + 1);  // its buffer was last read in step js - 1, before the barrier below
+    for (int js = js0; js < js1; ++js) {
+        if (js + 1 < js1) issue(js + 1);  // its buffer was last read in step js - 1, before the barrier below
         const char *buf = lds + (js & 1) * kHxStepBytes;
         auto frag = [&](int vb, int s) {
             return *reinterpret_cast<const bf16x8 *>(buf + (s >> 2) * 8192 + (32 * vb + jl) * 128 +
@@ -995,16 +1038,23 @@ __global__ __launch_bounds__(kHxThreads, 1) void head_x_kernel(HeadArgs p) {
                         if (d == 32 * vb + 8 * b + e) zl = logit(vb, 4 * b + e, a4);
                 }
         }
+        if ((js + 1) % kPer == 0) {  // a segment ends
+            sum += swap_halves(sum);
+            if (p.parts > 1) {
+                zl += swap_halves(zl);  // exactly one lane of the pair holds the target's row
+                if (hf == 0 && live)
+                    p.partial[(int64_t)(js / kPer) * p.pop.members * T + row] = float2{sum, zl};
+                zl = 0.f;
+            }
+            total += sum;
+            sum = 0.f;
+        }
         vm_wait<0>();
         __syncthreads();  // step js + 1 landed for every wave; every wave is done with buffer js & 1
     }
-    sum += swap_halves(sum);
-    zl += swap_halves(zl);  // exactly one lane of the pair holds the target's row
-    if (hf == 0) {
-        const float z = 15.0f - 30.0f / (exp2_fast(zl * k1) + 1.0f);
-        const float ce = 15.0f + __logf(sum) - z;
-        p.loss[row] = tgt == -1 ? 0.f : (tgt < 0 || tgt >= p.vocab ? __builtin_nanf("") : ce);
-    }
+    if (p.parts > 1) return;
+    zl += swap_halves(zl);
+    if (hf == 0 && live) p.loss[row] = head_token_loss(total, zl, tgt, p.vocab);
 }
 
 // The fp32 head as split-bf16x3 (K = 1536: x rows [hi | lo | hi], w rows [hi | hi | lo]), logits = x_hi w_hi +
@@ -1022,14 +1072,17 @@ constexpr int kH3Step = 2 * kH3Part;          // hi then lo
 #define HEAD3_AHEAD 4
 #endif
 
-template <bool PERT>
+// XF32: x is fp32 [T][512], its rows split here, their norm applied to the logits (the head_loss drop-in, unperturbed)
+template <bool PERT, bool XF32 = false>
 __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
     __shared__ __attribute__((aligned(16))) char lds[2 * kH3Step];
-    const int T = p.pop.tokens, tiles_t = T / kH3Tok;
-    const int m = blockIdx.x / tiles_t, t0 = (blockIdx.x % tiles_t) * kH3Tok;
+    const int T = p.pop.tokens, tiles_t = (T + kH3Tok - 1) / kH3Tok;
+    const int tile = blockIdx.x / p.parts, part = blockIdx.x % p.parts;
+    const int m = tile / tiles_t, t0 = (tile % tiles_t) * kH3Tok;
     const int tid = threadIdx.x, lane = tid & 63, tl = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tok = t0 + 16 * wave + tl;
+    const bool live = t0 + 16 * wave + tl < T;  // a ragged last tile repeats the last token, unstored
+    const int tok = live ? t0 + 16 * wave + tl : T - 1;
     const int64_t row = (int64_t)m * T + tok;
     const int dir = m / p.pop.dir_div;
     const unsigned lbase = lds_addr(lds);
@@ -1048,10 +1101,30 @@ __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
                              (unsigned)(r8 * 1536 * 2 + c * 16), dst + part * kH3Part + r0 * 128);
             }
     };
-    issue(0);
+    constexpr int kPer = kHeadSegment / kH3Rows;  // steps of a segment
+    const HeadSpan span = head_span(p.vocab / kHeadSegment, p.parts, part);
+    const int js0 = span.first * kPer, js1 = span.end * kPer;
+    issue(js0);
     // this lane's rows: xh[kb] = x_hi[tok][32 kb + 8 g .. + 8], xl[kb] the same of x_lo
     bf16x8 xh[16], xl[16];
-    {
+    float scale = 1.f;
+    if constexpr (XF32) {
+        // the raw values are split; the row's norm is a factor of its logits (every logit of a lane is one token's)
+        const float *xr = reinterpret_cast<const float *>(p.x) + m * p.xs_m + (int64_t)tok * p.xs_t + 8 * g;
+        float ss = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < 16; ++kb) {
+            const float4 u = ld4(xr + 32 * kb), v = ld4(xr + 32 * kb + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float f = e < 4 ? f4get(u, e) : f4get(v, e - 4);
+                ss += f * f;
+                xh[kb][e] = (__bf16)f;
+                xl[kb][e] = (__bf16)(f - (float)xh[kb][e]);
+            }
+        }
+        scale = rsqrtf(sum_lanes_16_32(ss) * (1.0f / 512.0f) + kEps);
+    } else {
         const __bf16 *xr = p.x + m * p.xs_m + (int64_t)tok * p.xs_t + 8 * g;
 #pragma unroll
         for (int kb = 0; kb < 16; ++kb) {
@@ -1062,17 +1135,16 @@ __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
     const int64_t tgt = p.targets[m * p.targets_sm + tok];
     const float corr = PERT ? p.pop.sign[m] * p.dots[row] : 0.f;
     const float *arow = PERT ? p.r1.a + dir * p.r1.a_stride + 4 * g : nullptr;
-    const float k1 = (2.0f / 15.0f) * kLog2e;     // u = 2^(k1 l) = e^(2 l / 15)
+    const float k1 = (2.0f / 15.0f) * kLog2e * scale;  // u = 2^(k1 l) = e^(2 l / 15)
     const float c2 = 1.0f / (-30.0f * kLog2e);    // rcp(c2 (1 + u)) = -30 log2(e) / (1 + u) = log2 e^(z - 15)
-    float sum = 0.f, zl = 0.f;                    // sum of e^(z - 15) over this lane's rows; the target's logit
+    float sum = 0.f, zl = 0.f, total = 0.f;       // e^(z - 15) over this lane's rows of a segment; the target's logit
     vm_wait<0>();
     __syncthreads();
-    const int nsteps = p.vocab / kH3Rows;
     const int fr = lane & 15, fc = lane >> 4;
     constexpr int kA = HEAD3_AHEAD;
 #pragma unroll 1
-    for (int js = 0; js < nsteps; ++js) {
-        if (js + 1 < nsteps) issue(js + 1);  // its buffer was last read in step js - 1, before the barrier below
+    for (int js = js0; js < js1; ++js) {
+        if (js + 1 < js1) issue(js + 1);  // its buffer was last read in step js - 1, before the barrier below
         const char *buf = lds + (js & 1) * kH3Step;
         // fragment f = 4 kb + 2 vb + part: rows 16 vb .. + 16 of segment part, k block kb
         auto frag = [&](int f) {
@@ -1125,21 +1197,52 @@ __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
             for (int vb = 0; vb < 2; ++vb)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (d == 16 * vb + r) zl = logit(vb, r);
+                    if (d == 16 * vb + r) zl = XF32 ? logit(vb, r) * scale : logit(vb, r);
+        }
+        if ((js + 1) % kPer == 0) {  // a segment ends
+            sum = sum_lanes_16_32(sum);
+            if (p.parts > 1) {
+                zl = sum_lanes_16_32(zl);  // exactly one of the token's four lanes holds the target's row
+                if (g == 0 && live)
+                    p.partial[(int64_t)(js / kPer) * p.pop.members * T + row] = float2{sum, zl};
+                zl = 0.f;
+            }
+            total += sum;
+            sum = 0.f;
         }
         vm_wait<0>();
         __syncthreads();  // step js + 1 landed for every wave; every wave is done with buffer js & 1
     }
-    // the four lanes of a token: sums add; exactly one of them holds the target's row (the others hold 0)
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    zl += __shfl_xor(zl, 16, 64);
-    zl += __shfl_xor(zl, 32, 64);
-    if (g == 0) {
-        const float z = 15.0f - 30.0f / (exp2_fast(zl * k1) + 1.0f);
-        const float ce = 15.0f + __logf(sum) - z;
-        p.loss[row] = tgt == -1 ? 0.f : (tgt < 0 || tgt >= p.vocab ? __builtin_nanf("") : ce);
+    if (p.parts > 1) return;
+    zl = sum_lanes_16_32(zl);
+    if (g == 0 && live) p.loss[row] = head_token_loss(total, zl, tgt, p.vocab);
+}
+
+// How many workgroups share a token tile's vocabulary sweep. One workgroup fills a CU, so a launch lasts
+// (rounds of 256) x (a part's segments + the tile's own start, about half a segment's time): with few tiles the sweep
+// is split until the CUs are busy, and a last round that would be nearly empty is evened out. 24 tiles of
+// the fp32 head (3,000 rows): 249 us on 24 workgroups, 53 on 192; 8 tiles of the bf16 head: 228 us on 8, 20 on 256.
+int head_parts(int64_t tiles, int segments) {
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int p = 1; p <= segments && p <= 32; ++p) {
+        const int64_t cost = (tiles * p + 255) / 256 * (2 * ((segments + p - 1) / p) + 1);
+        if (cost < least) {
+            least = cost;
+            best = p;
+        }
     }
+    return best;
+}
+
+// token tiles of the row-resident heads for K (0: the K loop head serves it)
+int64_t head_tiles(int64_t members, int64_t tokens, int64_t K) {
+    const int64_t tok = K == 512 ? kHxTok : K == 1536 ? kH3Tok : 0;
+    return tok ? members * ((tokens + tok - 1) / tok) : 0;
+}
+
+int64_t head_workspace(int64_t members, int64_t tokens, int64_t vocab) {
+    return vocab / kHeadSegment * members * tokens * (int64_t)sizeof(float2);
 }
 
 Pop make_pop(const noise_population_t *pp) {
@@ -1398,45 +1501,106 @@ extern "C" int noise_pop_linear(const noise_population_t *pop, noise_view_t x, c
     return launch_status(fn);
 }
 
+namespace noise {
+namespace {
+
+// the row-resident heads; workspace NULL: one workgroup per token tile
+int head_rows_launch(HeadArgs &a, const noise_population_t *pop, bool x_fp32, void *workspace, int64_t workspace_bytes,
+                     hipStream_t st, const char *fn) {
+    const int64_t rows = pop->members * pop->tokens, tiles = head_tiles(pop->members, pop->tokens, a.K);
+    a.parts = workspace ? head_parts(tiles, a.vocab / kHeadSegment) : 1;
+    const int64_t need = a.parts > 1 ? head_workspace(pop->members, pop->tokens, a.vocab) : 0;
+    NOISE_CHECK_ARG(workspace_bytes >= need, "%s: workspace of %lld B, %lld needed", fn, (long long)workspace_bytes,
+                    (long long)need);
+    NOISE_CHECK_ARG(tiles * a.parts <= INT32_MAX, "%s: too many tiles", fn);
+    a.partial = static_cast<float2 *>(workspace);
+    const dim3 grid((unsigned)(tiles * a.parts));
+    if (a.K == 512) {
+        // the bf16 head: token rows resident in registers, weights streamed once per 256 tokens
+        if (eager(pop))
+            hipLaunchKernelGGL((head_x_kernel<true, false>), grid, dim3(kHxThreads), 0, st, a);
+        else if (a.r1.a)
+            hipLaunchKernelGGL((head_x_kernel<false, true>), grid, dim3(kHxThreads), 0, st, a);
+        else
+            hipLaunchKernelGGL((head_x_kernel<false, false>), grid, dim3(kHxThreads), 0, st, a);
+    } else {
+        // the split-bf16x3 fp32 head: hi and lo token rows resident in registers, weights streamed once per 128 tokens
+        if (x_fp32)
+            hipLaunchKernelGGL((head3_kernel<false, true>), grid, dim3(kH3Threads), 0, st, a);
+        else if (a.r1.a)
+            hipLaunchKernelGGL((head3_kernel<true>), grid, dim3(kH3Threads), 0, st, a);
+        else
+            hipLaunchKernelGGL((head3_kernel<false>), grid, dim3(kH3Threads), 0, st, a);
+    }
+    NOISE_TRY(launch_status(fn));
+    if (a.parts > 1)
+        hipLaunchKernelGGL(head_combine_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, st, a, rows);
+    return launch_status(fn);
+}
+
+int head_args(const noise_population_t *pop, noise_view_t x, const void *w, int64_t K, int64_t vocab,
+              const noise_rank1_t *r1, const float *dots, const int64_t *targets, int64_t targets_sm, float *token_loss,
+              const char *fn, HeadArgs &a) {
+    NOISE_TRY(check_view(x, fn, "x"));
+    NOISE_CHECK_ARG(K > 0 && K % 64 == 0 && vocab > 0 && vocab % 256 == 0, "%s: K multiple of 64, vocab of 256", fn);
+    NOISE_CHECK_ARG(w && aligned(w, 16) && targets && token_loss, "%s: NULL w/targets/loss", fn);
+    NOISE_CHECK_ARG(!r1 || !r1->a || (dots && pop->sign), "%s: perturbation needs dots and sign", fn);
+    NOISE_CHECK_ARG(!eager(pop) || ((!r1 || !r1->a) && K == 512), "%s: eager rounding is for the unperturbed bf16 head", fn);
+    a.pop = make_pop(pop);
+    a.x = (const __bf16 *)x.ptr; a.xs_m = x.sm; a.xs_t = x.st;
+    a.w = (const __bf16 *)w; a.K = (int)K; a.vocab = (int)vocab;
+    a.r1 = make_r1(r1);
+    a.dots = dots; a.targets = targets; a.targets_sm = targets_sm; a.loss = token_loss;
+    a.parts = 1;
+    a.partial = nullptr;
+    return NOISE_OK;
+}
+
+}  // namespace
+}  // namespace noise
+
 extern "C" int noise_pop_head_ce(const noise_population_t *pop, noise_view_t x, const void *w, int64_t K,
                                  int64_t vocab, const noise_rank1_t *r1, const float *dots, const int64_t *targets,
                                  int64_t targets_sm, float *token_loss, noise_stream_t stream) {
     clear_error();
     const char *fn = "noise_pop_head_ce";
     NOISE_TRY(check_pop(pop, 256, fn));
-    NOISE_TRY(check_view(x, fn, "x"));
-    NOISE_CHECK_ARG(K > 0 && K % 64 == 0 && vocab > 0 && vocab % 256 == 0, "%s: K multiple of 64, vocab of 256", fn);
-    NOISE_CHECK_ARG(w && aligned(w, 16) && targets && token_loss, "%s: NULL w/targets/loss", fn);
-    NOISE_CHECK_ARG(!r1 || !r1->a || (dots && pop->sign), "%s: perturbation needs dots and sign", fn);
-    NOISE_CHECK_ARG(!eager(pop) || ((!r1 || !r1->a) && K == 512), "%s: eager rounding is for the unperturbed bf16 head", fn);
     HeadArgs a;
-    a.pop = make_pop(pop);
-    a.x = (const __bf16 *)x.ptr; a.xs_m = x.sm; a.xs_t = x.st;
-    a.w = (const __bf16 *)w; a.K = (int)K; a.vocab = (int)vocab;
-    a.r1 = make_r1(r1);
-    a.dots = dots; a.targets = targets; a.targets_sm = targets_sm; a.loss = token_loss;
-    dim3 grid((unsigned)(pop->members * (pop->tokens / 256)));
-    if (K == 512 && vocab % kHxRows == 0 && x.st % 8 == 0 && x.sm % 8 == 0) {
-        // the bf16 head: token rows resident in registers, weights streamed once per 256 tokens
-        if (eager(pop))
-            hipLaunchKernelGGL((head_x_kernel<true, false>), grid, dim3(kHxThreads), 0, (hipStream_t)stream, a);
-        else if (a.r1.a)
-            hipLaunchKernelGGL((head_x_kernel<false, true>), grid, dim3(kHxThreads), 0, (hipStream_t)stream, a);
-        else
-            hipLaunchKernelGGL((head_x_kernel<false, false>), grid, dim3(kHxThreads), 0, (hipStream_t)stream, a);
-    } else if (K == 1536 && !eager(pop) && vocab % kH3Rows == 0 && x.st % 8 == 0 && x.sm % 8 == 0) {
-        // the split-bf16x3 fp32 head: hi and lo token rows resident in registers, weights streamed once per 128 tokens
-        const dim3 g3((unsigned)(pop->members * (pop->tokens / kH3Tok)));
-        if (a.r1.a)
-            hipLaunchKernelGGL(head3_kernel<true>, g3, dim3(kH3Threads), 0, (hipStream_t)stream, a);
-        else
-            hipLaunchKernelGGL(head3_kernel<false>, g3, dim3(kH3Threads), 0, (hipStream_t)stream, a);
-    } else if (eager(pop)) {
+    NOISE_TRY(head_args(pop, x, w, K, vocab, r1, dots, targets, targets_sm, token_loss, fn, a));
+    if (head_tiles(pop->members, pop->tokens, K))
+        return head_rows_launch(a, pop, false, nullptr, 0, (hipStream_t)stream, fn);
+    const dim3 grid((unsigned)(pop->members * (pop->tokens / 256)));
+    if (eager(pop))
         hipLaunchKernelGGL(head_ce_kernel<true>, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
-    } else {
+    else
         hipLaunchKernelGGL(head_ce_kernel<false>, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
-    }
     return launch_status(fn);
+}
+
+extern "C" int64_t noise_head_ce_workspace_bytes(int64_t members, int64_t tokens, int64_t K, int64_t vocab) {
+    clear_error();
+    if (members <= 0 || tokens <= 0 || members >= (1ll << 31) / tokens || (K != 512 && K != 1536) || vocab <= 0 ||
+        vocab % 256) {
+        set_error("noise_head_ce_workspace_bytes: members and tokens positive, K 512 or 1536, vocab a multiple of 256");
+        return NOISE_EINVAL;
+    }
+    const int parts = head_parts(head_tiles(members, tokens, K), (int)(vocab / kHeadSegment));
+    return parts > 1 ? head_workspace(members, tokens, vocab) : 0;
+}
+
+extern "C" int noise_head_ce(const noise_population_t *pop, noise_view_t x, int x_fp32, const void *w, int64_t K,
+                             int64_t vocab, const noise_rank1_t *r1, const float *dots, const int64_t *targets,
+                             int64_t targets_sm, float *token_loss, void *workspace, int64_t workspace_bytes,
+                             noise_stream_t stream) {
+    clear_error();
+    const char *fn = "noise_head_ce";
+    NOISE_TRY(check_pop(pop, 1, fn));
+    NOISE_CHECK_ARG(K == 512 || K == 1536, "%s: K must be 512 or 1536", fn);
+    HeadArgs a;
+    NOISE_TRY(head_args(pop, x, w, K, vocab, r1, dots, targets, targets_sm, token_loss, fn, a));
+    NOISE_CHECK_ARG(!x_fp32 || (K == 1536 && !a.r1.a), "%s: fp32 rows are for the unperturbed split head", fn);
+    NOISE_CHECK_ARG(!workspace || aligned(workspace, 8), "%s: workspace misaligned", fn);
+    return head_rows_launch(a, pop, x_fp32 != 0, workspace, workspace_bytes, (hipStream_t)stream, fn);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -40,28 +40,22 @@ def head_loss_eager(x, weight, targets, vocab):
     if d != 512 or weight.shape[1] != 512 or vocab % 256 or weight.shape[0] < vocab:
         raise ValueError('head_loss: width 512 and vocab a multiple of 256 are supported')
     rows = x.numel() // d
-    pad = -rows % 256
-    xs = x.reshape(rows, d).to(F32)
-    if pad:
-        xs = torch.cat([xs, torch.zeros(pad, d, dtype=F32, device=dev)])
-    xs = xs.contiguous()
-    tg = targets.reshape(rows).to(device=dev, dtype=torch.int64)
-    if pad:
-        tg = torch.cat([tg, torch.full((pad,), -1, dtype=torch.int64, device=dev)])
-    tg = tg.contiguous()
+    xs = x.reshape(rows, d).to(F32).contiguous()
+    if xs.data_ptr() % 16:
+        xs = xs.clone()
+    tg = targets.reshape(rows).to(device=dev, dtype=torch.int64).contiguous()
     stream = _lib.stream_ptr(dev)
-    n = rows + pad
-    x3 = torch.empty(n, 3 * d, dtype=BF16, device=dev)
-    _lib.call('noise_split3', xs.data_ptr(), n, d, 1, 0, x3.data_ptr(), stream)
     w = weight[:vocab].to(device=dev, dtype=F32).contiguous()
     w3 = torch.empty(vocab, 3 * d, dtype=BF16, device=dev)
     _lib.call('noise_split3', w.data_ptr(), vocab, d, 0, 1, w3.data_ptr(), stream)
-    loss = torch.empty(n, dtype=F32, device=dev)
-    pop = _lib.Population(1, n, None, 1)
+    loss = torch.empty(rows, dtype=F32, device=dev)
+    pop = _lib.Population(1, rows, None, 1)
     none = _lib.Rank1(None, None, 0, 0)
-    _lib.call('noise_pop_head_ce', ctypes.byref(pop), _lib.View(x3.data_ptr(), 0, 3 * d), w3.data_ptr(), 3 * d, vocab,
-              ctypes.byref(none), None, tg.data_ptr(), 0, loss.data_ptr(), stream)
-    return loss[:rows]
+    ws, need = _lib.head_workspace(1, rows, 3 * d, vocab, dev)
+    # the kernel splits the fp32 rows as it reads them and norms their logits
+    _lib.call('noise_head_ce', ctypes.byref(pop), _lib.View(xs.data_ptr(), 0, d), 1, w3.data_ptr(), 3 * d, vocab,
+              ctypes.byref(none), None, tg.data_ptr(), 0, loss.data_ptr(), _lib.ptr(ws), need, stream)
+    return loss
 
 
 def coordinate_differences(raw, y, sigma):

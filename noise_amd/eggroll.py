@@ -192,6 +192,18 @@ class _Buffers:
         self.loss_tok = torch.empty(rows, dtype=F32, device=dev)
 
 
+def _head(popp, m, T, hx, hw, K, r1, B, targets, targets_sm, dev, stream):
+    """The head's per-token losses into B.loss_tok: its vocabulary shared out over several workgroups per token
+    tile (with a workspace for their sums) where the tiles leave CUs idle."""
+    ws, need = _lib.head_workspace(m, T, K, VOCAB, dev)
+    args = (hw.data_ptr(), K, VOCAB, ctypes.byref(r1), B.d_head.data_ptr(), targets.data_ptr(), targets_sm,
+            B.loss_tok.data_ptr())
+    if need:
+        _call('noise_head_ce', popp, hx, 0, *args, ws.data_ptr(), need, stream)
+    else:
+        _call('noise_pop_head_ce', popp, hx, *args, stream)
+
+
 _ZERO_ROWS = {}
 
 
@@ -398,8 +410,7 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
         hx, hw, K = _view(B.h3, T * 3 * E, 3 * E), W.lm_head3, 3 * E
     else:
         hx, hw, K = _view(B.h, T * E, E), W.lm_head, E
-    _call('noise_pop_head_ce', popp, hx, hw.data_ptr(), K, VOCAB, ctypes.byref(head_r1), B.d_head.data_ptr(),
-              targets.data_ptr(), idx_sm, B.loss_tok.data_ptr(), stream)
+    _head(popp, m, T, hx, hw, K, head_r1, B, targets, idx_sm, dev, stream)
     if per_token:
         return B.loss_tok.view(m, T)
     out = torch.empty(m, dtype=F32, device=dev)
@@ -526,8 +537,7 @@ def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=No
         hx, hw, K = _view(B.h3, T * 3 * E, 3 * E), W.lm_head3, 3 * E
     else:
         hx, hw, K = _view(B.h, T * E, E), W.lm_head, E
-    _call('noise_pop_head_ce', popp, hx, hw.data_ptr(), K, VOCAB, ctypes.byref(none), B.d_head.data_ptr(),
-          targets.data_ptr(), T, B.loss_tok.data_ptr(), stream)
+    _head(popp, m, T, hx, hw, K, none, B, targets, T, dev, stream)
     return B.loss_tok.view(m, T)
 
 
