@@ -57,6 +57,18 @@ int noise_normal_fill(float *out, int64_t n, int64_t first, uint64_t seed, uint6
 int noise_randint(int64_t *out, int64_t n, uint64_t seed, uint64_t offset, int64_t threads, uint64_t range,
                   int64_t base, noise_stream_t stream);
 
+/* Several randint draws of n values each in one launch (Eggroll.offsets: one draw per parameter, eggroll.py:117-120):
+ * out[k * n + i] = (u32 element i of the draw at (seed, offset[k], threads)) % range[k], k < count. The descriptor is
+ * passed by value to the kernel. */
+#define NOISE_RANDINT_SETS_MAX 64
+typedef struct {
+    int32_t count;
+    uint64_t offset[NOISE_RANDINT_SETS_MAX];
+    uint64_t range[NOISE_RANDINT_SETS_MAX];
+} noise_randint_set_t;
+int noise_randint_many(int64_t *out, int64_t n, const noise_randint_set_t *set, uint64_t seed, int64_t threads,
+                       noise_stream_t stream);
+
 /* out[r * width + j] = element (offsets[rows[r]] + j) of the normal draw (seed, offset, threads), for
  * r < nrows, j < width (rows == NULL: rows[r] = r). Replaces Eggroll.noise's gather
  * buffer[offsets[name][directions, None] + arange(sum(p.shape))] (eggroll.py:126) over the 1 GiB
@@ -353,6 +365,24 @@ int noise_pop_block_qkv_jit(const noise_population_t *pop, noise_view_t y, const
 /* w [rows][cols] bf16 -> the column order noise_pop_block reads: within every 32 columns, position 8g + j
  * (g < 4) holds column 4g + j for j < 4 and 16 + 4g + (j - 4) for j >= 4. cols a multiple of 32. */
 int noise_block_weight_layout(const void *w, void *out, int64_t rows, int64_t cols, noise_stream_t stream);
+
+/* A parameter update's device copies in one launch. Per entry: numel values of src (fp32, or bf16 when src_bf16) to dst
+ * (16 B aligned) as bf16 (NOISE_WEIGHT_BF16; also to dst_block, unless NULL, in the column order of
+ * noise_block_weight_layout), as fp32 (NOISE_WEIGHT_FP32), or as fp32 holding the values rounded to bf16
+ * (NOISE_WEIGHT_FP32_ROUNDED: autocast's weights where a kernel reads fp32). Passed by value to the kernel. */
+#define NOISE_WEIGHTS_MAX 64
+#define NOISE_WEIGHT_BF16 0
+#define NOISE_WEIGHT_FP32 1
+#define NOISE_WEIGHT_FP32_ROUNDED 2
+typedef struct {
+    const void *src;
+    void *dst;
+    void *dst_block;
+    int64_t numel;
+    int32_t src_bf16;
+    int32_t kind;
+} noise_weight_t;
+int noise_weights_prepare(const noise_weight_t *weights, int count, noise_stream_t stream);
 
 /* mlp.c_proj [rows][2048] bf16 -> the column order noise_pop_mlp reads: within every 16 columns, the groups of
  * 4 are stored in the order 0, 2, 1, 3 (so each 16-deep slice of the hidden layer pairs with the registers the

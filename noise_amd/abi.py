@@ -12,6 +12,7 @@ SIGNATURES = {
     'noise_draw_layout': [_i32, _i64, _p, _p],
     'noise_normal_fill': [_p, _i64, _i64, _u64, _u64, _i64, _f32, _f32, _p],
     'noise_randint': [_p, _i64, _u64, _u64, _i64, _u64, _i64, _p],
+    'noise_randint_many': [_p, _i64, _p, _u64, _i64, _p],
     'noise_gather_slices': [_p, _i64, _i64, _p, _p, _i64, _u64, _u64, _i64, _p],
     'noise_gather_slice_groups': [_p, _i64, _i64, _p, _p, _i64, _u64, _u64, _i64, _p],
     'noise_orthogonal_draws': [_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _p],
@@ -35,6 +36,7 @@ SIGNATURES = {
     'noise_pop_block_qkv': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
                             'View', _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p],
     'noise_block_weight_layout': [_p, _p, _i64, _i64, _p],
+    'noise_weights_prepare': [_p, _i32, _p],
     'noise_mlp_proj_layout': [_p, _p, _i64, _p],
     'noise_pop_linear': [_p, 'View', _p, _i64, _i64, _p, _p, _p, _i32, _i64, _i64, _p],
     'noise_pop_head_ce': [_p, 'View', _p, _i64, _i64, _p, _p, _p, _i64, _p, _p],
@@ -106,6 +108,26 @@ class SliceGroups(ctypes.Structure):
     """noise_slice_groups_t: up to 64 parameters' [pairs] offsets, widths and output columns."""
     _fields_ = [('count', ctypes.c_int32), ('offsets', ctypes.c_void_p * SLICE_GROUPS_MAX),
                 ('width', ctypes.c_int64 * SLICE_GROUPS_MAX), ('col', ctypes.c_int64 * SLICE_GROUPS_MAX)]
+
+
+RANDINT_SETS_MAX = 64  # NOISE_RANDINT_SETS_MAX
+
+
+class RandintSet(ctypes.Structure):
+    """noise_randint_set_t: generator offsets and ranges of up to 64 draws."""
+    _fields_ = [('count', ctypes.c_int32), ('offset', ctypes.c_uint64 * RANDINT_SETS_MAX),
+                ('range', ctypes.c_uint64 * RANDINT_SETS_MAX)]
+
+
+# kinds of noise_weight_t
+WEIGHTS_MAX = 64
+WEIGHT_BF16, WEIGHT_FP32, WEIGHT_FP32_ROUNDED = 0, 1, 2
+
+
+class Weight(ctypes.Structure):
+    """noise_weight_t: one parameter's copies of noise_weights_prepare."""
+    _fields_ = [('src', ctypes.c_void_p), ('dst', ctypes.c_void_p), ('dst_block', ctypes.c_void_p),
+                ('numel', ctypes.c_int64), ('src_bf16', ctypes.c_int32), ('kind', ctypes.c_int32)]
 
 
 class BlockJitter(ctypes.Structure):

@@ -62,6 +62,17 @@ __global__ __launch_bounds__(kBlock) void randint_kernel(int64_t *__restrict__ o
     }
 }
 
+// draw k of a set per blockIdx.y: one launch for a step's offsets (60 launches of 1.5 us each before)
+__global__ __launch_bounds__(kBlock) void randint_many_kernel(int64_t *__restrict__ out, int64_t n,
+                                                              noise_randint_set_t set, uint64_t seed,
+                                                              uint64_t threads) {
+    const int k = blockIdx.y;
+    const DrawLayout d{seed, set.offset[k], threads};
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
+        out[k * n + i] = (int64_t)(draw_u32(d, (uint64_t)i) % set.range[k]);
+}
+
 // grid = (ceil(width / 256), nrows)
 __global__ __launch_bounds__(kBlock) void gather_slices_kernel(float *__restrict__ out, int64_t width,
                                                                const int64_t *__restrict__ offsets,
@@ -234,6 +245,26 @@ extern "C" int noise_randint(int64_t *out, int64_t n, uint64_t seed, uint64_t of
     DrawLayout d{seed, offset, (uint64_t)threads};
     hipLaunchKernelGGL(randint_kernel, dim3(grid_for(n)), dim3(kBlock), 0, (hipStream_t)stream, out, n, d, range, base);
     return launch_status("noise_randint");
+}
+
+extern "C" int noise_randint_many(int64_t *out, int64_t n, const noise_randint_set_t *set, uint64_t seed,
+                                  int64_t threads, noise_stream_t stream) {
+    clear_error();
+    const char *fn = "noise_randint_many";
+    NOISE_CHECK_ARG(set != nullptr && set->count >= 1 && set->count <= NOISE_RANDINT_SETS_MAX, "%s: 1 .. %d draws", fn,
+                    NOISE_RANDINT_SETS_MAX);
+    NOISE_CHECK_ARG(n >= 0 && threads > 0 && threads % 256 == 0, "%s: n >= 0 and threads a positive multiple of 256", fn);
+    for (int k = 0; k < set->count; ++k) {
+        NOISE_CHECK_ARG(set->offset[k] % 4 == 0, "%s: draw %d: generator offset must be a multiple of 4", fn, k);
+        NOISE_CHECK_ARG(set->range[k] >= 1 && set->range[k] < (1ull << 28),
+                        "%s: draw %d: range must be in [1, 2^28) (torch's 32-bit path), got %llu", fn, k,
+                        (unsigned long long)set->range[k]);
+    }
+    if (n == 0) return NOISE_OK;
+    NOISE_CHECK_ARG(out != nullptr && aligned(out, 8), "%s: out must be a non-NULL 8-byte aligned pointer", fn);
+    hipLaunchKernelGGL(randint_many_kernel, dim3(grid_for(n), (unsigned)set->count), dim3(kBlock), 0, (hipStream_t)stream,
+                       out, n, *set, seed, (uint64_t)threads);
+    return launch_status(fn);
 }
 
 extern "C" int noise_gather_slices(float *out, int64_t nrows, int64_t width, const int64_t *offsets,

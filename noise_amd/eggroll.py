@@ -119,43 +119,55 @@ class Weights:
         if dev.type != 'cuda':
             raise ValueError('population_loss runs on the GPU')
         self.device, self.n_layer = dev, n_layer
-        g = lambda n: p[n].detach().to(dev)
-        bf = lambda n: g(n).to(BF16).contiguous()
-        # fp32 tables and scalars are copied even when the parameter is already fp32 on the device: a Weights
-        # is a snapshot of one update's parameters, never a view of the live ones
-        snap = lambda n: g(n).to(F32, copy=True).contiguous()
-        self.wte = snap('transformer.wte.weight')
-        self.lm_head = bf('lm_head.weight')
+        # every parameter is copied, also where it already has the dtype: a Weights is a snapshot of one update's
+        # parameters, never a view of the live ones. One launch per 64 parameters makes all the copies.
+        jobs = []
+
+        def add(name, kind, block=False):
+            t = p[name].detach().to(dev)
+            if t.dtype not in (F32, BF16):
+                t = t.to(BF16 if kind == _lib.WEIGHT_BF16 else F32)
+            t = t.contiguous()
+            dst = torch.empty(t.shape, dtype=BF16 if kind == _lib.WEIGHT_BF16 else F32, device=dev)
+            blk = torch.empty_like(dst) if block else None
+            jobs.append((t, dst, blk, kind))
+            return (dst, blk) if block else dst
+
+        self.wte = add('transformer.wte.weight', _lib.WEIGHT_FP32)
+        self.lm_head = add('lm_head.weight', _lib.WEIGHT_BF16)
         self.fp32_head = fp32_head
-        if fp32_head:
-            w = g('lm_head.weight').to(F32).contiguous()
-            self.lm_head3 = torch.empty(w.shape[0], 3 * w.shape[1], dtype=BF16, device=dev)
-            _lib.call('noise_split3', w.data_ptr(), w.shape[0], w.shape[1], 0, 1, self.lm_head3.data_ptr(),
-                      _lib.stream_ptr(dev))
         # the mixing scalars stay on the device: the kernels read them there (a host copy would wait for the
         # stream at every update)
-        self.resid_lambdas = snap('resid_lambdas')
-        self.x0_lambdas = snap('x0_lambdas')
+        self.resid_lambdas = add('resid_lambdas', _lib.WEIGHT_FP32)
+        self.x0_lambdas = add('x0_lambdas', _lib.WEIGHT_FP32)
         self.blocks = []
         for i in range(n_layer):
             pre = f'transformer.h.{i}.'
-            blk = dict(q=bf(pre + 'attn.c_q.weight'), k=bf(pre + 'attn.c_k.weight'), v=bf(pre + 'attn.c_v.weight'),
-                       o=bf(pre + 'attn.c_proj.weight'), fc=bf(pre + 'mlp.c_fc.weight'),
-                       mp=bf(pre + 'mlp.c_proj.weight'))
-            # mlp.c_fc and mlp.c_proj in the block kernel's column order (within every 32 columns); so are c_q, c_k
-            # and c_v of the blocks whose q/k/v the previous block's kernel forms
-            perm = [('mp', 'mp_blk'), ('fc', 'fc_blk')]
-            if i:
-                perm += [('q', 'q_blk'), ('k', 'k_blk'), ('v', 'v_blk')]
-            for src, dst in perm:
-                blk[dst] = torch.empty_like(blk[src])
-                _lib.call('noise_block_weight_layout', blk[src].data_ptr(), blk[dst].data_ptr(), blk[src].shape[0],
-                          blk[src].shape[1], _lib.stream_ptr(dev))
+            blk = {}
+            # mlp.c_fc and mlp.c_proj also in the block kernel's column order (within every 32 columns); so are c_q,
+            # c_k and c_v of the blocks whose q/k/v the previous block's kernel forms
+            for key, name, block in (('q', 'attn.c_q', i), ('k', 'attn.c_k', i), ('v', 'attn.c_v', i),
+                                     ('o', 'attn.c_proj', 0), ('fc', 'mlp.c_fc', 1), ('mp', 'mlp.c_proj', 1)):
+                if block:
+                    blk[key], blk[key + '_blk'] = add(f'{pre}{name}.weight', _lib.WEIGHT_BF16, True)
+                else:
+                    blk[key] = add(f'{pre}{name}.weight', _lib.WEIGHT_BF16)
             if has_ve(i, n_layer):
                 # the gate's product runs under autocast: its weights enter rounded to bf16
-                blk['gate'] = bf(pre + 'attn.ve_gate.weight').to(F32).contiguous()
-                blk['ve'] = snap(f'value_embeds.{i}.weight')
+                blk['gate'] = add(pre + 'attn.ve_gate.weight', _lib.WEIGHT_FP32_ROUNDED)
+                blk['ve'] = add(f'value_embeds.{i}.weight', _lib.WEIGHT_FP32)
             self.blocks.append(blk)
+        stream = _lib.stream_ptr(dev)
+        for first in range(0, len(jobs), _lib.WEIGHTS_MAX):
+            part = jobs[first:first + _lib.WEIGHTS_MAX]
+            table = (_lib.Weight * len(part))(*(
+                _lib.Weight(t.data_ptr(), d.data_ptr(), _lib.ptr(k), t.numel(), int(t.dtype == BF16), kind)
+                for t, d, k, kind in part))
+            _lib.call('noise_weights_prepare', table, len(part), stream)
+        if fp32_head:
+            w = p['lm_head.weight'].detach().to(dev, F32).contiguous()
+            self.lm_head3 = torch.empty(w.shape[0], 3 * w.shape[1], dtype=BF16, device=dev)
+            _lib.call('noise_split3', w.data_ptr(), w.shape[0], w.shape[1], 0, 1, self.lm_head3.data_ptr(), stream)
         self.windows = window_sizes(n_layer)
 
     def lam_r(self, i):
@@ -718,7 +730,8 @@ class Eggroll:
     def offsets(self, step):
         """eggroll.py:117-120: one randint draw of [pairs] per parameter, in named_parameters order."""
         g = DeviceGenerator(1_000_003 * self.seed + step, self.device)
-        return {name: g.randint(0, self.noise_numel - sum(p.shape), (self.pairs,)) for name, p in self.params.items()}
+        rows = g.randint_many([self.noise_numel - sum(p.shape) for p in self.params.values()], self.pairs)
+        return dict(zip(self.params, rows.unbind(0)))
 
     def noise(self, offsets, directions):
         """eggroll.py:122-128: name -> (a [n, out], b [n, in]) for matrices and embeddings, eps [n, L]."""
@@ -729,25 +742,22 @@ class Eggroll:
         return out
 
     def noise_tables(self, offsets, directions):
-        """Eggroll.noise's values for the parameters in `offsets` at `directions`, regenerated in one launch for
-        the matrices whose rows are whole multiples of 256 (every block matrix and the head: a [dirs, sum of
-        out + in] table, each parameter's a and b column views of it) and per parameter for the rest."""
+        """Eggroll.noise's values for the parameters in `offsets` at `directions`, regenerated in one launch per 64
+        parameters: column views of one [dirs, columns] table. Each parameter's columns start at a multiple of 256; a
+        narrower slice is followed by elements that nothing reads."""
         out = {}
-        grouped = [n for n in offsets if self.params[n].dim() == 2 and sum(self.params[n].shape) % 256 == 0]
-        if grouped:
-            widths = [sum(self.params[n].shape) for n in grouped]
-            table = self.buffer.gather_many([offsets[n] for n in grouped], widths, directions)
-            col = 0
-            for n, w in zip(grouped, widths):
-                o, i = self.params[n].shape
-                out[n] = (table[:, col:col + o], table[:, col + o:col + w])
-                col += w
-        for name, o in offsets.items():
-            if name in out:
-                continue
-            p = self.params[name]
-            rows = self.buffer.gather(o, sum(p.shape), rows=directions)
-            out[name] = tuple(rows.split(list(p.shape), dim=1)) if p.dim() == 2 else rows
+        names = list(offsets)
+        widths = [-(-sum(self.params[n].shape) // 256) * 256 for n in names]
+        table = self.buffer.gather_many([offsets[n] for n in names], widths, directions) if names else None
+        col = 0
+        for n, w in zip(names, widths):
+            shape = self.params[n].shape
+            if len(shape) == 2:
+                o, i = shape
+                out[n] = (table[:, col:col + o], table[:, col + o:col + o + i])
+            else:
+                out[n] = table[:, col:col + shape[0]]
+            col += w
         return out
 
     def population(self, step, x, y, weights=None, chunk=512, names=None, fp32_head=False):

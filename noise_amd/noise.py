@@ -128,6 +128,29 @@ class DeviceGenerator:
         return out
 
 
+    def randint_many(self, highs, n):
+        """[randint(0, high, n) for high in highs], bit for bit and in that order, in one launch per 64 draws: rows
+        of one int64 tensor [len(highs), n]."""
+        out = torch.empty(len(highs), n, device=self.device, dtype=torch.int64)
+        for high in highs:
+            if not 1 <= int(high) < 2 ** 28:
+                raise ValueError(f'randint range must be in [1, 2^28) (torch 32-bit path), got {int(high)}')
+        if n == 0 or not len(highs):
+            return out
+        threads, inc = draw_layout(n, self.device)
+        for first in range(0, len(highs), _lib.RANDINT_SETS_MAX):
+            part = highs[first:first + _lib.RANDINT_SETS_MAX]
+            desc = _lib.RandintSet()
+            desc.count = len(part)
+            for i, high in enumerate(part):
+                desc.offset[i] = self.offset
+                desc.range[i] = int(high)
+                self.offset += inc
+            _lib.call('noise_randint_many', out.data_ptr() + 8 * n * first, n, ctypes.byref(desc), self.seed, threads,
+                      _lib.stream_ptr(self.device))
+        return out
+
+
 class OrthogonalDraws:
     """DUST.orthogonal_noise (run.py:223-238) on the device, bit for bit.
 

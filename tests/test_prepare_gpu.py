@@ -1,0 +1,83 @@
+"""The one-launch preparations of an update, bit for bit: Weights (noise_weights_prepare) against torch's casts and
+the block layout's formula, DeviceGenerator.randint_many against torch.randint on a device generator, and
+Eggroll.noise_tables against Eggroll.noise for every parameter."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device('cuda', 0)
+
+
+def _block_order(w):
+    r, c = w.shape
+    g = w.view(r, c // 32, 8, 4)
+    return g[:, :, [0, 4, 1, 5, 2, 6, 3, 7]].reshape(r, c)
+
+
+@pytest.mark.parametrize('fp32_embeddings', [True, False])
+def test_weights_are_the_parameters(fp32_embeddings):
+    from noise_amd.eggroll import Weights
+    from noise_amd.model import make_model
+    model = make_model(DEV, 3, fp32_embeddings=fp32_embeddings)
+    for q in model.parameters():
+        if q.dim() == 1 or q.shape[0] == 8:
+            q.copy_(torch.randn(q.shape, device=DEV))
+    p = dict(model.named_parameters())
+    p['transformer.h.2.attn.c_q.weight'] = p['transformer.h.2.attn.c_q.weight'].t().contiguous().t()  # not contiguous
+    odd = torch.empty(512 * 512 + 1, device=DEV)[1:].view(512, 512).copy_(p['transformer.h.3.attn.c_k.weight'])
+    p['transformer.h.3.attn.c_k.weight'] = odd  # off the 16 B alignment
+    p['transformer.h.4.attn.c_v.weight'] = p['transformer.h.4.attn.c_v.weight'].double()
+    W = Weights(p)
+    keys = dict(q='attn.c_q', k='attn.c_k', v='attn.c_v', o='attn.c_proj', fc='mlp.c_fc', mp='mlp.c_proj')
+    for i, blk in enumerate(W.blocks):
+        for k, name in keys.items():
+            ref = p[f'transformer.h.{i}.{name}.weight'].bfloat16()
+            assert torch.equal(blk[k], ref), (i, k)
+            if k + '_blk' in blk:
+                assert torch.equal(blk[k + '_blk'], _block_order(ref)), (i, k)
+        assert ('q_blk' in blk) == (i > 0) and 'fc_blk' in blk and 'mp_blk' in blk
+        if 'gate' in blk:
+            assert torch.equal(blk['gate'], p[f'transformer.h.{i}.attn.ve_gate.weight'].bfloat16().float())
+            assert torch.equal(blk['ve'], p[f'value_embeds.{i}.weight'].float())
+    assert torch.equal(W.wte, p['transformer.wte.weight'].float()) and torch.equal(W.lm_head, p['lm_head.weight'].bfloat16())
+    assert torch.equal(W.resid_lambdas, p['resid_lambdas']) and torch.equal(W.x0_lambdas, p['x0_lambdas'])
+    p['x0_lambdas'].add_(1)
+    assert not torch.equal(W.x0_lambdas, p['x0_lambdas'])  # a snapshot
+
+
+@pytest.mark.parametrize('numel', [1, 7, 8, 2047, 2049])
+@pytest.mark.parametrize('kind', [0, 1, 2])
+def test_entry_tails(numel, kind):
+    from noise_amd import _lib
+    src = torch.randn(numel, device=DEV)
+    dst = torch.full((numel + 8,), 5.0, device=DEV, dtype=torch.bfloat16 if kind == 0 else torch.float32)
+    table = (_lib.Weight * 1)(_lib.Weight(src.data_ptr(), dst.data_ptr(), None, numel, 0, kind))
+    _lib.call('noise_weights_prepare', table, 1, _lib.stream_ptr(DEV))
+    ref = [src.bfloat16(), src, src.bfloat16().float()][kind]
+    assert torch.equal(dst[:numel], ref) and (dst[numel:] == 5).all()
+
+
+@pytest.mark.parametrize('n,count', [(1, 1), (5, 64), (300, 65), (70000, 3), (2 ** 21 + 3, 2)])
+def test_randint_many_is_torch(n, count):
+    from noise_amd.noise import DeviceGenerator
+    highs = [2 ** 28 - 1 - 977 * k for k in range(count)]
+    g, t = DeviceGenerator(11, DEV), torch.Generator(DEV).manual_seed(11)
+    got = g.randint_many(highs, n)
+    for k, h in enumerate(highs):
+        assert torch.equal(got[k], torch.randint(0, h, (n,), device=DEV, generator=t)), k
+    assert torch.equal(g.randint(0, 1000, 9), torch.randint(0, 1000, (9,), device=DEV, generator=t))
+
+
+def test_noise_tables_are_the_noise():
+    from noise_amd.eggroll import Eggroll
+    from noise_amd.model import make_model
+    es = Eggroll(make_model('cpu', 0).to(DEV), 7)
+    offsets = es.offsets(2)
+    directions = torch.tensor([6, 0, 3], device=DEV)
+    tables, ref = es.noise_tables(offsets, directions), es.noise(offsets, directions)
+    assert set(tables) == set(ref)
+    for n, v in ref.items():
+        for a, b in zip(v if isinstance(v, tuple) else (v,), tables[n] if isinstance(v, tuple) else (tables[n],)):
+            assert torch.equal(a, b), n
