@@ -1,5 +1,5 @@
-// EGGROLL's update reassembly: fitness weights and the rank-1 gradient sum, the noise regenerated from the
-// Philox counter inside the kernels (no 1 GiB buffer, no gathered fp32 noise rows).
+// EGGROLL's update reassembly: fitness weights and the rank-1 gradient sum over the noise slices, read from the
+// materialised draw or regenerated from the Philox counter a chunk of directions at a time (no 1 GiB buffer).
 //
 // Replaces eggroll.py:151-163:
 //   fitness = losses[1::2] - losses[0::2]; fitness = fitness / (fitness.std() + 1e-8)
@@ -11,13 +11,11 @@
 //
 // A 2-D parameter's gradient G = scale * sum_d w_d a_d b_d^T is a GEMM [rows x pairs] x [pairs x cols]. The
 // reference runs it in fp32 (TF32 under set_float32_matmul_precision('high'), run.py:676 / eggroll.py main);
-// gfx950 has no xf32 MFMA, so each chunk of directions is regenerated into a bf16 table holding the hi and lo
-// halves of every value (v = hi + lo to 2^-16; the weights folded into a's rows), in blocks of 32 directions
-// per 128 B line: [hi x 32 | lo x 32]. The GEMM reads a line of every row per stage and issues the three bf16
-// products hi_a hi_b, hi_a lo_b, lo_a hi_b of each 16 directions from one read of each fragment
-// (split-bf16x3, fp32 accumulation). Chunks accumulate into G in order (deterministic). Parameters whose
-// sides are not multiples of 256 (ve_gate [8, 32], the 1-D mixing scalars) are small: one workgroup per
-// gradient entry sums over all directions.
+// gfx950 has no xf32 MFMA, so the GEMM splits every value into a hi and a lo bf16 half (v = hi + lo to 2^-16; the
+// weights folded into a's side) as its fp32 slices land in LDS, and issues the three bf16 products hi_a hi_b,
+// hi_a lo_b, lo_a hi_b of each 16 directions from one read of each fragment (split-bf16x3, fp32 accumulation).
+// Chunks accumulate into G in order (deterministic). Parameters whose sides are not multiples of 256 (ve_gate
+// [8, 32], the 1-D mixing scalars) are small: their entries' sums run on the vector units.
 #include <atomic>
 
 #include "common.hpp"
@@ -34,7 +32,7 @@ constexpr int kTile = 256;
 struct UpdateSet {
     int n;
     const int64_t *offsets[kMaxParams];
-    __bf16 *table[kMaxParams];        // [rows + cols][2 np]: a rows, then b rows, [hi 32 | lo 32] blocks
+    float *slab[kMaxParams];          // [np][rows + cols]: a chunk's slices, where they are not read from a buffer
     float *grad[kMaxParams];          // [rows][cols]
     int rows[kMaxParams], cols[kMaxParams];
     int row_start[kMaxParams + 1];    // prefix sums of rows + cols
@@ -87,90 +85,28 @@ __global__ __launch_bounds__(1024) void update_weights_kernel(const float *__res
     }
 }
 
-// position of direction k's hi half in a table row ([hi x 32 | lo x 32] per 32 directions; lo 32 after it)
-__device__ __forceinline__ int64_t tab_pos(int64_t k) { return (k >> 5) * 64 + (k & 31); }
-
-// One table row per workgroup, 256 directions per thread block column: row r of parameter p holds, for
-// direction d0 + k, the element off_d + r of the draw (a for r < rows, scaled by weight * scale; b after).
-// Directions k >= n (padding up to np) are zero.
-__global__ __launch_bounds__(256) void update_tables_kernel(UpdateSet s, int64_t d0, int64_t n, int64_t np,
-                                                            const float *__restrict__ weight, float scale,
-                                                            DrawLayout dl, int64_t numel) {
-    const int r = blockIdx.x;
-    int p = 0;
-    while (p + 1 < s.n && s.row_start[p + 1] <= r) ++p;
-    const int rl = r - s.row_start[p];
-    const bool is_a = rl < s.rows[p];
-    __bf16 *row = s.table[p] + (int64_t)rl * 2 * np;
-    const int64_t k = (int64_t)blockIdx.y * 256 + threadIdx.x;
-    float v = 0.0f;
-    if (k < n) {
-        const int64_t d = d0 + k;
-        v = noise_at(dl, s.offsets[p][d] + rl, numel);
-        if (is_a) v *= weight[d] * scale;
-    }
-    {
-        // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract)
-#pragma clang fp contract(off)
-        const __bf16 hi = (__bf16)v;
-        row[tab_pos(k)] = hi;
-        row[tab_pos(k) + 32] = (__bf16)(v - (float)hi);
-    }
-}
-
-// As update_tables_kernel, reading the draw from a materialised buffer (fp32 [numel]) instead of the Philox
-// counter: a workgroup reads 32 directions x 256 consecutive elements (1 KiB per direction, coalesced) into
-// LDS, all 32 loads of a thread in flight together, then writes the 256 table rows' block of 32 directions
-// (4 lanes x 2 x 16 B per row: one whole 128 B line). The 33 KB tile lets four workgroups share a CU, which
-// keeps enough bytes in flight for the HBM's latency. grid = (rows_total / 256, np / 32).
-constexpr int kTabK = 32, kTabPad = 257;
-__global__ __launch_bounds__(256) void update_tables_from_buffer_kernel(UpdateSet s, int64_t d0, int64_t n,
-                                                                        int64_t np, const float *__restrict__ weight,
-                                                                        float scale, const float *__restrict__ buf,
-                                                                        int64_t numel) {
-    __shared__ float sm[kTabK * kTabPad];
-    const int r0 = blockIdx.x * 256, tid = threadIdx.x;
+// A chunk's slices: slab[p][k][r] = element off_d + r of the draw, d = d0 + k, from the Philox counter or (BUFFER) a
+// materialised buffer too long for the GEMM's own reads; NaN outside the draw. A thread per element, 256 elements of
+// one slice per workgroup and step, so the stores are whole lines. Bound by Philox's ten rounds of two 32 x 32 -> 64
+// multiplies per element (four elements 2^19 apart share a block, which slices cannot use): 512 directions of the 60
+// parameters, 38.4 M normals,
+// 159 us (split bf16 tables, one direction per lane and 2 B stores 2 np apart, took 662). grid = (sum of widths / 256, a share of the directions)
+template <bool BUFFER>
+__global__ __launch_bounds__(256) void update_slices_kernel(UpdateSet s, int64_t d0, int64_t n, DrawLayout dl,
+                                                            const float *__restrict__ buf, int64_t numel) {
+    const int r0 = blockIdx.x * 256;
     int p = 0;
     while (p + 1 < s.n && s.row_start[p + 1] <= r0) ++p;
-    const int rl0 = r0 - s.row_start[p];  // the 256 rows lie in one parameter (its row count is a multiple of 256)
-    const int64_t k0 = (int64_t)blockIdx.y * kTabK;
-    const int kv = n - k0 < kTabK ? (int)(n - k0) : kTabK;  // valid directions of this block (>= 1)
-    const int64_t *off = s.offsets[p] + d0 + k0;
-    // the tile's loads in flight together: addresses clamped into the buffer, out-of-range elements set after
-    for (int kb = 0; kb < kTabK; kb += 32) {
-        float v[32];
-        bool ok[32];
-#pragma unroll
-        for (int e = 0; e < 32; ++e) {
-            const int64_t L = (kb + e < kv ? off[kb + e] : 0) + rl0 + tid;
-            ok[e] = L >= 0 && L < numel;
-            v[e] = buf[L < 0 ? 0 : (L < numel ? L : numel - 1)];
-        }
-#pragma unroll
-        for (int e = 0; e < 32; ++e)
-            sm[(kb + e) * kTabPad + tid] = kb + e < kv ? (ok[e] ? v[e] : __builtin_nanf("")) : 0.0f;
-    }
-    __syncthreads();
-    const int c = tid & 3;  // directions 8c .. 8c + 7 of the block's 32
-    float wk[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) wk[e] = k0 + 8 * c + e < n ? weight[d0 + k0 + 8 * c + e] * scale : 0.0f;
-    for (int pass = 0; pass < 4; ++pass) {
-        const int rr = pass * 64 + (tid >> 2), rl = rl0 + rr;
-        const bool is_a = rl < s.rows[p];
-        bf16x8 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract)
-#pragma clang fp contract(off)
-            float v = sm[(8 * c + e) * kTabPad + rr];
-            if (is_a) v *= wk[e];
-            hi[e] = (__bf16)v;
-            lo[e] = (__bf16)(v - (float)hi[e]);
-        }
-        __bf16 *row = s.table[p] + (int64_t)rl * 2 * np + tab_pos(k0 + 8 * c);
-        *reinterpret_cast<bf16x8 *>(row) = hi;
-        *reinterpret_cast<bf16x8 *>(row + 32) = lo;
+    const int rl = r0 - s.row_start[p] + threadIdx.x;  // (every width is a multiple of 256)
+    const int64_t width = s.rows[p] + s.cols[p];
+    for (int64_t k = blockIdx.y; k < n; k += gridDim.y) {
+        const int64_t L = s.offsets[p][d0 + k] + rl;
+        float v;
+        if constexpr (BUFFER)
+            v = L >= 0 && L < numel ? buf[L] : __builtin_nanf("");
+        else
+            v = noise_at(dl, L, numel);
+        s.slab[p][k * width + rl] = v;
     }
 }
 
@@ -182,32 +118,25 @@ __global__ __launch_bounds__(256) void update_tables_from_buffer_kernel(UpdateSe
 // shorter. Per stage, 32 directions of the tile's 512 rows (64 KiB), two stages in flight; per 16 directions a
 // wave reads its hi and lo fragments once for 24 products.
 //
-// Tables (RAW false): a stage is one 128 B line of each row ([hi | lo] of 32 directions) copied global -> LDS,
-// chunks XOR-swizzled by row pair, read as 16 B fragments.
-//
-// Buffer (RAW true): no tables. A stage is the 32 directions' fp32 slices themselves, [direction][A rows | B
+// A stage is the 32 directions' fp32 slices themselves, from the materialised draw or a slab, [direction][A rows | B
 // rows] at a stride of 2176 B (2 KiB + 128), copied straight from the buffer (16 B per lane; slices start at any
 // element). Each wave copies 4 directions and, once its copies have landed, splits them in place: the 32 B
 // holding rows 8 c .. 8 c + 7 of a direction become [hi x 8 | lo x 8] (lo first where bit 1 of the direction is
 // set), so nothing crosses lanes or waves before the stage's barrier. Fragments are then read with gfx950's
 // transposing LDS read (ds_read_b64_tr_b16: in each 16 lanes, lane i takes element i % 4 of the 8 B that lane
 // i / 4 + 4 e addresses), which gathers a row's 4 consecutive directions from 4 direction rows. The odd stride
-// (128 B apart mod 256) and the hi / lo swap put a read's 4 directions on 4 disjoint sets of banks. The values,
-// hence the products and G, are those of the tables.
+// (128 B apart mod 256) and the hi / lo swap put a read's 4 directions on 4 disjoint sets of banks.
 struct UpdateRaw {
-    int64_t d0, n;             // the chunk's first direction and its valid directions (the rest up to np is zero)
+    int64_t d0, n;             // the chunk's first direction and its directions (zeros fill the last stage)
     const float *weight;
     float scale;
-    const float *buf;          // fp32 [numel], numel <= 2^30 (lane offsets are 32-bit byte offsets)
+    const float *buf;          // fp32 [numel], numel <= 2^30 (lane offsets are 32-bit byte offsets); NULL: the slabs
     int64_t numel;
 };
-constexpr int kUgStage = 512 * 128;  // tables: bytes per stage, 256 A rows, then 256 B rows
-constexpr int kUgDir = 2176;         // buffer: bytes per direction of a stage (2 KiB of rows, 128 B apart)
-constexpr int kUgRawStage = 32 * kUgDir;
-template <bool RAW>
-__global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, int accumulate, int full, int split,
+constexpr int kUgDir = 2176;         // bytes per direction of a stage (2 KiB of rows, 128 B apart)
+constexpr int kSt = 32 * kUgDir;
+__global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accumulate, int full, int split,
                                                           float *__restrict__ part, UpdateRaw raw) {
-    constexpr int kSt = RAW ? kUgRawStage : kUgStage;
     __shared__ __attribute__((aligned(16))) char lds[2 * kSt];
     // workgroups are dispatched round-robin over the 8 XCDs: each XCD takes a contiguous range of the full
     // tiles (and of the partial items), so the tiles that share a table panel run under one L2
@@ -229,32 +158,18 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn0 = 128 * (wave & 1), wm0 = 64 * (wave >> 1);
-    const int64_t ld = 2 * (int64_t)np;  // table row length (elements)
-    const __bf16 *A = s.table[p] + (int64_t)ot * kTile * ld, *B = s.table[p] + (int64_t)(rows + ct * kTile) * ld;
     const unsigned lbase = lds_addr(lds);
-    // stages k0 .. k0 + nk - 1 of the chunk's np / 32 (np is a multiple of 256: np / 32 divides by split)
-    const int nk = partial ? np / 32 / split : np / 32;
-    const int k0 = partial ? (item % split) * nk : 0;
+    // stages k0 .. k0 + nk - 1 of the chunk's, 32 directions each (a partial workgroup's range may be empty)
+    const int stages = (int)((raw.n + 31) / 32), q0 = partial ? item % split : 0, qn = partial ? split : 1;
+    const int k0 = stages * q0 / qn, nk = stages * (q0 + 1) / qn - k0;
 
-    // tables: copy i (0 .. 7) of a stage: tile rows 64 i + 8 wave .. + 8 (A for i < 4, B after); lane: row
-    // lane / 8 of the copy, LDS slot lane % 8 holds the line's chunk (lane % 8) ^ ((row >> 1) & 7)
-    const int rl = 8 * wave + (lane >> 3);
-    const int cl = (lane & 7) ^ ((rl >> 1) & 7);
-    const unsigned off = (unsigned)(rl * ld * 2 + cl * 16);
-    auto issue = [&](int ks) {  // stage k0 + ks into buffer ks % 2
-        const unsigned st = lbase + (ks & 1) * kUgStage + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const __bf16 *src = (i < 4 ? A + (int64_t)(64 * i) * ld : B + (int64_t)(64 * (i - 4)) * ld) + 64 * (k0 + ks);
-            lds_dma16_at(src, off, st + i * 8192);
-        }
-    };
-
-    // buffer: wave w copies and splits directions 4 w + i (i = 0 .. 3) of each stage. The offsets and weights
+    // wave w copies and splits directions 4 w + i (i = 0 .. 3) of each stage. The offsets and weights
     // are read through the scalar cache (address space 4: this kernel writes neither).
     typedef const __attribute__((address_space(4))) int64_t *c_i64p;
     typedef const __attribute__((address_space(4))) float *c_f32p;
     const c_i64p offs = (c_i64p)s.offsets[p];
+    const float *buf = raw.buf ? raw.buf : s.slab[p];
+    const int64_t numel = raw.buf ? raw.numel : raw.n * (rows + cols);
     const c_f32p wts = (c_f32p)raw.weight;
     const int64_t side0 = (int64_t)ot * kTile, side1 = (int64_t)rows + ct * kTile;  // first slice element per side
     // a side of a direction (256 rows, 1 KiB) in one copy of 16 B per lane (lane l: rows 4 l .. + 4; a slice may
@@ -266,7 +181,7 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
     float d_w[4];
     int d_kind[4];
     auto issue_raw = [&](int ks) {
-        const unsigned st = lbase + (ks & 1) * kUgRawStage;
+        const unsigned st = lbase + (ks & 1) * kSt;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int dl = 4 * wave + i;
@@ -275,16 +190,16 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
             int kind = 0;
             float w = 0.0f;
             if (k < raw.n) {
-                o = offs[raw.d0 + k];
+                o = raw.buf ? offs[raw.d0 + k] : k * (rows + cols);
                 w = wts[raw.d0 + k] * raw.scale;
-                kind = o + side0 >= 0 && o + side1 + kTile <= raw.numel ? 1 : 2;
+                kind = o + side0 >= 0 && o + side1 + kTile <= numel ? 1 : 2;
             }
             d_off[i] = o;
             d_w[i] = w;
             d_kind[i] = kind;
             if (kind == 1) {
-                lds_dma16_at(raw.buf + o + side0, (unsigned)(16 * lane), st + dl * kUgDir);
-                lds_dma16_at(raw.buf + o + side1, (unsigned)(16 * lane), st + dl * kUgDir + 1024);
+                lds_dma16_at(buf + o + side0, (unsigned)(16 * lane), st + dl * kUgDir);
+                lds_dma16_at(buf + o + side1, (unsigned)(16 * lane), st + dl * kUgDir + 1024);
             } else {
                 // 4 B copies with every lane's element clamped into the buffer (a padding direction reads row 0)
 #pragma unroll
@@ -292,8 +207,8 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         int64_t L = kind ? o + (side ? side1 : side0) + 64 * q + lane : 0;
-                        L = L < 0 ? 0 : (L < raw.numel ? L : raw.numel - 1);
-                        lds_dma4_at(raw.buf, (unsigned)(4 * L), st + dl * kUgDir + side * 1024 + 256 * q);
+                        L = L < 0 ? 0 : (L < numel ? L : numel - 1);
+                        lds_dma4_at(buf, (unsigned)(4 * L), st + dl * kUgDir + side * 1024 + 256 * q);
                     }
             }
         }
@@ -301,7 +216,7 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
     // split stage ks (buffer ks % 2) in place: lane l takes side l / 32, rows 64 q + 8 c .. + 8 (q = (l / 8) % 4,
     // c = l % 8) of each of the wave's 4 directions
     auto split_raw = [&](int ks) {
-        char *st = lds + (ks & 1) * kUgRawStage;
+        char *st = lds + (ks & 1) * kSt;
         const int side = lane >> 5, q = (lane >> 3) & 3, cp = lane & 7;
         // the two 16 B halves (rows + 0 .. 3, + 4 .. 7) in the order h, 1 - h with h = bit 3 of the lane: each
         // 16-lane pass then covers every bank once
@@ -318,7 +233,7 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
             auto convert = [&](const float4 (&x)[2], float wx) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract), as the tables
+                    // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract)
 #pragma clang fp contract(off)
                     const int hh = t ? 1 - h0 : h0;
                     const float v[4] = {x[t].x * wx, x[t].y * wx, x[t].z * wx, x[t].w * wx};
@@ -347,21 +262,14 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
                     const int64_t Lh = L + 4 * (t ? 1 - h0 : h0);
                     float *f = reinterpret_cast<float *>(&y[t]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) f[e] = (Lh + e >= 0 && Lh + e < raw.numel) ? f[e] : __builtin_nanf("");
+                    for (int e = 0; e < 4; ++e) f[e] = (Lh + e >= 0 && Lh + e < numel) ? f[e] : __builtin_nanf("");
                 }
                 convert(y, w);
             }
         }
     };
 
-    // tables: fragment rows wn0 + 32 fb + j (A) and 256 + wm0 + 32 tb + j (B) share the swizzle of row j; chunk
-    // 2 s + hf is the hi half of directions 16 s + 8 hf .. + 8, chunk 4 + 2 s + hf its lo half
-    int fo[2][2];
-#pragma unroll
-    for (int sk = 0; sk < 2; ++sk)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) fo[sk][h] = j * 128 + (((4 * h + 2 * sk + hf) ^ ((j >> 1) & 7)) << 4);
-    // buffer: lane 16 G + i addresses direction 8 (G / 2) + i / 4 (+ 16 sk + 4 e) and rows 16 (G % 2) + 4 (i % 4)
+    // lane 16 G + i addresses direction 8 (G / 2) + i / 4 (+ 16 sk + 4 e) and rows 16 (G % 2) + 4 (i % 4)
     // .. + 4 of a 32-row block; bit 1 of that direction (bit 3 of i) swaps hi and lo. tro[lo]
     int tro[2];
     {
@@ -386,28 +294,15 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
     // fragments of 16 directions, double buffered: those of the next step are read while this step's run
     bf16x8 ah[2][4], al[2][4], bh[2][2], bl[2][2];
     auto fetch = [&](int buf, const char *st, int sk) {
-        if constexpr (RAW) {
 #pragma unroll
-            for (int fb = 0; fb < 4; ++fb) {
-                ah[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 0);
-                al[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 1);
-            }
+        for (int fb = 0; fb < 4; ++fb) {
+            ah[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 0);
+            al[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 1);
+        }
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                bh[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 0);
-                bl[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 1);
-            }
-        } else {
-#pragma unroll
-            for (int fb = 0; fb < 4; ++fb) {
-                ah[buf][fb] = *reinterpret_cast<const bf16x8 *>(st + (wn0 + 32 * fb) * 128 + fo[sk][0]);
-                al[buf][fb] = *reinterpret_cast<const bf16x8 *>(st + (wn0 + 32 * fb) * 128 + fo[sk][1]);
-            }
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) {
-                bh[buf][tb] = *reinterpret_cast<const bf16x8 *>(st + (256 + wm0 + 32 * tb) * 128 + fo[sk][0]);
-                bl[buf][tb] = *reinterpret_cast<const bf16x8 *>(st + (256 + wm0 + 32 * tb) * 128 + fo[sk][1]);
-            }
+        for (int tb = 0; tb < 2; ++tb) {
+            bh[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 0);
+            bl[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 1);
         }
     };
     // the three products as three passes over the 8 accumulators: dependent products 8 apart
@@ -421,49 +316,32 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int np, i
                     acc[fb][tb] = mfma32x32x16(pr == 2 ? al[buf][fb] : ah[buf][fb], pr == 1 ? bl[buf][tb] : bh[buf][tb],
                                                acc[fb][tb]);
     };
-    if constexpr (RAW) {
-        // (a direction's copies number 2 or 8, so stage 0 lands and is split before stage 1 is issued: every
-        // later wait is for all copies in flight)
+    // (a direction's copies number 2 or 8, so stage 0 lands and is split before stage 1 is issued: every later wait
+    // is for all copies in flight)
+    if (nk > 0) {
         issue_raw(0);
         vm_wait<0>();
         asm volatile("" ::: "memory");
         split_raw(0);
         __syncthreads();
         if (nk > 1) issue_raw(1);
-    } else {
-        issue(0);
-        if (nk > 1) issue(1);
-        vm_wait_groups<8, 1>(nk > 1 ? 1 : 0);
-        __syncthreads();
+        fetch(0, lds, 0);
     }
-    fetch(0, lds, 0);
 #pragma unroll 1
     for (int ks = 0; ks < nk; ++ks) {
         const char *st = lds + (ks & 1) * kSt;
         fetch(1, st, 1);
         products(0);
-        if constexpr (RAW) {
-            // buffer: this wave splits its part of stage ks + 1 once its copies landed (nothing was issued after
-            // them), under the tail of this stage's products and with no fragments held
-            products(1);
-            if (ks + 1 < nk) {
-                vm_wait<0>();
-                asm volatile("" ::: "memory");
-                split_raw(ks + 1);
-                __syncthreads();  // stage ks + 1 split; every wave has read its fragments of stage ks
-                if (ks + 2 < nk) issue_raw(ks + 2);
-                fetch(0, lds + ((ks + 1) & 1) * kSt, 0);
-            }
-        } else {
-            if (ks + 1 < nk) {
-                // stage ks + 1 landed (nothing was issued after it); every wave has read its fragments of stage
-                // ks, whose buffer takes stage ks + 2
-                vm_wait<0>();
-                __syncthreads();
-                if (ks + 2 < nk) issue(ks + 2);
-                fetch(0, lds + ((ks + 1) & 1) * kUgStage, 0);
-            }
-            products(1);
+        // this wave splits its part of stage ks + 1 once its copies landed (nothing was issued after them), under the
+        // tail of this stage's products and with no fragments held
+        products(1);
+        if (ks + 1 < nk) {
+            vm_wait<0>();
+            asm volatile("" ::: "memory");
+            split_raw(ks + 1);
+            __syncthreads();  // stage ks + 1 split; every wave has read its fragments of stage ks
+            if (ks + 2 < nk) issue_raw(ks + 2);
+            fetch(0, lds + ((ks + 1) & 1) * kSt, 0);
         }
     }
     // lane (j, hf), register 4 g + e of block (fb, tb): row o = wn0 + 32 fb + 8 g + 4 hf + e, column
@@ -535,6 +413,68 @@ __global__ __launch_bounds__(256) void update_small_kernel(UpdateSmall s, int64_
     if (tid == 0) s.grad[p][el] = scale * red[0];
 }
 
+// Small parameters of at most kSmallWidth slice elements and kSmallEntries entries, many directions: a workgroup draws
+// each slice of its chunk of directions once into LDS (16 at a time, the weights folded into a's side) and every
+// thread adds up to four entries' products; the chunks' sums go to part [chunk][entry] and are summed in order by
+// update_small_reduce_kernel. One workgroup per entry (update_small_kernel) draws a and b again for each of the 256
+// entries of a gate, 13 times the normals: 131,072 directions of the model's 6 small parameters, 148 + 6 us
+// against 923; below
+// kSmallPairs its single launch is the shorter.
+constexpr int kSmallWidth = 512, kSmallEntries = 1024, kSmallDirs = 16;
+constexpr int64_t kSmallPairs = 4096;
+__global__ __launch_bounds__(256) void update_small_partial_kernel(UpdateSmall s, int64_t pairs, int64_t chunk,
+                                                                   int entries, const float *__restrict__ weight,
+                                                                   DrawLayout dl, int64_t numel,
+                                                                   float *__restrict__ part) {
+    __shared__ float sm[kSmallDirs * kSmallWidth];
+    const int p = blockIdx.y, tid = threadIdx.x;
+    const int rows = s.rows[p], cols = s.cols[p], width = rows + cols, n = rows * (cols ? cols : 1);
+    const int64_t *off = s.offsets[p];
+    const int64_t d0 = blockIdx.x * chunk, d1 = d0 + chunk < pairs ? d0 + chunk : pairs;
+    float acc[kSmallEntries / 256];
+#pragma unroll
+    for (int q = 0; q < kSmallEntries / 256; ++q) acc[q] = 0.0f;
+    for (int64_t d = d0; d < d1; d += kSmallDirs) {
+        const int m = d1 - d < kSmallDirs ? (int)(d1 - d) : kSmallDirs;
+        for (int i = tid; i < m * width; i += 256) {
+            const int k = i / width, r = i - k * width;
+            const float v = noise_at(dl, off[d + k] + r, numel);
+            sm[k * width + r] = r < rows ? weight[d + k] * v : v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kSmallEntries / 256; ++q) {
+            const int e = 256 * q + tid;
+            if (e < n) {
+                const int o = cols ? e / cols : e, i = cols ? rows + e % cols : 0;
+                for (int k = 0; k < m; ++k) acc[q] += sm[k * width + o] * (cols ? sm[k * width + i] : 1.0f);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kSmallEntries / 256; ++q)
+        if (256 * q + tid < n) part[(int64_t)blockIdx.x * entries + s.start[p] + 256 * q + tid] = acc[q];
+}
+
+// scale * the chunks' sums of one entry per workgroup, a fixed-order tree
+__global__ __launch_bounds__(256) void update_small_reduce_kernel(UpdateSmall s, int chunks, int entries, float scale,
+                                                                  const float *__restrict__ part) {
+    __shared__ float red[256];
+    const int e = blockIdx.x, tid = threadIdx.x;
+    int p = 0;
+    while (p + 1 < s.n && s.start[p + 1] <= e) ++p;
+    float acc = 0.0f;
+    for (int c = tid; c < chunks; c += 256) acc += part[(int64_t)c * entries + e];
+    red[tid] = acc;
+    __syncthreads();
+    for (int st = 128; st > 0; st >>= 1) {
+        if (tid < st) red[tid] += red[tid + st];
+        __syncthreads();
+    }
+    if (tid == 0) s.grad[p][e - s.start[p]] = scale * red[0];
+}
+
 bool is_big(const noise_update_param_t &q) {
     return q.cols > 0 && q.rows % kTile == 0 && q.cols % kTile == 0;
 }
@@ -599,7 +539,7 @@ extern "C" int64_t noise_update_workspace_bytes(const noise_update_param_t *para
             bytes += (params[i].rows + params[i].cols) * 2 * np * 2;
             tiles += (params[i].rows / kTile) * (params[i].cols / kTile);
         }
-    // the tables, then the GEMM's partial tiles for a device of 256 compute units
+    // the slabs, then the GEMM's partial tiles for a device of 256 compute units
     int64_t full;
     int split;
     gemm_split(tiles, 256, full, split);
@@ -621,7 +561,6 @@ extern "C" int noise_update_gradients(const noise_update_param_t *params, int np
     NOISE_CHECK_ARG(numel > 0, "noise_update_gradients: numel must be positive");
     NOISE_CHECK_ARG(buffer == nullptr || aligned(buffer, 4), "noise_update_gradients: buffer must be 4-byte aligned");
     const int64_t np = padded_chunk(chunk, pairs);
-    // (the GEMM's 32-bit copy offsets span 64 table rows of 2 np elements)
     NOISE_CHECK_ARG(np <= (1 << 22), "noise_update_gradients: chunk too large (at most 4194304 directions)");
     UpdateSet big{};
     UpdateSmall small{};
@@ -643,7 +582,7 @@ extern "C" int noise_update_gradients(const noise_update_param_t *params, int np
             big.cols[b] = (int)q.cols;
             big.row_start[b] = (int)rows_total;
             big.tile_start[b] = (int)tiles_total;
-            big.table[b] = reinterpret_cast<__bf16 *>(ws + need);
+            big.slab[b] = reinterpret_cast<float *>(ws + need);
             rows_total += q.rows + q.cols;
             tiles_total += (q.rows / kTile) * (q.cols / kTile);
             need += (q.rows + q.cols) * 2 * np * 2;
@@ -671,7 +610,7 @@ extern "C" int noise_update_gradients(const noise_update_param_t *params, int np
                     "see noise_update_workspace_bytes", (long long)need, (long long)workspace_bytes);
     DrawLayout dl{seed, offset, (uint64_t)threads};
     hipStream_t s = (hipStream_t)stream;
-    // the GEMM's partial tiles after the tables, when the workspace holds them (else whole tiles only)
+    // the GEMM's partial tiles after the slabs, when the workspace holds them (else whole tiles only)
     int64_t full;
     int split;
     gemm_split(tiles_total, device_cus(), full, split);
@@ -680,36 +619,48 @@ extern "C" int noise_update_gradients(const noise_update_param_t *params, int np
         if (split == 1) full = tiles_total;
     }
     float *part = split > 1 ? reinterpret_cast<float *>(ws + need) : nullptr;
-    if (small.n) {
+    bool shared_slices = pairs >= kSmallPairs;
+    for (int i = 0; i < small.n; ++i) {
+        const int64_t cols = small.cols[i], n = small.rows[i] * (cols ? cols : 1);
+        shared_slices = shared_slices && small.rows[i] + cols <= kSmallWidth && n <= kSmallEntries;
+    }
+    // 512 chunks of directions (whole steps of kSmallDirs); their sums use the slabs' area, which is written later
+    const int64_t chunk_small = ((pairs + 511) / 512 + kSmallDirs - 1) / kSmallDirs * kSmallDirs;
+    const int64_t chunks_small = (pairs + chunk_small - 1) / chunk_small;
+    if (small.n && shared_slices && chunks_small * entries_total * (int64_t)sizeof(float) <= need) {
+        hipLaunchKernelGGL(update_small_partial_kernel, dim3((unsigned)chunks_small, (unsigned)small.n), dim3(256), 0, s,
+                           small, pairs, chunk_small, (int)entries_total, weight, dl, numel, reinterpret_cast<float *>(ws));
+        hipLaunchKernelGGL(update_small_reduce_kernel, dim3((unsigned)entries_total), dim3(256), 0, s, small,
+                           (int)chunks_small, (int)entries_total, scale, reinterpret_cast<const float *>(ws));
+        int st = launch_status("noise_update_gradients (small parameters)");
+        if (st) return st;
+    } else if (small.n) {
         hipLaunchKernelGGL(update_small_kernel, dim3((unsigned)entries_total), dim3(256), 0, s, small, pairs, weight,
                            scale, dl, numel);
         int st = launch_status("noise_update_gradients (small parameters)");
         if (st) return st;
     }
     if (big.n) {
-        // with a buffer of at most 2^30 elements the GEMM reads the slices itself; otherwise tables first
+        // with a buffer of at most 2^30 elements the GEMM reads the slices itself; otherwise they are written out first
         const bool direct = buffer != nullptr && numel <= (1ll << 30);
         for (int64_t d0 = 0; d0 < pairs; d0 += np) {
             const int64_t n = pairs - d0 < np ? pairs - d0 : np;
             const int64_t wgs = full + (tiles_total - full) * split;
             int st;
-            if (direct) {
-                const UpdateRaw raw{d0, n, weight, scale, buffer, numel};
-                hipLaunchKernelGGL(update_gemm_kernel<true>, dim3((unsigned)wgs), dim3(512), 0, s, big, (int)np,
-                                   d0 > 0 ? 1 : 0, (int)full, split, part, raw);
-            } else {
+            if (!direct) {
+                // the directions shared out so that some 16 K workgroups are in the launch
+                const int64_t cols = rows_total / 256, share = 16384 / cols + 1;
+                const dim3 grid((unsigned)cols, (unsigned)(n < share ? n : share));
                 if (buffer)
-                    hipLaunchKernelGGL(update_tables_from_buffer_kernel, dim3((unsigned)(rows_total / 256),
-                                       (unsigned)(np / kTabK)), dim3(256), 0, s, big, d0, n, np, weight, scale, buffer,
-                                       numel);
+                    hipLaunchKernelGGL(update_slices_kernel<true>, grid, dim3(256), 0, s, big, d0, n, dl, buffer, numel);
                 else
-                    hipLaunchKernelGGL(update_tables_kernel, dim3((unsigned)rows_total, (unsigned)(np / 256)),
-                                       dim3(256), 0, s, big, d0, n, np, weight, scale, dl, numel);
-                st = launch_status("noise_update_gradients (tables)");
+                    hipLaunchKernelGGL(update_slices_kernel<false>, grid, dim3(256), 0, s, big, d0, n, dl, buffer, numel);
+                st = launch_status("noise_update_gradients (slices)");
                 if (st) return st;
-                hipLaunchKernelGGL(update_gemm_kernel<false>, dim3((unsigned)wgs), dim3(512), 0, s, big, (int)np,
-                                   d0 > 0 ? 1 : 0, (int)full, split, part, UpdateRaw{});
             }
+            const UpdateRaw raw{d0, n, weight, scale, direct ? buffer : nullptr, numel};
+            hipLaunchKernelGGL(update_gemm_kernel, dim3((unsigned)wgs), dim3(512), 0, s, big, d0 > 0 ? 1 : 0, (int)full,
+                               split, part, raw);
             st = launch_status("noise_update_gradients (gemm)");
             if (st) return st;
             if (split > 1) {
