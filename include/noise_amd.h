@@ -116,7 +116,8 @@ int noise_orthogonal_draws(void *out, int out_bf16, int64_t n, int64_t bt, int64
  * q, k, o: element (b, t, h, d) at b*s_b + h*s_h + t*s_t + d (the reference's [B, T, H, D] and its
  * transposes are all expressible). v: the same with vs_x = token stride, or, with flag
  * NOISE_ATTN_V_TRANSPOSED, element (b, t, h, d) at b*vs_b + h*vs_h + d*vs_x + t. head_dim must be 64.
- * A seq in whole 256-query tiles runs the ring kernel with either V layout, other lengths the general one.
+ * Natural V runs the ring kernel at any seq, transposed V at a seq in whole 256-query tiles; the rest the general one.
+ * NOISE_ATTN_OUT_FP32 (natural V): o is fp32 (strides in its elements, multiples of 4) holding the bf16 results.
  * NOISE_ATTN_QK_NORMED: the caller guarantees every q and k row has RMS <= 1, as RMSNorm outputs do (the
  * reference normalises both, utils/model.py:94); scores are then bounded and the softmax runs with a
  * fixed shift instead of a running maximum (same result; rows that break the promise by less than a
@@ -126,6 +127,18 @@ int noise_orthogonal_draws(void *out, int out_bf16, int64_t n, int64_t bt, int64
  * (eggroll.py:58), NULL to skip. */
 #define NOISE_ATTN_V_TRANSPOSED 1
 #define NOISE_ATTN_QK_NORMED 2
+#define NOISE_ATTN_OUT_FP32 4
+
+/* Up to three fp32 tensors [batch, tokens, heads, 64] (element (b, t, h, d) of tensor i at src[i] + b*s_b[i] + t*s_t[i] +
+ * h*s_h[i] + d) rounded to bf16 [batch][tokens][heads][64] in one launch: noise_attention_fwd's operands. */
+typedef struct {
+    int32_t count;
+    const float *src[3];
+    void *dst[3];
+    int64_t s_b[3], s_t[3], s_h[3];
+} noise_cast_heads_t;
+int noise_cast_heads(const noise_cast_heads_t *cast, int64_t batch, int64_t tokens, int64_t heads,
+                     noise_stream_t stream);
 
 /* V element (b, t, h, d) at b*vs_b + h*vs_h + t*vs_t + d -> vt [batch][heads][64][seq] contiguous, the
  * NOISE_ATTN_V_TRANSPOSED layout that the population path writes (no counterpart in the reference; a layout

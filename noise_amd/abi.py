@@ -18,6 +18,7 @@ SIGNATURES = {
     'noise_orthogonal_draws': [_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _p],
     'noise_attention_fwd': [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                             _i64, _i64, _i64, _i32, _i64, _i64, _i64, _i64, _f32, _p, _i64, _i64, _p, _p],
+    'noise_cast_heads': [_p, _i64, _i64, _i64, _p],
     'noise_v_transpose': [_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p],
     'noise_pop_embed': [_p, _i32, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p],
     'noise_member_dots': [_p, 'View', _i64, _p, _i64, _p, _p],
@@ -82,6 +83,7 @@ ROUNDING_EAGER = 1
 # noise_attention_fwd flags (include/noise_amd.h)
 ATTN_V_TRANSPOSED = 1
 ATTN_QK_NORMED = 2
+ATTN_OUT_FP32 = 4
 
 
 class View(ctypes.Structure):
@@ -128,6 +130,12 @@ class Weight(ctypes.Structure):
     """noise_weight_t: one parameter's copies of noise_weights_prepare."""
     _fields_ = [('src', ctypes.c_void_p), ('dst', ctypes.c_void_p), ('dst_block', ctypes.c_void_p),
                 ('numel', ctypes.c_int64), ('src_bf16', ctypes.c_int32), ('kind', ctypes.c_int32)]
+
+
+class CastHeads(ctypes.Structure):
+    """noise_cast_heads_t: up to three fp32 [batch, tokens, heads, 64] tensors to round to bf16."""
+    _fields_ = [('count', ctypes.c_int32), ('src', ctypes.c_void_p * 3), ('dst', ctypes.c_void_p * 3),
+                ('s_b', ctypes.c_int64 * 3), ('s_t', ctypes.c_int64 * 3), ('s_h', ctypes.c_int64 * 3)]
 
 
 class BlockJitter(ctypes.Structure):

@@ -10,11 +10,12 @@
 // 64-key tile with v_mfma_f32_32x32x16_bf16 (4 k-steps over D = 64), so a lane holds the scores of one
 // query and row reductions need one exchange with lane ^ 32; P is fed from registers as the B operand of
 // O^T = V^T P^T with the key index permuted identically on both sides, so P never touches LDS.
-//  - attention_fwd_kernel (any layout and length): 4 waves of 64 queries, K / V tiles register-staged
+//  - attention_fwd_kernel (V transposed with a length off the 256-query tiles, or row strides the ring's 32-bit
+//    copy offsets do not span): 4 waves of 64 queries, K / V tiles register-staged
 //    into double-buffered LDS (rows padded to 144 B), running-max softmax (rescaled only when the maximum
 //    grows by more than 2^8).
-//  - attention_vt_kernel (length a multiple of 256; V transposed, the population path, or natural, the
-//    drop-in's): 8 waves of 32 queries (four waves per SIMD) in two groups half a tile apart, K and V (or V^T)
+//  - attention_vt_kernel (V transposed, the population path, at lengths in whole 256-query tiles; or natural, the
+//    drop-in's, at any length): 8 waves of 32 queries (four waves per SIMD) in two groups half a tile apart, K and V (or V^T)
 //    copied global -> LDS into a four-stage swizzled ring, and an optional fixed-shift softmax for RMS-normed
 //    q, k (described at the kernel).
 // Key tiles outside a wave's band are skipped; masking runs only on band-edge tiles. All query tiles of
@@ -306,7 +307,7 @@ __device__ __forceinline__ int key_sigma(int i) { return (i & ~12) | ((i & 4) <<
 // the slot of tile t - 1, which B finished reading before that barrier.
 // VNAT: V in its natural layout [.., token, dim] (the drop-in's), copied as K is, with the 16 B chunks of row R
 // swizzled by 2 (R % 4) instead, and each V^T fragment put together from two transposing LDS reads.
-template <bool BOUNDED, bool VNAT>
+template <bool BOUNDED, bool VNAT, bool OF32 = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_vt_kernel(AttnArgs a) {
     constexpr int QT = kVtQT, NS = 4;
     constexpr int QB = 1, NW = QT / 32, QW = 32, CPW = 4;  // waves, queries per wave, copies per A wave
@@ -335,12 +336,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int j = lane & 31, hf = lane >> 5;
     const int T = a.seq, W = a.window;
     const int q0w = qt * QT + wave * QW;
+    // VNAT takes any length: rows past the last token are the last token's (queries there are not stored, and keys there
+    // are visible to no query before them)
+    const int last = T - 1;
 
     bf16x8 qf[QB][4];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) qf[qb][s] = load_bf16x8(Qb + (int64_t)(q0w + 32 * qb + j) * a.qs_t + 16 * s + 8 * hf);
+        for (int s = 0; s < 4; ++s) {
+            const int q = q0w + 32 * qb + j;
+            qf[qb][s] = load_bf16x8(Qb + (int64_t)(VNAT && q > last ? last : q) * a.qs_t + 16 * s + 8 * hf);
+        }
     // the query fragments land before any tile copy is issued: the compiler's own wait for them inside the
     // tile loop would otherwise be a vmcnt that also drains the copies in flight
     vm_wait<0>();
@@ -369,6 +376,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const unsigned voff = (unsigned)((lane >> 3) * a.vs_x * 2 + vchunk * 16);
     const unsigned lb = lds_addr(lds);
     auto issue = [&](int k0, unsigned st) {  // st: LDS byte address of the stage
+        if (VNAT && k0 + kBKV > T) {
+            // the tile that holds the last token: each lane's row is clamped (row strides below 2^25 elements)
+#pragma unroll
+            for (int i = 0; i < CPW; ++i) {
+                const int c = 4 * i + wave, r = 8 * (c & 7) + (lane >> 3);
+                const unsigned row = (unsigned)(k0 + r > last ? last - k0 : r);
+                if (c < 8)
+                    lds_dma16_at(Kb + (int64_t)k0 * a.ks_t, row * (unsigned)a.ks_t * 2 + chunk * 16, st + c * 1024);
+                else
+                    lds_dma16_at(Vb + (int64_t)k0 * a.vs_x, row * (unsigned)a.vs_x * 2 + vchunk * 16, st + c * 1024);
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < CPW; ++i) {
             const int c = 4 * i + wave;  // A waves only: copy c's row parity is the wave's
@@ -406,11 +426,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
 
     const int wg_q_lo = qt * QT;
-    const int wg_q_hi = wg_q_lo + QT - 1;
+    const int wg_q_hi = VNAT ? min(wg_q_lo + QT - 1, last) : wg_q_lo + QT - 1;
     const int kv_first = max(0, wg_q_lo - W) / kBKV;
     const int kv_last = wg_q_hi / kBKV;
     const int nt = kv_last - kv_first + 1;
-    const int wq_lo = q0w, wq_hi = q0w + QW - 1;
+    // (a wave whose queries all lie past the last token has no active tile)
+    const int wq_lo = q0w, wq_hi = VNAT ? (q0w > last ? -1 : min(q0w + QW - 1, last)) : q0w + QW - 1;
     const float c2 = a.scale_log2, shift = a.shift;
 
     f32x16 sc[2][QB];
@@ -599,46 +620,104 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         const float inv = 1.0f / lt;  // the diagonal key is always visible: lt > 0
         float dsum = 0.f;
         const float *dv = a.dot ? a.dvec + (int64_t)(b / a.ddiv) * a.ds_b + h * kD : nullptr;
-        __bf16 *orow = a.o + b * a.os_b + h * a.os_h + (int64_t)q * a.os_t;
-        // with 16 B aligned output rows the wave's 32 x 64 block is staged in LDS (the K / V ring, free once
-        // both groups are past their last tile) and stored as whole 128 B row segments: in the MFMA layout
-        // one 8 B store would touch 32 rows
-        constexpr int kOP = 72;  // staging row pitch (bf16)
-        static_assert(QB == 1, "one staging block per wave");
-        __bf16 *stg = reinterpret_cast<__bf16 *>(lds) + wave * 32 * kOP;
-        if (a.o_lines) __syncthreads();
-        __bf16 *dst = a.o_lines ? stg + j * kOP : orow;
+        if constexpr (OF32) {
+            // fp32 rows holding the bf16 results: the wave's 32 x 64 block through LDS ([32 rows][16 chunks of 4 dims],
+            // chunk c of row r at c ^ (r % 16)), stored as whole 256 B rows
+            char *stg = lds + wave * (32 * 256);
+            __syncthreads();
 #pragma unroll
-        for (int db = 0; db < 2; ++db)
+            for (int db = 0; db < 2; ++db)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                bf16x4 v;
+                for (int g = 0; g < 4; ++g) {
+                    const int c = 8 * db + 2 * g + hf;
+                    float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = (__bf16)(o[db][qb][4 * g + e] * inv);
-                const int d = 32 * db + 8 * g + 4 * hf;
-                store_bf16x4(dst + d, v);
-                if (dv) {
+                    for (int e = 0; e < 4; ++e) v[e] = bfr(o[db][qb][4 * g + e] * inv);
+                    *reinterpret_cast<float4 *>(stg + j * 256 + ((c ^ (j & 15)) << 4)) = float4{v[0], v[1], v[2], v[3]};
+                    if (dv) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) dsum += (float)v[e] * dv[d + e];
+                        for (int e = 0; e < 4; ++e) dsum += v[e] * dv[4 * c + e];
+                    }
                 }
-            }
-        if (a.o_lines) {
             wave_lds_sync();
-            __bf16 *ob = a.o + b * a.os_b + h * a.os_h + (int64_t)(q0w + 32 * qb) * a.os_t;
+            float *ob = reinterpret_cast<float *>(a.o) + b * a.os_b + h * a.os_h;
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int c = it * 64 + lane, r = c >> 3, ch = c & 7;
-                store_bf16x8(ob + (int64_t)r * a.os_t + ch * 8, load_bf16x8(stg + r * kOP + ch * 8));
+            for (int it = 0; it < 8; ++it) {
+                const int r = 4 * it + (lane >> 4), ch = lane & 15;
+                if (q0w + r <= last)
+                    *reinterpret_cast<float4 *>(ob + (int64_t)(q0w + r) * a.os_t + 4 * ch) =
+                        *reinterpret_cast<const float4 *>(stg + r * 256 + ((ch ^ (r & 15)) << 4));
+            }
+        } else {
+            __bf16 *orow = a.o + b * a.os_b + h * a.os_h + (int64_t)q * a.os_t;
+            const bool live = !VNAT || q <= last;
+            // with 16 B aligned output rows the wave's 32 x 64 block is staged in LDS (the K / V ring, free once
+            // both groups are past their last tile) and stored as whole 128 B row segments: in the MFMA layout
+            // one 8 B store would touch 32 rows
+            constexpr int kOP = 72;  // staging row pitch (bf16)
+            static_assert(QB == 1, "one staging block per wave");
+            __bf16 *stg = reinterpret_cast<__bf16 *>(lds) + wave * 32 * kOP;
+            if (a.o_lines) __syncthreads();
+            __bf16 *dst = a.o_lines ? stg + j * kOP : orow;
+#pragma unroll
+            for (int db = 0; db < 2; ++db)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    bf16x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (__bf16)(o[db][qb][4 * g + e] * inv);
+                    const int d = 32 * db + 8 * g + 4 * hf;
+                    if (a.o_lines || live) store_bf16x4(dst + d, v);
+                    if (dv) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) dsum += (float)v[e] * dv[d + e];
+                    }
+                }
+            if (a.o_lines) {
+                wave_lds_sync();
+                __bf16 *ob = a.o + b * a.os_b + h * a.os_h + (int64_t)(q0w + 32 * qb) * a.os_t;
+#pragma unroll
+                for (int it = 0; it < 4; ++it) {
+                    const int c = it * 64 + lane, r = c >> 3, ch = c & 7;
+                    if (!VNAT || q0w + 32 * qb + r <= last)
+                        store_bf16x8(ob + (int64_t)r * a.os_t + ch * 8, load_bf16x8(stg + r * kOP + ch * 8));
+                }
             }
         }
         if (a.dot) {
             dsum += swap_halves(dsum);
-            if (hf == 0) a.dot[((int64_t)b * T + q) * a.heads + h] = dsum;
+            if (hf == 0 && (!VNAT || q <= last)) a.dot[((int64_t)b * T + q) * a.heads + h] = dsum;
         }
     }
 }
 
 
+
+// Up to three fp32 tensors [b, t, h, 64] (unit inner stride) -> bf16 [b][t][h][64] contiguous, 8 dims per thread.
+// grid = (chunks / 256, tensors)
+struct CastArgs {
+    const float *src[3];
+    int64_t s_b[3], s_t[3], s_h[3];
+    __bf16 *dst[3];
+    int wide[3];       // 16 B aligned rows
+    int64_t tokens, heads, chunks;
+};
+__global__ __launch_bounds__(256) void cast_heads_kernel(CastArgs p) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= p.chunks) return;
+    const int k = blockIdx.y;
+    const int64_t row = i >> 3, bt = row / p.heads, h = row - bt * p.heads, b = bt / p.tokens, t = bt - b * p.tokens;
+    const float *s = p.src[k] + b * p.s_b[k] + t * p.s_t[k] + h * p.s_h[k] + 8 * (i & 7);
+    bf16x8 o;
+    if (p.wide[k]) {
+        const float4 x = *reinterpret_cast<const float4 *>(s), y = *reinterpret_cast<const float4 *>(s + 4);
+        o = bf16x8{(__bf16)x.x, (__bf16)x.y, (__bf16)x.z, (__bf16)x.w, (__bf16)y.x, (__bf16)y.y, (__bf16)y.z, (__bf16)y.w};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (__bf16)s[e];
+    }
+    store_bf16x8(p.dst[k] + 8 * i, o);
+}
 
 // V [b, t, h, d] (d contiguous) -> V^T [b][h][d][t]: one workgroup per (b*h, 64-token tile); each thread
 // reads two 16 B pieces of token rows and writes two 16 B pieces of dim rows through a padded LDS tile.
@@ -687,6 +766,28 @@ extern "C" int noise_v_transpose(const void *v, int64_t batch, int64_t heads, in
     return launch_status("noise_v_transpose");
 }
 
+extern "C" int noise_cast_heads(const noise_cast_heads_t *cast, int64_t batch, int64_t tokens, int64_t heads,
+                                noise_stream_t stream) {
+    clear_error();
+    const char *fn = "noise_cast_heads";
+    NOISE_CHECK_ARG(cast && cast->count >= 1 && cast->count <= 3, "%s: 1 .. 3 tensors", fn);
+    NOISE_CHECK_ARG(batch >= 0 && tokens >= 0 && heads > 0, "%s: bad batch/tokens/heads", fn);
+    CastArgs p;
+    p.tokens = tokens; p.heads = heads; p.chunks = batch * tokens * heads * (kD / 8);
+    if (p.chunks == 0) return NOISE_OK;
+    NOISE_CHECK_ARG((p.chunks + 255) / 256 <= INT32_MAX, "%s: too many rows", fn);
+    for (int i = 0; i < cast->count; ++i) {
+        NOISE_CHECK_ARG(cast->src[i] && cast->dst[i] && aligned(cast->src[i], 4) && aligned(cast->dst[i], 16),
+                        "%s: tensor %d NULL or misaligned", fn, i);
+        p.src[i] = cast->src[i]; p.dst[i] = (__bf16 *)cast->dst[i];
+        p.s_b[i] = cast->s_b[i]; p.s_t[i] = cast->s_t[i]; p.s_h[i] = cast->s_h[i];
+        p.wide[i] = aligned(cast->src[i], 16) && p.s_b[i] % 4 == 0 && p.s_t[i] % 4 == 0 && p.s_h[i] % 4 == 0;
+    }
+    hipLaunchKernelGGL(cast_heads_kernel, dim3((unsigned)((p.chunks + 255) / 256), (unsigned)cast->count), dim3(256), 0,
+                       (hipStream_t)stream, p);
+    return launch_status(fn);
+}
+
 extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, void *o, int64_t batch,
                                    int64_t heads, int64_t seq, int64_t head_dim, int64_t qs_b, int64_t qs_h,
                                    int64_t qs_t, int64_t ks_b, int64_t ks_h, int64_t ks_t, int64_t vs_b,
@@ -695,7 +796,7 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
                                    int64_t dot_vec_stride, int64_t dot_div, float *dot_out,
                                    noise_stream_t stream) {
     clear_error();
-    NOISE_CHECK_ARG((flags & ~(NOISE_ATTN_V_TRANSPOSED | NOISE_ATTN_QK_NORMED)) == 0,
+    NOISE_CHECK_ARG((flags & ~(NOISE_ATTN_V_TRANSPOSED | NOISE_ATTN_QK_NORMED | NOISE_ATTN_OUT_FP32)) == 0,
                     "noise_attention_fwd: unknown flags 0x%x", flags);
     const bool v_transposed = flags & NOISE_ATTN_V_TRANSPOSED;
     NOISE_CHECK_ARG(head_dim == kD, "noise_attention_fwd: head_dim must be 64, got %lld", (long long)head_dim);
@@ -718,8 +819,13 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     NOISE_CHECK_ARG(dot_out == nullptr || (dot_vec != nullptr && dot_div >= 1),
                     "noise_attention_fwd: dot_out needs dot_vec and dot_div >= 1");
     int64_t bh = batch * heads;
-    // lengths in whole 256-query tiles run the ring kernel, with V in either layout
-    const bool vt_path = seq % kVtQT == 0;
+    // the ring kernel takes natural V at any length (its copies of the last, clamped tile span 63 row strides by 32-bit
+    // byte offsets) and transposed V in whole 256-query tiles: 5 x 8 heads x 1111 tokens, window 500, 22 us
+    // against 45 by the register-staged kernel; 8 heads x 100 tokens, 6.7 against 11.5
+    const bool vt_path = v_transposed ? seq % kVtQT == 0 : ks_t < (1 << 25) && vs_x < (1 << 25) && ks_t >= 0 && vs_x >= 0;
+    const bool out_fp32 = flags & NOISE_ATTN_OUT_FP32;
+    NOISE_CHECK_ARG(!out_fp32 || (vt_path && !v_transposed && aligned(o, 16)),
+                    "noise_attention_fwd: fp32 output needs natural v, row strides below 2^25 and o 16 B aligned");
     const int64_t qtile = vt_path ? kVtQT : kBQ;
     int64_t qtiles = (seq + qtile - 1) / qtile;
     NOISE_CHECK_ARG(bh * qtiles < (1ll << 31), "noise_attention_fwd: too many workgroups");
@@ -743,7 +849,8 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     dim3 grid((unsigned)(bh * qtiles));
     if (vt_path) {
         const bool bounded = flags & NOISE_ATTN_QK_NORMED;
-        auto kernel = v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
+        auto kernel = out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
+                      : v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
                                    : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>);
         hipLaunchKernelGGL(kernel, grid, dim3(512), 0, (hipStream_t)stream, a);
     } else if (v_transposed)

@@ -4,6 +4,7 @@ attention(q, k, v, window)  replaces utils/model.py:24-31 (flex_attention over t
 GPTConfig / GPT / make_model hold the same parameters under the same state-dict names as
 utils/model.py:34-175 and train/val/eggroll.py:38-53, so weights load strictly either way.
 """
+import ctypes
 import math
 from dataclasses import dataclass
 
@@ -11,7 +12,7 @@ import torch
 from torch import nn
 
 from . import _lib
-from ._lib import ATTN_QK_NORMED, ATTN_V_TRANSPOSED
+from ._lib import ATTN_OUT_FP32, ATTN_QK_NORMED, ATTN_V_TRANSPOSED
 
 BF16 = torch.bfloat16
 N_LAYER, N_HEAD, HEAD_DIM, N_EMBD, VOCAB, SEQ = 8, 8, 64, 512, 4096, 2048
@@ -164,15 +165,32 @@ def attention(q, k, v, window):
     if not (q.is_cuda and k.is_cuda and v.is_cuda):
         raise ValueError('attention: tensors must be on a GPU')
     B, T, H, D = q.shape
-    qb, kb, vb = _operand(q), _operand(k), _operand(v)
-    out = torch.empty(B, T, H, D, dtype=BF16, device=q.device)
-    # V in its own layout: lengths in whole 256-query tiles run the ring kernel, which reads V^T fragments
-    # from natural V tiles with transposing LDS reads; other lengths run the general kernel
+    stream = _lib.stream_ptr(q.device)
+    ops, cast, n = [q, k, v], None, 0
+    for i, t in enumerate(ops):
+        if t.dtype == torch.float32 and D == HEAD_DIM and t.stride(-1) == 1:
+            # fp32 operands are rounded together, in one launch
+            if cast is None:
+                cast = _lib.CastHeads()
+            ops[i] = torch.empty(B, T, H, D, dtype=BF16, device=t.device)
+            cast.src[n], cast.dst[n] = t.data_ptr(), ops[i].data_ptr()
+            cast.s_b[n], cast.s_t[n], cast.s_h[n] = t.stride()[:3]
+            n += 1
+        else:
+            ops[i] = _operand(t)
+    if n:
+        cast.count = n
+        _lib.call('noise_cast_heads', ctypes.byref(cast), B, T, H, stream)
+    qb, kb, vb = ops
+    ks, vs = kb.stride(), vb.stride()
+    # V in its own layout: the ring kernel reads V^T fragments from natural V tiles with transposing LDS reads
+    fp32 = q.dtype == torch.float32 and max(ks[1], vs[1]) < 1 << 25
+    out = torch.empty(B, T, H, D, dtype=torch.float32 if fp32 else BF16, device=q.device)
+    qs, os = qb.stride(), out.stride()
     _lib.call('noise_attention_fwd', qb.data_ptr(), kb.data_ptr(), vb.data_ptr(), out.data_ptr(), B, H, T, D,
-              qb.stride(0), qb.stride(2), qb.stride(1), kb.stride(0), kb.stride(2), kb.stride(1),
-              vb.stride(0), vb.stride(2), vb.stride(1), 0, out.stride(0), out.stride(2), out.stride(1),
-              int(window), 1.0 / math.sqrt(D), None, 0, 1, None, _lib.stream_ptr(q.device))
-    return out if q.dtype == BF16 else out.to(q.dtype)
+              qs[0], qs[2], qs[1], ks[0], ks[2], ks[1], vs[0], vs[2], vs[1], ATTN_OUT_FP32 if fp32 else 0,
+              os[0], os[2], os[1], int(window), 1.0 / math.sqrt(D), None, 0, 1, None, stream)
+    return out if out.dtype == q.dtype else out.to(q.dtype)
 
 
 def attention_raw(q, k, v, out, window, v_transposed=False, dot_vec=None, dot_div=1, dot_out=None,

@@ -1,0 +1,62 @@
+"""The attention drop-in (utils/model.py:24-31) at lengths on and off its 64-key and 256-query tiles, with the strides
+and dtypes its operands pass takes, against a dense fp32 softmax of the bf16 operands: bf16 weights and output round
+each value by 2^-9 of itself, so errors stay within 2e-2 of the largest value (the bar of the fixed-length tests). Rows
+past the last token must neither be read (the tensors end there) nor written."""
+import pytest
+import torch
+
+from tests.test_attention_gpu import DEV, fp32_reference_gpu, rel_ok
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('T', [1, 2, 31, 32, 33, 63, 64, 65, 100, 255, 257, 320, 511, 1111])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_lengths(T, dtype):
+    from noise_amd.model import attention
+    for B, H, window in ((1, 1, T), (2, 8, 40), (3, 5, 0)):
+        print(B, T, H, window, dtype, flush=True)
+        g = torch.Generator(DEV).manual_seed(T)
+        q, k, v = (torch.randn(B, T, H, 64, device=DEV, generator=g).to(dtype) for _ in range(3))
+        out = attention(q, k, v, window)
+        assert out.dtype == dtype and out.is_contiguous()
+        rel_ok(out, fp32_reference_gpu(q.bfloat16(), k.bfloat16(), v.bfloat16(), window))
+        assert torch.equal(attention(q.bfloat16(), k.bfloat16(), v.bfloat16(), window).to(dtype), out)
+
+
+def test_views_and_dtypes():
+    from noise_amd.model import attention
+    g = torch.Generator(DEV).manual_seed(9)
+    B, T, H = 2, 203, 3
+    qkv = torch.randn(B, T, 3, H, 64, device=DEV, generator=g)
+    wide = torch.randn(B, T, H, 3 * 64 + 1, device=DEV, generator=g)
+    cases = [qkv.unbind(2), qkv.bfloat16().unbind(2), [qkv[:, :, 0], qkv[:, :, 1].bfloat16(), qkv[:, :, 2].half()],
+             [qkv[:, :, 0].half(), qkv[:, :, 1], qkv[:, :, 2].double()], [wide[..., i + 1:i + 65] for i in (0, 64, 128)],
+             [t.transpose(1, 2).contiguous().transpose(1, 2) for t in qkv.unbind(2)],
+             [t.transpose(2, 3).contiguous().transpose(2, 3) for t in qkv.unbind(2)],
+             [qkv[:1, :, i].expand(B, T, H, 64) for i in range(3)]]
+    for q, k, v in cases:
+        print([(t.dtype, t.stride()) for t in (q, k, v)], flush=True)
+        out = attention(q, k, v, 90)
+        assert out.dtype == q.dtype
+        rel_ok(out, fp32_reference_gpu(q.bfloat16(), k.bfloat16(), v.bfloat16(), 90))
+
+
+@pytest.mark.parametrize('flags', [0, 2, 4, 6])
+def test_rows_past_the_end_are_not_written(flags):
+    from noise_amd import _lib
+    g = torch.Generator(DEV).manual_seed(4)
+    B, T, H, pad = 2, 131, 2, 200
+    q, k, v = (torch.nn.functional.rms_norm(torch.randn(B, T, H, 64, device=DEV, generator=g), (64,)).bfloat16()
+               for _ in range(3))
+    out = torch.full((B, T + pad, H, 64), 9.0, device=DEV, dtype=torch.float32 if flags & 4 else torch.bfloat16)
+    dots, vec = torch.full((B * T * H + 64,), 9.0, device=DEV), torch.randn(B, H * 64, device=DEV, generator=g)
+    s = [x for t in (q, k, v) for x in (t.stride(0), t.stride(2), t.stride(1))]
+    _lib.call('noise_attention_fwd', q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, T, 64, *s, flags,
+              out.stride(0), out.stride(2), out.stride(1), 77, 0.125, vec.data_ptr(), H * 64, 1, dots.data_ptr(),
+              _lib.stream_ptr(DEV))
+    ref = fp32_reference_gpu(q, k, v, 77)
+    rel_ok(out[:, :T], ref)
+    assert (out[:, T:] == 9).all() and (dots[B * T * H:] == 9).all()
+    expect = (out[:, :T].float() * vec.view(B, 1, H, 64)).sum(-1)
+    assert torch.allclose(dots[:B * T * H].view(B, T, H), expect, rtol=1e-4, atol=1e-4)
