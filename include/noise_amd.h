@@ -375,6 +375,29 @@ int noise_pop_block_qkv_jit(const noise_population_t *pop, noise_view_t y, const
                             const float *ve, int64_t vocab, const int64_t *idx, int64_t idx_sm, const float *gate_w,
                             void *const out[3], const noise_block_jitter_t *jit, noise_stream_t stream);
 
+/* noise_pop_block and noise_pop_block_qkv for few token tiles, their work shared out over the CUs by output features in
+ * four launches (the same results, bit for bit), x_mid and the MLP's hidden rows passing through a workspace of
+ * noise_block_split_workspace_bytes (16 B aligned; 0: the one-launch forms are faster at this size; negative: invalid).
+ * xout is required; jit NULL or as in the _jit forms (the block then unperturbed); at most one next vector. */
+int64_t noise_block_split_workspace_bytes(int64_t members, int64_t tokens);
+int noise_pop_block_split(const noise_population_t *pop, noise_view_t y, const void *w_o, const noise_rank1_t *r_o,
+                          const float *o_dots, int64_t o_dots_n, noise_view_t xres, const void *w_fc,
+                          const noise_rank1_t *r_fc, const void *w_proj, const noise_rank1_t *r_proj, float *xout,
+                          int mix, const float *lam_r, const float *lam_x, const float *eps_r, const float *eps_x,
+                          int64_t eps_stride, noise_view_t x0, void *hout, int split3, const noise_rank1_t *next,
+                          int64_t nnext, float *next_dots, const noise_block_jitter_t *jit, void *workspace,
+                          int64_t workspace_bytes, noise_stream_t stream);
+int noise_pop_block_qkv_split(const noise_population_t *pop, noise_view_t y, const void *w_o, const noise_rank1_t *r_o,
+                              const float *o_dots, int64_t o_dots_n, noise_view_t xres, const void *w_fc,
+                              const noise_rank1_t *r_fc, const void *w_proj, const noise_rank1_t *r_proj, float *xout,
+                              int mix, const float *lam_r, const float *lam_x, const float *eps_r, const float *eps_x,
+                              int64_t eps_stride, noise_view_t x0, const void *const w_qkv[3],
+                              const noise_rank1_t r_qkv[3], const void *rope_cos, const void *rope_sin, const float *ve,
+                              int64_t vocab, const int64_t *idx, int64_t idx_sm, const float *gate_w,
+                              const noise_rank1_t *gate_noise, const noise_rank1_t *ve_noise, void *const out[3],
+                              const noise_block_jitter_t *jit, void *workspace, int64_t workspace_bytes,
+                              noise_stream_t stream);
+
 /* w [rows][cols] bf16 -> the column order noise_pop_block reads: within every 32 columns, position 8g + j
  * (g < 4) holds column 4g + j for j < 4 and 16 + 4g + (j - 4) for j >= 4. cols a multiple of 32. */
 int noise_block_weight_layout(const void *w, void *out, int64_t rows, int64_t cols, noise_stream_t stream);

@@ -36,6 +36,11 @@ SIGNATURES = {
                         'View', _p, _i32, _p, _i64, _p, _p],
     'noise_pop_block_qkv': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
                             'View', _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p],
+    'noise_block_split_workspace_bytes': [_i64, _i64],
+    'noise_pop_block_split': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
+                              'View', _p, _i32, _p, _i64, _p, _p, _p, _i64, _p],
+    'noise_pop_block_qkv_split': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
+                                  'View', _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p],
     'noise_block_weight_layout': [_p, _p, _i64, _i64, _p],
     'noise_weights_prepare': [_p, _i32, _p],
     'noise_mlp_proj_layout': [_p, _p, _i64, _p],
@@ -70,8 +75,8 @@ SIGNATURES = {
     'noise_update_gradients': [_p, _i32, _i64, _p, _f32, _i64, _i64, _u64, _u64, _i64, _p, _p, _i64, _p],
 }
 _RESTYPES = {'noise_last_error': ctypes.c_char_p, 'noise_update_workspace_bytes': ctypes.c_int64,
-             'noise_head_ce_workspace_bytes': ctypes.c_int64, 'noise_dust_block_workspace_bytes': ctypes.c_int64,
-             'noise_dust_block_static_max_bytes': ctypes.c_int64}
+             'noise_head_ce_workspace_bytes': ctypes.c_int64, 'noise_block_split_workspace_bytes': ctypes.c_int64,
+             'noise_dust_block_workspace_bytes': ctypes.c_int64, 'noise_dust_block_static_max_bytes': ctypes.c_int64}
 
 # y_fp32 of noise_pop_linear / noise_rank1_expand: fp32 output in autocast's form (bf16 product and dot)
 LINEAR_AUTOCAST = 2

@@ -563,6 +563,14 @@ __global__ __launch_bounds__(256) void block_layout_kernel(const __bf16 *w, __bf
     store_bf16x4(out + 4 * i, load_bf16x4(w + 32 * q + 4 * src));
 }
 
+}  // namespace
+}  // namespace noise
+
+#include "block_split.hpp"
+
+namespace noise {
+namespace {
+
 template <bool MIX, int NNEXT>
 void launch_block_n(const BlockArgs &a, bool split3, dim3 grid, hipStream_t s) {
     if (split3)
@@ -722,13 +730,27 @@ int block_jitter(const char *fn, BlockArgs &a, const noise_block_jitter_t *jit) 
     return NOISE_OK;
 }
 
+#define NOISE_TRY_SPLIT(x)          \
+    do {                            \
+        const int _s = (x);         \
+        if (_s != NOISE_OK) return _s; \
+    } while (0)
+
+int split_check(const char *fn, const BlockArgs &a, const float *xout, const void *workspace, int64_t bytes) {
+    const int64_t need = split_bytes((int64_t)a.members * a.tokens);
+    NOISE_CHECK_ARG(xout, "%s: xout must not be NULL", fn);
+    NOISE_CHECK_ARG(workspace && aligned(workspace, 16) && bytes >= need,
+                    "%s: a 16 B aligned workspace of %lld B is needed, got %lld", fn, (long long)need, (long long)bytes);
+    return NOISE_OK;
+}
+
 int pop_block_impl(const char *fn, const noise_population_t *pop, noise_view_t y, const void *w_o,
                    const noise_rank1_t *r_o, const float *o_dots, int64_t o_dots_n, noise_view_t xres,
                    const void *w_fc, const noise_rank1_t *r_fc, const void *w_proj, const noise_rank1_t *r_proj,
                    float *xout, int mix, const float *lam_r, const float *lam_x, const float *eps_r,
                    const float *eps_x, int64_t eps_stride, noise_view_t x0, void *hout, int split3,
                    const noise_rank1_t *next, int64_t nnext, float *next_dots, const noise_block_jitter_t *jit,
-                   noise_stream_t stream) {
+                   noise_stream_t stream, void *workspace = nullptr, int64_t workspace_bytes = 0, bool split = false) {
     BlockArgs a;
     const int st = block_args(fn, a, pop, y, w_o, r_o, o_dots, o_dots_n, xres, w_fc, r_fc, w_proj, r_proj, xout, mix,
                               lam_r, lam_x, eps_r, eps_x, eps_stride, x0, next, nnext);
@@ -737,6 +759,14 @@ int pop_block_impl(const char *fn, const noise_population_t *pop, noise_view_t y
     NOISE_CHECK_ARG(nnext == 0 || next_dots, "%s: next dots need an output", fn);
     a.hout = (__bf16 *)hout;
     a.ndots = next_dots;
+    if (split) {
+        NOISE_CHECK_ARG(nnext <= 1, "%s: at most one next vector", fn);
+        NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
+        if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
+        split_tail_launch(a, mix != 0, xout, workspace, (hipStream_t)stream);
+        split_norm_launch(a, xout, (int)nnext, split3 != 0, (hipStream_t)stream);
+        return launch_status(fn);
+    }
     const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
     if (jit) {
         const int js = block_jitter(fn, a, jit);
@@ -758,7 +788,8 @@ int pop_block_qkv_impl(const char *fn, const noise_population_t *pop, noise_view
                        const noise_rank1_t r_qkv[3], const void *rope_cos, const void *rope_sin, const float *ve,
                        int64_t vocab, const int64_t *idx, int64_t idx_sm, const float *gate_w,
                        const noise_rank1_t *gate_noise, const noise_rank1_t *ve_noise, void *const out[3],
-                       const noise_block_jitter_t *jit, noise_stream_t stream) {
+                       const noise_block_jitter_t *jit, noise_stream_t stream, void *workspace = nullptr,
+                       int64_t workspace_bytes = 0, bool split = false) {
     const bool pq = r_qkv && (r_qkv[0].a || r_qkv[1].a || r_qkv[2].a);
     BlockArgs a;
     const int st = block_args(fn, a, pop, y, w_o, r_o, o_dots, o_dots_n, xres, w_fc, r_fc, w_proj, r_proj, xout, mix,
@@ -793,6 +824,14 @@ int pop_block_qkv_impl(const char *fn, const noise_population_t *pop, noise_view
     a.q.gate_w = gate_w;
     a.q.gate_a = gn ? gate_noise->a : nullptr; a.q.gate_b = gn ? gate_noise->b : nullptr;
     a.q.gate_a_stride = gn ? gate_noise->a_stride : 0; a.q.gate_b_stride = gn ? gate_noise->b_stride : 0;
+    if (split) {
+        NOISE_CHECK_ARG(!jit || (!pq && !gn && !vn), "%s: a jittered block's next q/k/v take no noise", fn);
+        NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
+        if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
+        split_tail_launch(a, mix != 0, xout, workspace, (hipStream_t)stream);
+        split_qkv_launch(a, ve != nullptr, (hipStream_t)stream);
+        return launch_status(fn);
+    }
     const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
     if (jit) {
         NOISE_CHECK_ARG(!pq && !gn && !vn, "%s: a jittered block's next q/k/v take no noise", fn);
@@ -859,4 +898,47 @@ extern "C" int noise_pop_block_qkv_jit(const noise_population_t *pop, noise_view
     return pop_block_qkv_impl("noise_pop_block_qkv_jit", pop, y, w_o, nullptr, nullptr, 0, xres, w_fc, nullptr,
                               w_proj, nullptr, xout, 1, lam_r, lam_x, nullptr, nullptr, 0, x0, w_qkv, nullptr,
                               rope_cos, rope_sin, ve, vocab, idx, idx_sm, gate_w, nullptr, nullptr, out, jit, stream);
+}
+
+extern "C" int64_t noise_block_split_workspace_bytes(int64_t members, int64_t tokens) {
+    clear_error();
+    if (members <= 0 || tokens <= 0 || members >= (1ll << 31) / tokens) {
+        set_error("noise_block_split_workspace_bytes: members and tokens positive, members * tokens below 2^31");
+        return NOISE_EINVAL;
+    }
+    // few enough token tiles that one workgroup each leaves CUs idle
+    return members * tokens / kBlkTok <= kSplitTiles ? split_bytes(members * tokens) : 0;
+}
+
+extern "C" int noise_pop_block_split(const noise_population_t *pop, noise_view_t y, const void *w_o,
+                                     const noise_rank1_t *r_o, const float *o_dots, int64_t o_dots_n, noise_view_t xres,
+                                     const void *w_fc, const noise_rank1_t *r_fc, const void *w_proj,
+                                     const noise_rank1_t *r_proj, float *xout, int mix, const float *lam_r,
+                                     const float *lam_x, const float *eps_r, const float *eps_x, int64_t eps_stride,
+                                     noise_view_t x0, void *hout, int split3, const noise_rank1_t *next, int64_t nnext,
+                                     float *next_dots, const noise_block_jitter_t *jit, void *workspace,
+                                     int64_t workspace_bytes, noise_stream_t stream) {
+    clear_error();
+    return pop_block_impl("noise_pop_block_split", pop, y, w_o, r_o, o_dots, o_dots_n, xres, w_fc, r_fc, w_proj, r_proj,
+                          xout, mix, lam_r, lam_x, eps_r, eps_x, eps_stride, x0, hout, split3, next, nnext, next_dots,
+                          jit, stream, workspace, workspace_bytes, true);
+}
+
+extern "C" int noise_pop_block_qkv_split(const noise_population_t *pop, noise_view_t y, const void *w_o,
+                                         const noise_rank1_t *r_o, const float *o_dots, int64_t o_dots_n,
+                                         noise_view_t xres, const void *w_fc, const noise_rank1_t *r_fc,
+                                         const void *w_proj, const noise_rank1_t *r_proj, float *xout, int mix,
+                                         const float *lam_r, const float *lam_x, const float *eps_r, const float *eps_x,
+                                         int64_t eps_stride, noise_view_t x0, const void *const w_qkv[3],
+                                         const noise_rank1_t r_qkv[3], const void *rope_cos, const void *rope_sin,
+                                         const float *ve, int64_t vocab, const int64_t *idx, int64_t idx_sm,
+                                         const float *gate_w, const noise_rank1_t *gate_noise,
+                                         const noise_rank1_t *ve_noise, void *const out[3],
+                                         const noise_block_jitter_t *jit, void *workspace, int64_t workspace_bytes,
+                                         noise_stream_t stream) {
+    clear_error();
+    return pop_block_qkv_impl("noise_pop_block_qkv_split", pop, y, w_o, r_o, o_dots, o_dots_n, xres, w_fc, r_fc, w_proj,
+                              r_proj, xout, mix, lam_r, lam_x, eps_r, eps_x, eps_stride, x0, w_qkv, r_qkv, rope_cos,
+                              rope_sin, ve, vocab, idx, idx_sm, gate_w, gate_noise, ve_noise, out, jit, stream,
+                              workspace, workspace_bytes, true);
 }

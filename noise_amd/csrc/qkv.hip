@@ -17,11 +17,15 @@
 namespace noise {
 namespace {
 
-template <bool VE>
-__global__ __launch_bounds__(kQThreads, 1) void qkv16_kernel(QkvRowsArgs p) {
+// PART: few token tiles, each shared by `parts` workgroups of 24 / parts heads
+template <bool VE, bool PART = false>
+__global__ __launch_bounds__(kQThreads, 1) void qkv16_kernel(QkvRowsArgs p, int parts = 1) {
     __shared__ __attribute__((aligned(16))) char lds[kQLds];
     const int T = p.tokens, tiles_t = T / kQTok;
-    const int m = blockIdx.x / tiles_t, t0 = (blockIdx.x % tiles_t) * kQTok;
+    int tile = blockIdx.x, part = 0;
+    if (PART && !part_order(blockIdx.x, p.members * tiles_t, parts, tile, part)) return;
+    const int heads = PART ? 24 / parts : 24, s0 = part * heads, s1 = s0 + heads;
+    const int m = tile / tiles_t, t0 = (tile % tiles_t) * kQTok;
     const int tid = threadIdx.x, lane = tid & 63, tl = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int dir = m / p.dir_div;
@@ -31,7 +35,8 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv16_kernel(QkvRowsArgs p) {
     const unsigned lbase = lds_addr(lds);
 
 #pragma unroll
-    for (int k = 0; k < 3; ++k) qkv_issue(p, lbase, wave, lane, k);
+    for (int k = 2 * s0; k < 2 * s0 + 3; ++k)
+        if (!PART || k < 2 * s1) qkv_issue(p, lbase, wave, lane, k);
     // this lane's input row: xf[kb] = x[tok][32 kb + 8 g .. + 8]
     bf16x8 xf[16];
     {
@@ -46,9 +51,9 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv16_kernel(QkvRowsArgs p) {
     L.dq1 = p.a[1] ? sgn * p.dots[row * 3 + 1] : 0.f;
     L.dq2 = p.a[2] ? sgn * p.dots[row * 3 + 2] : 0.f;
     qkv_token_scalars<VE>(p, L);
-    vm_wait<8>();  // stage 0 landed (stages 1 and 2 may still be in flight); the rows and scalars above too
+    vm_wait<PART ? 0 : 8>();  // stage 0 landed (stages 1 and 2 may still be in flight); the rows and scalars above too
     __syncthreads();
-    qkv_phase<VE, false>(p, lds, xf, L);
+    qkv_phase<VE, false, PART>(p, lds, xf, L, s0, s1);
 }
 
 }  // namespace
@@ -59,11 +64,23 @@ int qkv_rows_launch(const noise_population_t *pop, noise_view_t x, const void *c
                     void *const out[3], noise_stream_t stream) {
     const QkvRowsArgs a = qkv_rows_args(pop, x, w, r1, dots, rope_cos, rope_sin, ve, vocab, idx, idx_sm, gates,
                                         ve_noise, out);
-    const dim3 grid((unsigned)(pop->members * (pop->tokens / kQTok)));
+    const int64_t tiles = pop->members * (pop->tokens / kQTok);
+    if (tiles <= 128) {
+        // the heads of a tile shared out while CUs would idle: 16 tiles, 57 us on 16 workgroups, 14
+        // on 192
+        const int parts = qkv_parts(tiles);
+        const dim3 grid((unsigned)part_grid(tiles, parts));
+        if (ve)
+            hipLaunchKernelGGL((qkv16_kernel<true, true>), grid, dim3(kQThreads), 0, (hipStream_t)stream, a, parts);
+        else
+            hipLaunchKernelGGL((qkv16_kernel<false, true>), grid, dim3(kQThreads), 0, (hipStream_t)stream, a, parts);
+        return launch_status("noise_pop_qkv");
+    }
+    const dim3 grid((unsigned)tiles);
     if (ve)
-        hipLaunchKernelGGL(qkv16_kernel<true>, grid, dim3(kQThreads), 0, (hipStream_t)stream, a);
+        hipLaunchKernelGGL((qkv16_kernel<true>), grid, dim3(kQThreads), 0, (hipStream_t)stream, a, 1);
     else
-        hipLaunchKernelGGL(qkv16_kernel<false>, grid, dim3(kQThreads), 0, (hipStream_t)stream, a);
+        hipLaunchKernelGGL((qkv16_kernel<false>), grid, dim3(kQThreads), 0, (hipStream_t)stream, a, 1);
     return launch_status("noise_pop_qkv");
 }
 

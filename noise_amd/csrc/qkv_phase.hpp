@@ -89,6 +89,33 @@ inline QkvRowsArgs qkv_rows_args(const noise_population_t *pop, noise_view_t x, 
     return a;
 }
 
+// workgroups per token tile (a divisor of the 24 heads, 2 to 12 heads each) that put about one on every CU
+inline int qkv_parts(int64_t tiles) {
+    const int heads[] = {2, 3, 4, 6, 8, 12};
+    for (int h : heads)
+        if (tiles * (24 / h) <= 256) return 24 / h;
+    return 2;
+}
+
+// Workgroup -> (token tile, part) of a launch whose tiles are shared by `parts` workgroups. Workgroups are dispatched
+// round-robin over the 8 XCDs: with at least 8 tiles a tile's parts run on one XCD, in every launch of a block, so that
+// its rows are fetched into (and found in) one L2 instead of eight. The grid is rounded up; false: nothing to do.
+constexpr int kXcds = 8;
+__device__ __forceinline__ bool part_order(int wg, int tiles, int parts, int &tile, int &part) {
+    if (tiles < kXcds) {
+        tile = wg / parts;
+        part = wg % parts;
+        return true;
+    }
+    const int slot = wg / kXcds;
+    part = slot % parts;
+    tile = slot / parts * kXcds + wg % kXcds;
+    return tile < tiles;
+}
+inline int64_t part_grid(int64_t tiles, int parts) {
+    return (tiles < kXcds ? tiles : (tiles + kXcds - 1) / kXcds * kXcds) * parts;
+}
+
 __device__ __forceinline__ float token_sum4(float v) { return sum_lanes_16_32(v); }
 
 // the per-token scalars of the phase's epilogues: rotary rows, value-table row and its noise scale
@@ -165,8 +192,11 @@ __device__ __forceinline__ void qkv_issue(const QkvRowsArgs &p, unsigned lbase, 
 
 // The phase itself; stages 0 .. 2 are issued and stage 0 has landed for every wave (a barrier) when it starts.
 // GATE_LOCAL: the V heads' gates computed from h[:32] (xf in the permuted k order) instead of read from p.gates.
-template <bool VE, bool GATE_LOCAL>
-__device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const bf16x8 (&xf)[16], const QkvLane &L) {
+// PART: heads s0 .. s1 only (the stages issued then are 2 s0 .. 2 s0 + 2, as far as 2 s1).
+template <bool VE, bool GATE_LOCAL, bool PART = false>
+__device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const bf16x8 (&xf)[16], const QkvLane &L,
+                                          int s0 = 0, int s1 = 24) {
+    const int first = PART ? s0 : 0, end = PART ? s1 : 24, stages = PART ? 2 * s1 : kQStages;
     const int T = p.tokens, m = L.m, t0 = L.t0, wave = L.wave, lane = L.lane, tid = L.tid, dir = L.dir;
     const int tl = lane & 15, g = lane >> 4;
     const int64_t row = L.row;
@@ -211,7 +241,7 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
 
     // GATE_LOCAL: the token's 8 value-head gates, once for the phase (NaN for a token id outside the table)
     float gates[8];
-    if constexpr (VE && GATE_LOCAL) {
+    if (VE && GATE_LOCAL && (!PART || end > 16)) {  // (a part without V heads needs none)
         float xg[32];
         gather_h32(xf[0], tl, xg);
         local_gates(p, xg, L.sgn, dir, gates);
@@ -222,12 +252,12 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
     float4 av[4], ev[4], bv[4];  // the head's epilogue inputs (rank-1 a; value rows and value-table b)
     float gate = 0.f;
 #pragma unroll 1
-    for (int s = 0; s < 24; ++s) {
+    for (int s = first; s < end; ++s) {
         const int mat = s >> 3, hd = s & 7;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 2 * s + h;
-            if (k + 3 < kQStages) issue(k + 3);  // into the buffer of stage k - 1 (every wave passed its barrier)
+            if (k + 3 < stages) issue(k + 3);  // into the buffer of stage k - 1 (every wave passed its barrier)
             if (qk_pending >= 0) {
                 flush_qk(qk_pending);
                 qk_pending = -1;
@@ -340,7 +370,7 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
             }
             // stage k + 1 landed for every wave (the stages issued after it may still fly); every wave is done
             // with buffer k & 3 and with the staging it filled in this stage
-            vm_wait_groups<4, 2>(kQStages - 2 - k < 2 ? kQStages - 2 - k : 2);
+            vm_wait_groups<4, 2>(stages - 2 - k < 2 ? stages - 2 - k : 2);
             __syncthreads();
         }
     }

@@ -216,6 +216,22 @@ def _head(popp, m, T, hx, hw, K, r1, B, targets, targets_sm, dev, stream):
         _call('noise_pop_head_ce', popp, hx, *args, stream)
 
 
+def _split_workspace(m, T, dev):
+    """Workspace of the blocks' split launches (None where a workgroup per token tile fills the chip)."""
+    need = _lib.lib().noise_block_split_workspace_bytes(m, T)
+    if need < 0:
+        raise RuntimeError(_lib.lib().noise_last_error().decode(errors='replace'))
+    return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+
+
+def _block(name, split, args, stream, jit=None, label='block'):
+    """One block launch (noise_pop_block or noise_pop_block_qkv) with its plain arguments, or its split form."""
+    if split is None:
+        _call(name, *args, stream, label=label)
+    else:
+        _call(name + '_split', *args, jit, split.data_ptr(), split.numel(), stream, label=label)
+
+
 _ZERO_ROWS = {}
 
 
@@ -309,6 +325,7 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
         _call('noise_member_dots', popp, _view(B.h0, sm_e, E), E, dot_vecs(n0, E), 3, B.d_qkv.data_ptr(), stream)
 
     qkv_out = (ctypes.c_void_p * 3)(*(B.qkv[i].data_ptr() for i in range(3)))
+    split = _split_workspace(m, T, dev) if fuse_qkv and rounding == _lib.ROUNDING_FUSED else None
     qkv_ready = False
     for i in range(L):
         pre = f'transformer.h.{i}.'
@@ -377,19 +394,23 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
                 nws = (ctypes.c_void_p * 3)(nblk['q_blk'].data_ptr(), nblk['k_blk'].data_ptr(),
                                             nblk['v_blk'].data_ptr())
                 n_ve, n_gate = _rank1(nz(f'value_embeds.{i + 1}.weight')), _rank1(nz(npre + 'attn.ve_gate.weight'))
-                _call('noise_pop_block_qkv', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
-                      B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
-                      blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1), B.resid.data_ptr(), *mixargs,
-                      _view(B.x0, sm_e, E), nws, _rank1_array(nn), cos_t.data_ptr(), sin_t.data_ptr(),
-                      nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
-                      idx.data_ptr(), idx_sm, nblk['gate'].data_ptr() if 've' in nblk else None,
-                      ctypes.byref(n_gate), ctypes.byref(n_ve), qkv_out, stream, label='block')
+                _block('noise_pop_block_qkv', split,
+                       (popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
+                        B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
+                        blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1), B.resid.data_ptr(), *mixargs,
+                        _view(B.x0, sm_e, E), nws, _rank1_array(nn), cos_t.data_ptr(), sin_t.data_ptr(),
+                        nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
+                        idx.data_ptr(), idx_sm, nblk['gate'].data_ptr() if 've' in nblk else None,
+                        ctypes.byref(n_gate), ctypes.byref(n_ve), qkv_out), stream)
                 qkv_ready = True
                 continue
-            _call('noise_pop_block', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
-                  B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
-                  blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1), None if last else B.resid.data_ptr(), *mixargs,
-                  _view(B.x0, sm_e, E), hout.data_ptr(), split3, nxt, nnext, ndots, stream, label='block')
+            tail = split if last else None
+            _block('noise_pop_block', tail,
+                   (popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
+                    B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
+                    blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1),
+                    None if last and tail is None else B.resid.data_ptr(), *mixargs,
+                    _view(B.x0, sm_e, E), hout.data_ptr(), split3, nxt, nnext, ndots), stream)
             continue
         # eager rounding: attn.c_proj + residual; h = norm(x_mid) (no rank-1 terms in this mode)
         _call('noise_pop_residual', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), E, ctypes.byref(o_r1),
@@ -487,6 +508,7 @@ def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=No
     none3 = _rank1_array([None, None, None])
     qkv_out = (ctypes.c_void_p * 3)(*(B.qkv[i].data_ptr() for i in range(3)))
     x0v = _view(x0, T * E, E)
+    split = _split_workspace(m, T, dev)
     # block `first`: its value-embedding gates and q/k/v from h_in
     blk = W.blocks[first]
     ws = (ctypes.c_void_p * 3)(blk['q'].data_ptr(), blk['k'].data_ptr(), blk['v'].data_ptr())
@@ -507,44 +529,42 @@ def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=No
               yv.stride(0), yv.stride(2), yv.stride(1), W.windows[i], 1.0 / math.sqrt(HEAD_DIM), None, 0, 1, None,
               stream, label=f'window {W.windows[i]}')
         xres = _view(x_in, T * E, E) if i == first else _view(B.resid, T * E, E)
+        js = None
         if i == first and jit:
             if 'o' in jit:
                 _call('noise_add_bf16', B.y.data_ptr(), jit['o'].data_ptr(), B.y.numel(), stream)
             if 'fc' in jit or 'mlp' in jit:
                 js = _lib.BlockJitter(_lib.ptr(jit.get('fc')), _lib.ptr(jit.get('mlp')),
                                       _zero_row_bf16(dev).data_ptr())
-                if i < L - 1:
-                    nblk = W.blocks[i + 1]
-                    nws = (ctypes.c_void_p * 3)(nblk['q_blk'].data_ptr(), nblk['k_blk'].data_ptr(),
-                                                nblk['v_blk'].data_ptr())
-                    _call('noise_pop_block_qkv_jit', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), xres,
-                          blk['fc_blk'].data_ptr(), blk['mp_blk'].data_ptr(), B.resid.data_ptr(), W.lam_r(i + 1),
-                          W.lam_x(i + 1), x0v, nws, cos_t.data_ptr(), sin_t.data_ptr(),
-                          nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
-                          idx.data_ptr(), T, nblk['gate'].data_ptr() if 've' in nblk else None, qkv_out,
-                          ctypes.byref(js), stream, label='block (jitter)')
-                else:
-                    _call('noise_pop_block_jit', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), xres,
-                          blk['fc_blk'].data_ptr(), blk['mp_blk'].data_ptr(), 0, None, None, x0v, B.h3.data_ptr(), 1,
-                          ctypes.byref(js), stream, label='block (jitter)')
-                continue
+        yv, wo, wfc, wmp = _view(B.y, T * E, E), blk['o'].data_ptr(), blk['fc_blk'].data_ptr(), blk['mp_blk'].data_ptr()
+        plain = (popp, yv, wo, ctypes.byref(none), B.d_attn.data_ptr(), N_HEAD, xres, wfc, ctypes.byref(none), wmp,
+                 ctypes.byref(none))
+        label = 'block' if js is None else 'block (jitter)'
+        jsp = None if js is None else ctypes.byref(js)
         if i < L - 1:
             # the block, then the next block's mixing, norm, gates and q/k/v (norm and dots stay in registers)
             nblk = W.blocks[i + 1]
             nws = (ctypes.c_void_p * 3)(nblk['q_blk'].data_ptr(), nblk['k_blk'].data_ptr(), nblk['v_blk'].data_ptr())
-            _call('noise_pop_block_qkv', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(none),
-                  B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(none),
-                  blk['mp_blk'].data_ptr(), ctypes.byref(none), B.resid.data_ptr(), 1, W.lam_r(i + 1),
-                  W.lam_x(i + 1), None, None, 0, x0v, nws, none3, cos_t.data_ptr(), sin_t.data_ptr(),
-                  nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
-                  idx.data_ptr(), T, nblk['gate'].data_ptr() if 've' in nblk else None, ctypes.byref(none),
-                  ctypes.byref(none), qkv_out, stream, label='block')
+            ve = (nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
+                  idx.data_ptr(), T, nblk['gate'].data_ptr() if 've' in nblk else None)
+            if js is not None and split is None:
+                _call('noise_pop_block_qkv_jit', popp, yv, wo, xres, wfc, wmp, B.resid.data_ptr(), W.lam_r(i + 1),
+                      W.lam_x(i + 1), x0v, nws, cos_t.data_ptr(), sin_t.data_ptr(), *ve, qkv_out, jsp, stream,
+                      label=label)
+            else:
+                _block('noise_pop_block_qkv', split,
+                       (*plain, B.resid.data_ptr(), 1, W.lam_r(i + 1), W.lam_x(i + 1), None, None, 0, x0v, nws, none3,
+                        cos_t.data_ptr(), sin_t.data_ptr(), *ve, ctypes.byref(none), ctypes.byref(none), qkv_out),
+                       stream, jsp, label)
         else:
             hout, split3 = (B.h3, 1) if W.fp32_head else (B.h, 0)
-            _call('noise_pop_block', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(none),
-                  B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(none),
-                  blk['mp_blk'].data_ptr(), ctypes.byref(none), None, 0, None, None, None, None, 0, x0v,
-                  hout.data_ptr(), split3, None, 0, None, stream, label='block')
+            if js is not None and split is None:
+                _call('noise_pop_block_jit', popp, yv, wo, xres, wfc, wmp, 0, None, None, x0v, hout.data_ptr(), split3,
+                      jsp, stream, label=label)
+            else:
+                _block('noise_pop_block', split,
+                       (*plain, None if split is None else B.resid.data_ptr(), 0, None, None, None, None, 0, x0v,
+                        hout.data_ptr(), split3, None, 0, None), stream, jsp, label)
     if W.fp32_head:
         hx, hw, K = _view(B.h3, T * 3 * E, 3 * E), W.lm_head3, 3 * E
     else:
