@@ -39,7 +39,11 @@ def call(name, *args):
 
 def stream_ptr(device=None):
     """hipStream_t of torch's current stream on `device`, as an integer for ctypes."""
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    # the same stream without a Stream object: this is asked for at every launch
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t):

@@ -97,10 +97,10 @@ def _rank1(pair):
     if pair is None:
         return _lib.Rank1(None, None, 0, 0)
     a, b = pair
-    for t in (a, b):
-        if t.dtype != F32 or t.stride(-1) != 1 or t.data_ptr() % 16 or t.stride(0) % 4:
-            raise ValueError('noise rows must be fp32, 16 B aligned, unit inner stride')
-    return _lib.Rank1(a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0))
+    pa, pb, sa, sb = a.data_ptr(), b.data_ptr(), a.stride(), b.stride()
+    if a.dtype != F32 or b.dtype != F32 or sa[-1] != 1 or sb[-1] != 1 or (pa | pb) % 16 or (sa[0] | sb[0]) % 4:
+        raise ValueError('noise rows must be fp32, 16 B aligned, unit inner stride')
+    return _lib.Rank1(pa, pb, sa[0], sb[0])
 
 
 def _rank1_array(pairs):
@@ -118,17 +118,20 @@ class Weights:
         dev = torch.device(device) if device is not None else p['lm_head.weight'].device
         if dev.type != 'cuda':
             raise ValueError('population_loss runs on the GPU')
+        if dev.index is None:
+            dev = torch.device('cuda', torch.cuda.current_device())
         self.device, self.n_layer = dev, n_layer
         # every parameter is copied, also where it already has the dtype: a Weights is a snapshot of one update's
         # parameters, never a view of the live ones. One launch per 64 parameters makes all the copies.
         jobs = []
 
         def add(name, kind, block=False):
-            t = p[name].detach().to(dev)
-            if t.dtype not in (F32, BF16):
-                t = t.to(BF16 if kind == _lib.WEIGHT_BF16 else F32)
-            t = t.contiguous()
-            dst = torch.empty(t.shape, dtype=BF16 if kind == _lib.WEIGHT_BF16 else F32, device=dev)
+            t = p[name]
+            want = BF16 if kind == _lib.WEIGHT_BF16 else F32
+            if t.device != dev or t.dtype not in (F32, BF16) or not t.is_contiguous():
+                t = t.detach().to(dev)
+                t = (t if t.dtype in (F32, BF16) else t.to(want)).contiguous()
+            dst = torch.empty(t.shape, dtype=want, device=dev)
             blk = torch.empty_like(dst) if block else None
             jobs.append((t, dst, blk, kind))
             return (dst, blk) if block else dst
@@ -326,11 +329,18 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
 
     qkv_out = (ctypes.c_void_p * 3)(*(B.qkv[i].data_ptr() for i in range(3)))
     split = _split_workspace(m, T, dev) if fuse_qkv and rounding == _lib.ROUNDING_FUSED else None
+    # the attention's operands are the same buffers in every block: q, k [m, T, H, D] views of [m, H, T, D], V^T as the
+    # q/k/v kernels write it, y [m, T, H, D]
+    attn = (*qkv_out, B.y.data_ptr(), m, N_HEAD, T, HEAD_DIM, N_HEAD * T * HEAD_DIM, T * HEAD_DIM, HEAD_DIM,
+            N_HEAD * T * HEAD_DIM, T * HEAD_DIM, HEAD_DIM, N_HEAD * HEAD_DIM * T, HEAD_DIM * T, T,
+            ATTN_V_TRANSPOSED | ATTN_QK_NORMED, T * E, HEAD_DIM, E)
+    y_view, resid_view, x0_view = _view(B.y, T * E, E), _view(B.resid, T * E, E), _view(B.x0, sm_e, E)
     qkv_ready = False
+    nn = qkv_noise(0)
     for i in range(L):
         pre = f'transformer.h.{i}.'
         blk = W.blocks[i]
-        nq = qkv_noise(i)
+        nq = nn
         x_in = _view(B.h0, sm_e, E) if i == 0 else _view(B.h, T * E, E)
         ws = (ctypes.c_void_p * 3)(blk['q'].data_ptr(), blk['k'].data_ptr(), blk['v'].data_ptr())
         ve_r1 = _rank1(nz(f'value_embeds.{i}.weight'))
@@ -357,19 +367,12 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
                       B.gates.data_ptr() if 've' in blk else None, ctypes.byref(ve_r1), qkv_out, stream)
         # attention; its epilogue also forms y . b_o per head for c_proj's rank-1 term
         no = nz(pre + 'attn.c_proj.weight')
-        q4, k4 = (B.qkv[j].transpose(1, 2) for j in range(2))  # [m, T, H, D] views of [m, H, T, D]
-        vt = B.qkv[2].view(m, N_HEAD, HEAD_DIM, T)               # V^T as the qkv kernel writes it
-        yv = B.y.view(m, T, N_HEAD, HEAD_DIM)
-        _call('noise_attention_fwd', q4.data_ptr(), k4.data_ptr(), vt.data_ptr(), yv.data_ptr(), m, N_HEAD, T,
-                  HEAD_DIM, q4.stride(0), q4.stride(2), q4.stride(1), k4.stride(0), k4.stride(2), k4.stride(1),
-                  vt.stride(0), vt.stride(1), vt.stride(2), ATTN_V_TRANSPOSED | ATTN_QK_NORMED,
-                  yv.stride(0), yv.stride(2), yv.stride(1),
-                  W.windows[i], 1.0 / math.sqrt(HEAD_DIM), None if no is None else no[1].data_ptr(),
-                  0 if no is None else no[1].stride(0), dir_div, None if no is None else B.d_attn.data_ptr(),
-                  stream, label=f'window {W.windows[i]}')
+        _call('noise_attention_fwd', *attn, W.windows[i], 1.0 / math.sqrt(HEAD_DIM),
+              None if no is None else no[1].data_ptr(), 0 if no is None else no[1].stride(0), dir_div,
+              None if no is None else B.d_attn.data_ptr(), stream, label=f'window {W.windows[i]}')
         nfc, nmp = nz(pre + 'mlp.c_fc.weight'), nz(pre + 'mlp.c_proj.weight')
         o_r1 = _rank1(no)
-        xres = _view(B.xin0, sm_e, E) if i == 0 else _view(B.resid, T * E, E)
+        xres = _view(B.xin0, sm_e, E) if i == 0 else resid_view
         fc_r1 = _rank1(nfc)
         mp_r1 = _rank1(nmp)
         last = i == L - 1
@@ -379,9 +382,10 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
             # mix, norm and q/k/v dots (or the head input)
             if not last:
                 nn = qkv_noise(i + 1)
-                want = any(v is not None for v in nn)
-                nxt, nnext, ndots = (dot_vecs(nn, E), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
-                hout, split3 = B.h, 0
+                if not fuse_qkv:
+                    want = any(v is not None for v in nn)
+                    nxt, nnext, ndots = (dot_vecs(nn, E), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
+                    hout, split3 = B.h, 0
                 mixargs = (1, W.lam_r(i + 1), W.lam_x(i + 1), eps_ptr(eps_r, i + 1), eps_ptr(eps_x, i + 1), eps_stride)
             else:
                 nh = nz('lm_head.weight')
@@ -395,10 +399,10 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
                                             nblk['v_blk'].data_ptr())
                 n_ve, n_gate = _rank1(nz(f'value_embeds.{i + 1}.weight')), _rank1(nz(npre + 'attn.ve_gate.weight'))
                 _block('noise_pop_block_qkv', split,
-                       (popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
+                       (popp, y_view, blk['o'].data_ptr(), ctypes.byref(o_r1),
                         B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
                         blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1), B.resid.data_ptr(), *mixargs,
-                        _view(B.x0, sm_e, E), nws, _rank1_array(nn), cos_t.data_ptr(), sin_t.data_ptr(),
+                        x0_view, nws, _rank1_array(nn), cos_t.data_ptr(), sin_t.data_ptr(),
                         nblk['ve'].data_ptr() if 've' in nblk else None, nblk['ve'].shape[0] if 've' in nblk else 0,
                         idx.data_ptr(), idx_sm, nblk['gate'].data_ptr() if 've' in nblk else None,
                         ctypes.byref(n_gate), ctypes.byref(n_ve), qkv_out), stream)
@@ -406,16 +410,16 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
                 continue
             tail = split if last else None
             _block('noise_pop_block', tail,
-                   (popp, _view(B.y, T * E, E), blk['o'].data_ptr(), ctypes.byref(o_r1),
+                   (popp, y_view, blk['o'].data_ptr(), ctypes.byref(o_r1),
                     B.d_attn.data_ptr(), N_HEAD, xres, blk['fc_blk'].data_ptr(), ctypes.byref(fc_r1),
                     blk['mp_blk'].data_ptr(), ctypes.byref(mp_r1),
                     None if last and tail is None else B.resid.data_ptr(), *mixargs,
-                    _view(B.x0, sm_e, E), hout.data_ptr(), split3, nxt, nnext, ndots), stream)
+                    x0_view, hout.data_ptr(), split3, nxt, nnext, ndots), stream)
             continue
         # eager rounding: attn.c_proj + residual; h = norm(x_mid) (no rank-1 terms in this mode)
-        _call('noise_pop_residual', popp, _view(B.y, T * E, E), blk['o'].data_ptr(), E, ctypes.byref(o_r1),
+        _call('noise_pop_residual', popp, y_view, blk['o'].data_ptr(), E, ctypes.byref(o_r1),
                   B.d_attn.data_ptr(), N_HEAD, N_HEAD, xres, B.resid.data_ptr(), 0, None, None, None, None, 0,
-                  _view(B.x0, sm_e, E), B.h.data_ptr(), 0, None, 0, None, stream, label='attn.c_proj')
+                  x0_view, B.h.data_ptr(), 0, None, 0, None, stream, label='attn.c_proj')
         # mlp.c_fc, ReLU^2 and partial dots for mlp.c_proj, then mlp.c_proj + residual
         mp_next = _rank1(nmp)
         _call('noise_pop_fc', popp, _view(B.h, T * E, E), blk['fc'].data_ptr(), ctypes.byref(fc_r1),
@@ -426,16 +430,16 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
             want = any(v is not None for v in nn)
             nxt, nnext, ndots = (dot_vecs(nn, E), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
             _call('noise_pop_residual', popp, _view(B.act, T * 4 * E, 4 * E), blk['mp'].data_ptr(), 4 * E,
-                  ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, _view(B.resid, T * E, E), B.resid.data_ptr(),
+                  ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, resid_view, B.resid.data_ptr(),
                   1, W.lam_r(i + 1), W.lam_x(i + 1), eps_ptr(eps_r, i + 1), eps_ptr(eps_x, i + 1),
-                  eps_stride, _view(B.x0, sm_e, E), B.h.data_ptr(), 0, nxt, nnext, ndots, stream, label='mlp.c_proj')
+                  eps_stride, x0_view, B.h.data_ptr(), 0, nxt, nnext, ndots, stream, label='mlp.c_proj')
         else:
             nh = nz('lm_head.weight')
             nxt, nnext, ndots = (dot_vecs([nh], E), 1, B.d_head.data_ptr()) if nh is not None else (None, 0, None)
             hout = B.h3 if W.fp32_head else B.h
             _call('noise_pop_residual', popp, _view(B.act, T * 4 * E, 4 * E), blk['mp'].data_ptr(), 4 * E,
-                  ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, _view(B.resid, T * E, E), None, 0, None, None,
-                  None, None, 0, _view(B.x0, sm_e, E), hout.data_ptr(), 1 if W.fp32_head else 0, nxt, nnext,
+                  ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, resid_view, None, 0, None, None,
+                  None, None, 0, x0_view, hout.data_ptr(), 1 if W.fp32_head else 0, nxt, nnext,
                   ndots, stream, label='mlp.c_proj')
     nh = nz('lm_head.weight')
     head_r1 = _rank1(nh)
@@ -768,16 +772,18 @@ class Eggroll:
         out = {}
         names = list(offsets)
         widths = [-(-sum(self.params[n].shape) // 256) * 256 for n in names]
-        table = self.buffer.gather_many([offsets[n] for n in names], widths, directions) if names else None
-        col = 0
+        if not names:
+            return out
+        table = self.buffer.gather_many([offsets[n] for n in names], widths, directions)
+        # every column view in one call: a, b (or eps) and the columns after a narrower slice
+        sizes = []
         for n, w in zip(names, widths):
             shape = self.params[n].shape
-            if len(shape) == 2:
-                o, i = shape
-                out[n] = (table[:, col:col + o], table[:, col + o:col + o + i])
-            else:
-                out[n] = table[:, col:col + shape[0]]
-            col += w
+            sizes += [*shape, w - sum(shape)]
+        views = iter(table.split(sizes, dim=1))
+        for n in names:
+            out[n] = (next(views), next(views)) if self.params[n].dim() == 2 else next(views)
+            next(views)
         return out
 
     def population(self, step, x, y, weights=None, chunk=512, names=None, fp32_head=False):

@@ -150,7 +150,8 @@ def _operand(t):
     """bf16 view usable by the kernels: contiguous head dim, 8-element-aligned strides, 16 B base."""
     if t.dtype != BF16:
         t = t.to(BF16)
-    if (t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16):
+    s = t.stride()
+    if s[-1] != 1 or (s[0] | s[1] | s[2]) % 8 or t.data_ptr() % 16:
         t = t.contiguous()
     return t
 

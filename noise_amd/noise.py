@@ -68,7 +68,8 @@ class Draw:
         nrows = rows.numel()
         if nrows > 65535:
             raise ValueError('gather_many: at most 65535 rows per call')
-        offsets = [o.to(device=self.device, dtype=torch.int64).contiguous() for o in offsets]
+        offsets = [o if o.dtype == torch.int64 and o.device == self.device and o.is_contiguous() else
+                   o.to(device=self.device, dtype=torch.int64).contiguous() for o in offsets]
         total = int(sum(widths))
         out = torch.empty(nrows, total, device=self.device, dtype=torch.float32)
         col = 0
