@@ -398,13 +398,26 @@ int noise_pop_block_qkv_split(const noise_population_t *pop, noise_view_t y, con
                               const noise_block_jitter_t *jit, void *workspace, int64_t workspace_bytes,
                               noise_stream_t stream);
 
+/* One unperturbed block on its own (DUST's block_forward, run.py:102-117), around noise_attention_fwd:
+ * noise_rows_qkv: q, k, v (as noise_pop_block_qkv writes them) of fp32 rows x [members * tokens][512]: h = norm(x), the
+ * value-embedding gates from h[:32] and gate_w, value rows ve_rows bf16 [members * tokens][512] (NULL: none), rotary and
+ * head norm; w_qkv in the column order of noise_block_weight_layout.
+ * noise_block_tail: xout = x + attn.c_proj, residual, MLP as noise_pop_block without noise and mixing; jit NULL or as in
+ * the _jit forms; workspace NULL, or of noise_block_split_workspace_bytes for the split launches. */
+int noise_rows_qkv(const noise_population_t *pop, const float *x, const void *const w_qkv[3], const void *rope_cos,
+                   const void *rope_sin, const void *ve_rows, const float *gate_w, void *const out[3],
+                   noise_stream_t stream);
+int noise_block_tail(const noise_population_t *pop, noise_view_t y, const void *w_o, noise_view_t xres,
+                     const void *w_fc, const void *w_proj, float *xout, const noise_block_jitter_t *jit, void *workspace,
+                     int64_t workspace_bytes, noise_stream_t stream);
+
 /* w [rows][cols] bf16 -> the column order noise_pop_block reads: within every 32 columns, position 8g + j
  * (g < 4) holds column 4g + j for j < 4 and 16 + 4g + (j - 4) for j >= 4. cols a multiple of 32. */
 int noise_block_weight_layout(const void *w, void *out, int64_t rows, int64_t cols, noise_stream_t stream);
 
 /* A parameter update's device copies in one launch. Per entry: numel values of src (fp32, or bf16 when src_bf16) to dst
  * (16 B aligned) as bf16 (NOISE_WEIGHT_BF16; also to dst_block, unless NULL, in the column order of
- * noise_block_weight_layout), as fp32 (NOISE_WEIGHT_FP32), or as fp32 holding the values rounded to bf16
+ * noise_block_weight_layout; either may be NULL), as fp32 (NOISE_WEIGHT_FP32), or as fp32 holding the values rounded to bf16
  * (NOISE_WEIGHT_FP32_ROUNDED: autocast's weights where a kernel reads fp32). Passed by value to the kernel. */
 #define NOISE_WEIGHTS_MAX 64
 #define NOISE_WEIGHT_BF16 0

@@ -36,6 +36,8 @@ SIGNATURES = {
                         'View', _p, _i32, _p, _i64, _p, _p],
     'noise_pop_block_qkv': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
                             'View', _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p],
+    'noise_rows_qkv': [_p, _p, _p, _p, _p, _p, _p, _p, _p],
+    'noise_block_tail': [_p, 'View', _p, 'View', _p, _p, _p, _p, _p, _i64, _p],
     'noise_block_split_workspace_bytes': [_i64, _i64],
     'noise_pop_block_split': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
                               'View', _p, _i32, _p, _i64, _p, _p, _p, _i64, _p],

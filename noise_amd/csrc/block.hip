@@ -519,6 +519,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void block_kernel(BlockArgs p) {
         qkv_phase<QKV == 2, true>(p.q, lds, xf, L);
         return;
     }
+    if (!p.hout) return;  // (the residual alone)
     // bf16 rows (hi, and lo for the split3 head input): 1 KiB rows, 16 B chunk c of row t at c ^ t
     const int width = SPLIT3 ? 3 * kModel : kModel;
 #pragma unroll
@@ -610,7 +611,9 @@ void launch_block_qkv(const BlockArgs &a, int nnext, bool ve, dim3 grid, hipStre
 // block followed by the next block's q/k/v with or without its value embeddings (with the next mixing)
 template <int JIT>
 bool launch_block_jit_n(const BlockArgs &a, bool mix, bool split3, int qkv, dim3 grid, hipStream_t s) {
-    if (qkv == 0 && !mix && split3)
+    if (qkv == 0 && !mix && !a.hout)
+        hipLaunchKernelGGL((block_kernel<false, 0, false, 0, JIT>), grid, dim3(kBlkThreads), 0, s, a);
+    else if (qkv == 0 && !mix && split3)
         hipLaunchKernelGGL((block_kernel<false, 0, true, 0, JIT>), grid, dim3(kBlkThreads), 0, s, a);
     else if (qkv == 1 && mix)
         hipLaunchKernelGGL((block_kernel<true, 0, false, 1, JIT>), grid, dim3(kBlkThreads), 0, s, a);
@@ -829,7 +832,7 @@ int pop_block_qkv_impl(const char *fn, const noise_population_t *pop, noise_view
         NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
         if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
         split_tail_launch(a, mix != 0, xout, workspace, (hipStream_t)stream);
-        split_qkv_launch(a, ve != nullptr, (hipStream_t)stream);
+        split_qkv_launch(a, ve ? 1 : 0, (hipStream_t)stream);
         return launch_status(fn);
     }
     const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
@@ -941,4 +944,51 @@ extern "C" int noise_pop_block_qkv_split(const noise_population_t *pop, noise_vi
                               r_proj, xout, mix, lam_r, lam_x, eps_r, eps_x, eps_stride, x0, w_qkv, r_qkv, rope_cos,
                               rope_sin, ve, vocab, idx, idx_sm, gate_w, gate_noise, ve_noise, out, jit, stream,
                               workspace, workspace_bytes, true);
+}
+
+// x_out = the block's tail alone (attn.c_proj, residual, MLP) on an attention output, for a block on its own
+extern "C" int noise_block_tail(const noise_population_t *pop, noise_view_t y, const void *w_o, noise_view_t xres,
+                                const void *w_fc, const void *w_proj, float *xout, const noise_block_jitter_t *jit,
+                                void *workspace, int64_t workspace_bytes, noise_stream_t stream) {
+    clear_error();
+    const char *fn = "noise_block_tail";
+    BlockArgs a;
+    NOISE_TRY_SPLIT(block_args(fn, a, pop, y, w_o, nullptr, nullptr, 0, xres, w_fc, nullptr, w_proj, nullptr, xout, 0,
+                               nullptr, nullptr, nullptr, nullptr, 0, noise_view_t{nullptr, 0, 0}, nullptr, 0));
+    NOISE_CHECK_ARG(xout, "%s: xout must not be NULL", fn);
+    if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
+    if (workspace) {
+        NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
+        split_tail_launch(a, false, xout, workspace, (hipStream_t)stream);
+        return launch_status(fn);
+    }
+    const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
+    if (jit) return launch_block_jit(fn, a, false, false, 0, grid, (hipStream_t)stream);
+    launch_block<false>(a, 0, false, grid, (hipStream_t)stream);
+    return launch_status(fn);
+}
+
+extern "C" int noise_rows_qkv(const noise_population_t *pop, const float *x, const void *const w_qkv[3],
+                              const void *rope_cos, const void *rope_sin, const void *ve_rows, const float *gate_w,
+                              void *const out[3], noise_stream_t stream) {
+    clear_error();
+    const char *fn = "noise_rows_qkv";
+    NOISE_CHECK_ARG(pop && pop->members > 0 && pop->tokens > 0 && pop->dir_div >= 1, "%s: bad population", fn);
+    NOISE_CHECK_ARG(pop->tokens % kBlkTok == 0 && pop->members * pop->tokens < (1ll << 31),
+                    "%s: tokens must be a multiple of %d and members * tokens below 2^31", fn, kBlkTok);
+    NOISE_CHECK_ARG(x && aligned(x, 16) && w_qkv && out && rope_cos && rope_sin && aligned(rope_cos, 16) &&
+                        aligned(rope_sin, 16), "%s: NULL or misaligned argument", fn);
+    for (int i = 0; i < 3; ++i)
+        NOISE_CHECK_ARG(w_qkv[i] && out[i] && aligned(w_qkv[i], 16) && aligned(out[i], 16),
+                        "%s: weight or output %d NULL or not 16 B aligned", fn, i);
+    NOISE_CHECK_ARG(!ve_rows || (gate_w && aligned(ve_rows, 16)), "%s: value rows (16 B aligned) need gate weights", fn);
+    BlockArgs a{};
+    a.members = (int)pop->members; a.tokens = (int)pop->tokens;
+    a.xout = const_cast<float *>(x);  // (read only)
+    a.q = qkv_rows_args(pop, noise_view_t{nullptr, 0, 0}, w_qkv, nullptr, nullptr, rope_cos, rope_sin, nullptr, 0, nullptr,
+                        0, nullptr, nullptr, out);
+    a.q.ve_rows = (const __bf16 *)ve_rows;
+    a.q.gate_w = gate_w;
+    split_qkv_launch(a, ve_rows ? 2 : 0, (hipStream_t)stream);
+    return launch_status(fn);
 }

@@ -339,7 +339,7 @@ struct SplitQkvArgs {
     int parts, heads;                 // heads per part (24 / parts)
 };
 
-template <bool VE>
+template <int VE>
 __global__ __launch_bounds__(kQThreads, 1) void split_qkv_kernel(SplitQkvArgs p) {
     __shared__ __attribute__((aligned(16))) char lds[kQLds];
     const int T = p.q.tokens, tiles_t = T / kQTok;
@@ -464,7 +464,7 @@ void split_tail_launch(const BlockArgs &a, bool mix, float *xout, void *workspac
     split_rows_launch<true>(r, tiles, s);
 }
 
-void split_qkv_launch(const BlockArgs &a, bool ve, hipStream_t s) {
+void split_qkv_launch(const BlockArgs &a, int ve, hipStream_t s) {
     const int64_t tiles = (int64_t)a.members * a.tokens / kBlkTok;
     SplitQkvArgs q;
     q.q = a.q; q.x = a.xout;
@@ -475,10 +475,12 @@ void split_qkv_launch(const BlockArgs &a, bool ve, hipStream_t s) {
     q.parts = qkv_parts(tiles);
     q.heads = 24 / q.parts;
     const dim3 grid((unsigned)part_grid(tiles, q.parts));
-    if (ve)
-        hipLaunchKernelGGL(split_qkv_kernel<true>, grid, dim3(kQThreads), 0, s, q);
+    if (ve == 2)
+        hipLaunchKernelGGL(split_qkv_kernel<2>, grid, dim3(kQThreads), 0, s, q);
+    else if (ve)
+        hipLaunchKernelGGL(split_qkv_kernel<1>, grid, dim3(kQThreads), 0, s, q);
     else
-        hipLaunchKernelGGL(split_qkv_kernel<false>, grid, dim3(kQThreads), 0, s, q);
+        hipLaunchKernelGGL(split_qkv_kernel<0>, grid, dim3(kQThreads), 0, s, q);
 }
 
 void split_norm_launch(const BlockArgs &a, const float *x, int nnext, bool split3, hipStream_t s) {

@@ -50,7 +50,8 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (__bf16)v[e];
         __bf16 *d = static_cast<__bf16 *>(w.dst) + i;
-        if (whole) {
+        if (!w.dst) {
+        } else if (whole) {
             store_bf16x8(d, o);
         } else {
             for (int e = 0; i + e < w.numel; ++e) d[e] = o[e];
@@ -94,7 +95,7 @@ extern "C" int noise_weights_prepare(const noise_weight_t *weights, int count, n
     p.count = count;
     for (int i = 0; i < count; ++i) {
         const noise_weight_t &w = weights[i];
-        NOISE_CHECK_ARG(w.src && w.dst && w.numel > 0 && aligned(w.dst, 16) && aligned(w.src, w.src_bf16 ? 2 : 4),
+        NOISE_CHECK_ARG(w.src && (w.dst || w.dst_block) && w.numel > 0 && aligned(w.dst, 16) && aligned(w.src, w.src_bf16 ? 2 : 4),
                         "%s: entry %d: NULL, empty or misaligned", fn, i);
         NOISE_CHECK_ARG(w.kind >= NOISE_WEIGHT_BF16 && w.kind <= NOISE_WEIGHT_FP32_ROUNDED, "%s: entry %d: unknown kind %d",
                         fn, i, w.kind);

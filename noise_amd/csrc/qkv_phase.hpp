@@ -48,6 +48,7 @@ struct QkvRowsArgs {
     const float *ve_a, *ve_b;          // value-table noise a [dirs][V], b [dirs][512] or NULL
     int64_t ve_a_stride, ve_b_stride;
     __bf16 *out[3];                    // q, k [m][8][T][64]; v transposed [m][8][64][T]
+    const __bf16 *ve_rows;             // VE = 2: the value-embedding rows themselves, bf16 [m T][512]
     // the gates computed in the kernel (qkv_phase<.., true>) instead of read from `gates`
     const float *gate_w;               // [8][32] fp32
     const float *gate_a, *gate_b;      // [dirs][8], [dirs][32] or NULL
@@ -89,12 +90,12 @@ inline QkvRowsArgs qkv_rows_args(const noise_population_t *pop, noise_view_t x, 
     return a;
 }
 
-// workgroups per token tile (a divisor of the 24 heads, 2 to 12 heads each) that put about one on every CU
+// workgroups per token tile (a divisor of the 24 heads, 2 to 24 heads each) that put about one on every CU
 inline int qkv_parts(int64_t tiles) {
     const int heads[] = {2, 3, 4, 6, 8, 12};
     for (int h : heads)
         if (tiles * (24 / h) <= 256) return 24 / h;
-    return 2;
+    return 1;
 }
 
 // Workgroup -> (token tile, part) of a launch whose tiles are shared by `parts` workgroups. Workgroups are dispatched
@@ -118,8 +119,9 @@ inline int64_t part_grid(int64_t tiles, int parts) {
 
 __device__ __forceinline__ float token_sum4(float v) { return sum_lanes_16_32(v); }
 
+// VE: value embeddings: 0 none, 1 from the table by token id, 2 given as bf16 rows
 // the per-token scalars of the phase's epilogues: rotary rows, value-table row and its noise scale
-template <bool VE>
+template <int VE>
 __device__ __forceinline__ void qkv_token_scalars(const QkvRowsArgs &p, QkvLane &L) {
     const int g = L.lane >> 4;
 #pragma unroll
@@ -130,7 +132,7 @@ __device__ __forceinline__ void qkv_token_scalars(const QkvRowsArgs &p, QkvLane 
     L.tv = 0;
     L.bad = false;
     L.vesc = 0.f;
-    if constexpr (VE) {
+    if constexpr (VE == 1) {
         const int64_t id = p.idx[L.m * p.idx_m + L.tok];
         L.bad = id < 0 || id >= p.vocab;  // an id outside the table: no read leaves it, V is NaN
         L.tv = L.bad ? 0 : id;
@@ -193,7 +195,7 @@ __device__ __forceinline__ void qkv_issue(const QkvRowsArgs &p, unsigned lbase, 
 // The phase itself; stages 0 .. 2 are issued and stage 0 has landed for every wave (a barrier) when it starts.
 // GATE_LOCAL: the V heads' gates computed from h[:32] (xf in the permuted k order) instead of read from p.gates.
 // PART: heads s0 .. s1 only (the stages issued then are 2 s0 .. 2 s0 + 2, as far as 2 s1).
-template <bool VE, bool GATE_LOCAL, bool PART = false>
+template <int VE, bool GATE_LOCAL, bool PART = false>
 __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const bf16x8 (&xf)[16], const QkvLane &L,
                                           int s0 = 0, int s1 = 24) {
     const int first = PART ? s0 : 0, end = PART ? s1 : 24, stages = PART ? 2 * s1 : kQStages;
@@ -241,7 +243,7 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
 
     // GATE_LOCAL: the token's 8 value-head gates, once for the phase (NaN for a token id outside the table)
     float gates[8];
-    if (VE && GATE_LOCAL && (!PART || end > 16)) {  // (a part without V heads needs none)
+    if (VE != 0 && GATE_LOCAL && (!PART || end > 16)) {  // (a part without V heads needs none)
         float xg[32];
         gather_h32(xf[0], tl, xg);
         local_gates(p, xg, L.sgn, dir, gates);
@@ -274,7 +276,7 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
 #pragma unroll
                     for (int b = 0; b < 4; ++b) av[b] = ld4(ar + 16 * b);
                 }
-                if constexpr (VE) {
+                if constexpr (VE != 0) {
                     if (mat == 2) {
                         if constexpr (GATE_LOCAL) {
                             gate = gates[0];
@@ -283,9 +285,18 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
                         } else {
                             gate = bad ? __builtin_nanf("") : p.gates[row * 8 + hd];
                         }
-                        const float *er = p.ve + tv * 512 + 64 * hd + 4 * g;  // one value table for every member
+                        if constexpr (VE == 2) {
+                            const __bf16 *er = p.ve_rows + row * 512 + 64 * hd + 4 * g;
 #pragma unroll
-                        for (int b = 0; b < 4; ++b) ev[b] = ld4(er + 16 * b);
+                            for (int b = 0; b < 4; ++b) {
+                                const bf16x4 e = load_bf16x4(er + 16 * b);
+                                ev[b] = float4{(float)e[0], (float)e[1], (float)e[2], (float)e[3]};
+                            }
+                        } else {
+                            const float *er = p.ve + tv * 512 + 64 * hd + 4 * g;  // one value table for every member
+#pragma unroll
+                            for (int b = 0; b < 4; ++b) ev[b] = ld4(er + 16 * b);
+                        }
                         if (p.ve_a) {
                             const float *br = p.ve_b + dir * p.ve_b_stride + 64 * hd + 4 * g;
 #pragma unroll
@@ -319,7 +330,7 @@ __device__ __forceinline__ void qkv_phase(const QkvRowsArgs &p, char *lds, const
                         for (int r = 0; r < 4; ++r) acc[b][r] += corr * f4get(av[b], r);
                 }
                 if (mat == 2) {
-                    if constexpr (VE) {
+                    if constexpr (VE != 0) {
                         // v += gate * (ve[idx[t], head*64 + d] (+ sign a_ve[idx[t]] b_ve[d]))   (eggroll.py:85-89)
 #pragma unroll
                         for (int b = 0; b < 4; ++b)

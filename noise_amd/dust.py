@@ -84,9 +84,9 @@ def head_error(logits, y, vocab, sigma=0.1):
     return out
 
 
-def _bf16_weight(t):
-    """bf16 contiguous copy of a weight (the reference's autocast casts it at every call too)."""
-    return t.detach().to(BF16).contiguous()
+def _aligned(t):
+    """t at a 16 B address (contiguous tensors may start at any element of their storage)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def block_forward(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, mlp=None):
@@ -102,8 +102,80 @@ def block_forward_eager(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, 
     (attn.c_proj product), fc (mlp.c_fc product, before ReLU^2) or mlp (mlp.c_proj product), each
     [B, T, width]. w: the reference's dict q, k, v, gate (None without value embeddings), proj, fc, out.
     ve: [B, T, 512] value-embedding rows or None. cos, sin: the model's rotary tables (bf16, T x 32 values).
-    Returns x_out fp32 [B, T, 512]. One HIP chain (noise_dust_block): bf16 products with fp32 accumulation,
-    bf16 attention, fp32 residual stream, as the reference's autocast."""
+    Returns x_out fp32 [B, T, 512]: bf16 products with fp32 accumulation, bf16 attention, fp32 residual stream, as the
+    reference's autocast. Four launches on the population kernels, one sequence per member: the weights' bf16 copies,
+    norm with gates and q/k/v, attention, and the rest of the block (with few sequences shared out over the CUs)."""
+    from .eggroll import _split_workspace, _zero_row_bf16
+    dev = x.device
+    B, T, C = x.shape
+    if C != 512 or T % 256:
+        raise ValueError('block_forward: width 512 and a multiple of 256 tokens are supported')
+    gate = w.get('gate')
+    if ve is not None and gate is None:
+        raise ValueError('block_forward: value embeddings need the ve_gate weight')
+    xs = _aligned(x.to(F32).contiguous())
+    stream = _lib.stream_ptr(dev)
+    # q, k, v, c_fc and mlp.c_proj in the block kernel's column order, attn.c_proj and the gate as they are
+    table, keep, ws = (_lib.Weight * 7)(), [], {}
+    for i, name in enumerate(('q', 'k', 'v', 'fc', 'out', 'proj', 'gate')):
+        t = w.get(name) if name == 'gate' else w[name]
+        if t is None:
+            continue
+        t = t.detach()
+        if t.dtype not in (F32, BF16):
+            t = t.to(BF16)
+        t = t.contiguous()
+        ws[name] = torch.empty(t.shape, dtype=F32 if name == 'gate' else BF16, device=dev)
+        keep.append(t)
+        ptr = ws[name].data_ptr()
+        table[len(keep) - 1] = _lib.Weight(t.data_ptr(), None if i < 5 else ptr, ptr if i < 5 else None, t.numel(),
+                                           int(t.dtype == BF16),
+                                           _lib.WEIGHT_FP32_ROUNDED if name == 'gate' else _lib.WEIGHT_BF16)
+    _lib.call('noise_weights_prepare', table, len(keep), stream)
+    if ve is not None:
+        ve = _aligned(ve.reshape(B, T, C).to(BF16).contiguous())
+    cs = _aligned(cos.reshape(-1)[:T * 32].view(T, 32).to(BF16).contiguous())
+    sn = _aligned(sin.reshape(-1)[:T * 32].view(T, 32).to(BF16).contiguous())
+    jit = []
+    for t, width in ((o, C), (attn, C), (fc, 4 * C), (mlp, C)):
+        jit.append(None if t is None else _aligned(t.reshape(B, T, width).to(BF16).contiguous()))
+    o, attn, fc, mlp = jit
+    pop = ctypes.byref(_lib.Population(B, T, None, 1, _lib.ROUNDING_FUSED))
+    qkv = torch.empty(3, B, 8, T, 64, dtype=BF16, device=dev)
+    y = torch.empty(B, T, C, dtype=BF16, device=dev)
+    out = torch.empty(B, T, C, dtype=F32, device=dev)
+    wqkv = (ctypes.c_void_p * 3)(*(ws[n].data_ptr() for n in 'qkv'))
+    qkv_out = (ctypes.c_void_p * 3)(*(qkv[i].data_ptr() for i in range(3)))
+    _lib.call('noise_rows_qkv', pop, xs.data_ptr(), wqkv, cs.data_ptr(), sn.data_ptr(), _lib.ptr(ve),
+              _lib.ptr(ws.get('gate')), qkv_out, stream)
+    if attn is not None:
+        # the attn.c_proj jitter rides with the residual rows its product is added to (y serves as the norm's scratch)
+        moved = torch.empty(B, T, C, dtype=F32, device=dev)
+        _lib.call('noise_block_entry', xs.data_ptr(), B * T, attn.data_ptr(), B * T, moved.data_ptr(), y.data_ptr(), stream)
+        xs = moved
+    _lib.call('noise_attention_fwd', *qkv_out, y.data_ptr(), B, 8, T, 64, 8 * T * 64, T * 64, 64, 8 * T * 64, T * 64, 64,
+              8 * T * 64, T * 64, T, _lib.ATTN_V_TRANSPOSED | _lib.ATTN_QK_NORMED, T * C, 64, C, int(window), 0.125, None,
+              0, 1, None, stream)
+    if o is not None:
+        _lib.call('noise_add_bf16', y.data_ptr(), o.data_ptr(), y.numel(), stream)
+    js = None
+    if fc is not None or mlp is not None:
+        js = ctypes.byref(_lib.BlockJitter(_lib.ptr(fc), _lib.ptr(mlp), _zero_row_bf16(dev).data_ptr()))
+    split = _split_workspace(B, T, dev)
+    _lib.call('noise_block_tail', pop, _lib.View(y.data_ptr(), T * C, C), ws['proj'].data_ptr(),
+              _lib.View(xs.data_ptr(), T * C, C), ws['fc'].data_ptr(), ws['out'].data_ptr(), out.data_ptr(), js,
+              _lib.ptr(split), 0 if split is None else split.numel(), stream)
+    return out
+
+
+def _bf16_weight(t):
+    """bf16 contiguous copy of a weight (the reference's autocast casts it at every call too)."""
+    return t.detach().to(BF16).contiguous()
+
+
+def block_forward_tiled(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, mlp=None):
+    """block_forward_eager's results from the tiled kernels (noise_dust_block, no weight layouts): rerun_tiled's blocks, the
+    cross-check of the population kernels."""
     dev = x.device
     B, T, C = x.shape
     if C != 512 or T % 256:
@@ -305,7 +377,7 @@ def rerun_tiled(dust, n, entry, jitter):
         ve = dust.outputs.get(f'value_embeds.{i}')
         ve = None if ve is None else ve.detach().repeat(n, 1, 1)
         sites = {key: jitter.get(site.format(i)) for key, site in SITES.items()} if i == entry else {}
-        x = block_forward_eager(x, dust.weights[i], ve, cos, sin, model.window_sizes[i][0], **sites)
+        x = block_forward_tiled(x, dust.weights[i], ve, cos, sin, model.window_sizes[i][0], **sites)
     loss = head_loss_eager(x, model.lm_head.weight.detach().float(), dust.y.repeat(n, 1), model.config.vocab_size)
     return loss.view(n, b, T)
 

@@ -130,3 +130,27 @@ def test_workspace_is_checked():
     h, work = torch.empty(2, 128, 512, dtype=torch.bfloat16, device=DEV), _workspace(2, 128)
     with pytest.raises(RuntimeError, match='workspace'):
         _lib.call('noise_pop_block_split', *head, h.data_ptr(), 0, None, 0, None, None, work.data_ptr(), 100, stream)
+
+
+@pytest.mark.parametrize('B,T,layer,site', [(1, 256, 1, 'fc'), (1, 512, 0, None), (3, 256, 3, 'attn'), (5, 512, 2, 'mlp'),
+                                            (49, 256, 1, 'o'), (49, 256, 1, 'fc'), (56, 256, 5, 'mlp'), (65, 512, 7, 'attn'),
+                                            (100, 256, 4, None)])
+def test_block_forward_against_the_tiled_kernels(B, T, layer, site):
+    """block_forward at few and at many sequences (split launches, one workgroup per tile) against noise_dust_block. Both
+    round to bf16 at the same six places (h, q/k/v, weights, y, h, hidden) with sums in other orders: an increment differs by
+    less than sqrt(6) 2^-9 = 4.8e-3 of itself."""
+    from noise_amd.dust import block_forward, block_forward_tiled
+    from noise_amd.model import rotary_tables, window_sizes
+    g = torch.Generator(DEV).manual_seed(B + T)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    w = dict(q=r(512, 512) * .044, k=r(512, 512) * .044, v=r(512, 512) * .044, proj=r(512, 512) * .044,
+             fc=r(2048, 512) * .044, out=r(512, 2048) * .022, gate=r(8, 32) * .3 if layer % 2 else None)
+    ve = r(B, T, 512) if layer % 2 else None
+    jit = {site: r(B, T, 2048 if site == 'fc' else 512) * .1} if site else {}
+    x = r(B * T * 512 + 1)[1:].view(B, T, 512)  # off the 16 B alignment
+    cos, sin = (t.to(DEV) for t in rotary_tables(T))
+    got = block_forward(x, w, ve, cos, sin, window_sizes()[layer], **jit)
+    ref = block_forward_tiled(x.clone(), w, ve, cos, sin, window_sizes()[layer], **jit)
+    rel = float((got - ref).norm() / (ref - x).norm())
+    print(B, T, layer, site, rel, flush=True)
+    assert rel <= 4.8e-3
