@@ -89,8 +89,8 @@ __global__ __launch_bounds__(1024) void update_weights_kernel(const float *__res
 // materialised buffer too long for the GEMM's own reads; NaN outside the draw. A thread per element, 256 elements of
 // one slice per workgroup and step, so the stores are whole lines. Bound by Philox's ten rounds of two 32 x 32 -> 64
 // multiplies per element (four elements 2^19 apart share a block, which slices cannot use): 512 directions of the 60
-// parameters, 38.4 M normals,
-// 159 us (split bf16 tables, one direction per lane and 2 B stores 2 np apart, took 662). grid = (sum of widths / 256, a share of the directions)
+// parameters, 38.4 M normals, 159 us (split bf16 tables, one direction per lane and 2 B stores 2 np apart, took 662).
+// grid = (sum of widths / 256, a share of the directions)
 template <bool BUFFER>
 __global__ __launch_bounds__(256) void update_slices_kernel(UpdateSet s, int64_t d0, int64_t n, DrawLayout dl,
                                                             const float *__restrict__ buf, int64_t numel) {
@@ -110,22 +110,32 @@ __global__ __launch_bounds__(256) void update_slices_kernel(UpdateSet s, int64_t
     }
 }
 
-// G[o][i] (+)= sum_d A[o][d] B[i][d] over the chunk's np directions, A = hi_a + lo_a and B = hi_b + lo_b, as
+// G[o][i] (+)= sum_d A[o][d] B[i][d] over the chunk's directions, A = hi_a + lo_a and B = hi_b + lo_b, as
 // hi_a hi_b + hi_a lo_b + lo_a hi_b: one 256 x 256 tile of one parameter per workgroup. 8 waves of 128 (A rows)
 // x 64 (B rows), four 32 x 32 accumulator blocks by two. Workgroups past the first `full` take part q of `split`
 // equal ranges of the chunk's directions for tile full + (wg - full) / split and write that partial tile to part
 // (summed in order by update_reduce_kernel): the last, partial round of workgroups then runs `split` times
-// shorter. Per stage, 32 directions of the tile's 512 rows (64 KiB), two stages in flight; per 16 directions a
-// wave reads its hi and lo fragments once for 24 products.
+// shorter. A stage is 16 directions of the tile's 512 rows (34 KiB) in a ring of four; a wave reads its hi and lo
+// fragments once for 24 products.
 //
-// A stage is the 32 directions' fp32 slices themselves, from the materialised draw or a slab, [direction][A rows | B
+// A stage is the 16 directions' fp32 slices themselves, from the materialised draw or a slab, [direction][A rows | B
 // rows] at a stride of 2176 B (2 KiB + 128), copied straight from the buffer (16 B per lane; slices start at any
-// element). Each wave copies 4 directions and, once its copies have landed, splits them in place: the 32 B
-// holding rows 8 c .. 8 c + 7 of a direction become [hi x 8 | lo x 8] (lo first where bit 1 of the direction is
+// element). Each wave copies 2 directions and, once its copies have landed, splits them in place: the 16 B
+// holding rows 4 c .. 4 c + 3 of a direction become [hi x 4 | lo x 4] (lo first where bit 1 of the direction is
 // set), so nothing crosses lanes or waves before the stage's barrier. Fragments are then read with gfx950's
 // transposing LDS read (ds_read_b64_tr_b16: in each 16 lanes, lane i takes element i % 4 of the 8 B that lane
 // i / 4 + 4 e addresses), which gathers a row's 4 consecutive directions from 4 direction rows. The odd stride
 // (128 B apart mod 256) and the hi / lo swap put a read's 4 directions on 4 disjoint sets of banks.
+//
+// Between two barriers every wave forms stage s's products and splits its share of stage s + 1: waves 0-3 in that
+// order, waves 4-7 (the others of each SIMD) the other way round, so that one wave's conversions and LDS round trips
+// run under the other's products; copies of stages s + 2 and s + 3 are in flight meanwhile. What a wave does besides
+// its products bounds the stage, so that path is kept short: addresses, weights and the test that a slice lies inside
+// the buffer are formed for 32 stages at once, one (stage, direction) per lane, and stages of which one slice does
+// not (or is padding) take a branch of their own. 8192 directions of the 576 tiles from a 1 GiB draw: 1868 us (0.99
+// PFLOP/s of products). With stages of 32 directions, all waves in one order, both directions' addresses and tests
+// formed at each stage and the hi / lo halves stored as 8 B each it took 2158 (the matrix cores busy 38% of the time).
+// Of the 1868, splitting accounts for about 330 and the slices' distance (HBM against a draw that fits in L2) for 320.
 struct UpdateRaw {
     int64_t d0, n;             // the chunk's first direction and its directions (zeros fill the last stage)
     const float *weight;
@@ -133,13 +143,17 @@ struct UpdateRaw {
     const float *buf;          // fp32 [numel], numel <= 2^30 (lane offsets are 32-bit byte offsets); NULL: the slabs
     int64_t numel;
 };
+constexpr int kUgDirs = 16;          // directions per stage
 constexpr int kUgDir = 2176;         // bytes per direction of a stage (2 KiB of rows, 128 B apart)
-constexpr int kSt = 32 * kUgDir;
+constexpr int kSt = kUgDirs * kUgDir;
+constexpr int kUgRing = 4;           // stages in LDS
+constexpr int kUgOwn = kUgRing * kSt;        // each wave's offsets and weights of 32 stages (lo, hi, weight: 256 B)
+constexpr int kUgLds = kUgOwn + 8 * 768;
 __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accumulate, int full, int split,
                                                           float *__restrict__ part, UpdateRaw raw) {
-    __shared__ __attribute__((aligned(16))) char lds[2 * kSt];
+    __shared__ __attribute__((aligned(16))) char lds[kUgLds];
     // workgroups are dispatched round-robin over the 8 XCDs: each XCD takes a contiguous range of the full
-    // tiles (and of the partial items), so the tiles that share a table panel run under one L2
+    // tiles (and of the partial items), so the tiles that share a slice's panel run under one L2
     int wg = blockIdx.x;
     if (wg < full) {
         if ((full & 7) == 0) wg = (wg & 7) * (full >> 3) + (wg >> 3);
@@ -159,129 +173,146 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accum
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn0 = 128 * (wave & 1), wm0 = 64 * (wave >> 1);
     const unsigned lbase = lds_addr(lds);
-    // stages k0 .. k0 + nk - 1 of the chunk's, 32 directions each (a partial workgroup's range may be empty)
-    const int stages = (int)((raw.n + 31) / 32), q0 = partial ? item % split : 0, qn = partial ? split : 1;
-    const int k0 = stages * q0 / qn, nk = stages * (q0 + 1) / qn - k0;
+    // stages k0 .. k0 + nk - 1 of the chunk's, 16 directions each (a partial workgroup's range may be empty)
+    const int stages = (int)((raw.n + kUgDirs - 1) / kUgDirs);
+    const int q0 = partial ? item % split : 0, qn = partial ? split : 1;
+    const int k0 = (int)((int64_t)stages * q0 / qn), nk = (int)((int64_t)stages * (q0 + 1) / qn) - k0;
 
-    // wave w copies and splits directions 4 w + i (i = 0 .. 3) of each stage. The offsets and weights
-    // are read through the scalar cache (address space 4: this kernel writes neither).
-    typedef const __attribute__((address_space(4))) int64_t *c_i64p;
-    typedef const __attribute__((address_space(4))) float *c_f32p;
-    const c_i64p offs = (c_i64p)s.offsets[p];
     const float *buf = raw.buf ? raw.buf : s.slab[p];
     const int64_t numel = raw.buf ? raw.numel : raw.n * (rows + cols);
-    const c_f32p wts = (c_f32p)raw.weight;
     const int64_t side0 = (int64_t)ot * kTile, side1 = (int64_t)rows + ct * kTile;  // first slice element per side
+
+    // this wave's directions of a stage: dir0 and dir0 + 2 (so that bit 1 of a direction is its place i)
+    const int dir0 = 4 * (wave >> 1) + (wave & 1);
+    // 32 stages at a time, lane l holds direction l % 2 of stage l / 2: the address of its slice's side 0, its weight
+    // and whether both sides lie inside the buffer. own() copies the offsets and weights to this wave's LDS area,
+    // take() reads them when the copies have landed.
+    const int64_t lane_dir = (int64_t)(lane >> 1) * kUgDirs + dir0 + 2 * (lane & 1);
+    auto own = [&](int ks) {
+        const int64_t e = (int64_t)(k0 + ks) * kUgDirs + lane_dir, last = raw.n - 1;
+        const unsigned k = (unsigned)(e < last ? e : last), at = lbase + kUgOwn + 768 * wave;
+        if (raw.buf) {
+            lds_dma4_at(s.offsets[p] + raw.d0, 8 * k, at);
+            lds_dma4_at(s.offsets[p] + raw.d0, 8 * k + 4, at + 256);
+        }
+        lds_dma4_at(raw.weight + raw.d0, 4 * k, at + 512);
+    };
+    unsigned a_lo = 0, a_hi = 0;
+    float w_own = 0.0f;
+    uint64_t inside = 0;
+    auto take = [&](int ks) {
+        const int64_t k = (int64_t)(k0 + ks) * kUgDirs + lane_dir;
+        const char *at = lds + kUgOwn + 768 * wave + 4 * lane;
+        const int64_t o = raw.buf ? (int64_t)(((uint64_t)*reinterpret_cast<const uint32_t *>(at + 256) << 32) |
+                                              *reinterpret_cast<const uint32_t *>(at))
+                                  : k * (rows + cols);
+        w_own = k < raw.n ? *reinterpret_cast<const float *>(at + 512) * raw.scale : 0.0f;
+        inside = __builtin_amdgcn_ballot_w64(k < raw.n && o >= 0 && o <= numel - side1 - kTile);
+        const uint64_t addr = (uint64_t)buf + 4 * (uint64_t)(o + side0);
+        a_lo = (unsigned)addr;
+        a_hi = (unsigned)(addr >> 32);
+    };
     // a side of a direction (256 rows, 1 KiB) in one copy of 16 B per lane (lane l: rows 4 l .. + 4; a slice may
-    // start at any element, so a lane's 16 B are 4 B aligned, which multi-dword global loads accept). The split
-    // of a stage follows its copies' issue with no other issue between (issue 0, split 0, issue 1, ...; split
-    // ks + 1 then issue ks + 2), so each direction's offset, scaled weight and kind pass from one to the other
-    // in wave-uniform registers. kind: 0 padding, 1 inside the buffer, 2 leaving it (elements outside: NaN)
-    int64_t d_off[4];
-    float d_w[4];
-    int d_kind[4];
-    auto issue_raw = [&](int ks) {
-        const unsigned st = lbase + (ks & 1) * kSt;
+    // start at any element, so a lane's 16 B are 4 B aligned, which multi-dword global loads accept). The weights pass
+    // from here to the split in wave-uniform registers; bit `slot` of slow: a direction of the stage is padding or
+    // leaves the buffer
+    float wt[3][2] = {};  // of stages ks + 1 .. ks + 3
+    unsigned slow = 0;
+    auto offset = [&](int64_t k) { return raw.buf ? s.offsets[p][raw.d0 + k] : k * (rows + cols); };
+    auto issue = [&](int ks, float (&w)[2]) {
+        const int slot = ks & (kUgRing - 1), at = 2 * (ks & 31);
+        const unsigned st = lbase + slot * kSt + dir0 * kUgDir;
+        if (((inside >> at) & 3) == 3) {
+            slow &= ~(1u << slot);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int dl = 4 * wave + i;
-            const int64_t k = (int64_t)(k0 + ks) * 32 + dl;
-            int64_t o = 0;
-            int kind = 0;
-            float w = 0.0f;
-            if (k < raw.n) {
-                o = raw.buf ? offs[raw.d0 + k] : k * (rows + cols);
-                w = wts[raw.d0 + k] * raw.scale;
-                kind = o + side0 >= 0 && o + side1 + kTile <= numel ? 1 : 2;
+            for (int i = 0; i < 2; ++i) {
+                const uint64_t addr = ((uint64_t)(unsigned)__builtin_amdgcn_readlane((int)a_hi, at + i) << 32) |
+                                      (unsigned)__builtin_amdgcn_readlane((int)a_lo, at + i);
+                w[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w_own), at + i));
+                lds_dma16_at((const void *)addr, (unsigned)(16 * lane), st + 2 * i * kUgDir);
+                lds_dma16_at((const void *)(addr + 4 * (side1 - side0)), (unsigned)(16 * lane),
+                             st + 2 * i * kUgDir + 1024);
             }
-            d_off[i] = o;
-            d_w[i] = w;
-            d_kind[i] = kind;
-            if (kind == 1) {
-                lds_dma16_at(buf + o + side0, (unsigned)(16 * lane), st + dl * kUgDir);
-                lds_dma16_at(buf + o + side1, (unsigned)(16 * lane), st + dl * kUgDir + 1024);
-            } else {
-                // 4 B copies with every lane's element clamped into the buffer (a padding direction reads row 0)
-#pragma unroll
-                for (int side = 0; side < 2; ++side)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        int64_t L = kind ? o + (side ? side1 : side0) + 64 * q + lane : 0;
-                        L = L < 0 ? 0 : (L < numel ? L : numel - 1);
-                        lds_dma4_at(buf, (unsigned)(4 * L), st + dl * kUgDir + side * 1024 + 256 * q);
-                    }
+        } else {
+            // 4 B copies with every lane's element clamped into the buffer (a padding direction reads element 0)
+            slow |= 1u << slot;
+#pragma unroll 1
+            for (int i = 0; i < 2; ++i) {
+                const int64_t k = (int64_t)(k0 + ks) * kUgDirs + dir0 + 2 * i;
+                const int64_t o = k < raw.n ? offset(k) : 0;
+#pragma unroll 1
+                for (int q = 0; q < 8; ++q) {
+                    int64_t L = k < raw.n ? o + (q >= 4 ? side1 : side0) + 64 * (q & 3) + lane : 0;
+                    L = L < 0 ? 0 : (L < numel ? L : numel - 1);
+                    lds_dma4_at(buf, (unsigned)(4 * L), st + 2 * i * kUgDir + 256 * q);
+                }
             }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                w[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w_own), at + i));
         }
     };
-    // split stage ks (buffer ks % 2) in place: lane l takes side l / 32, rows 64 q + 8 c .. + 8 (q = (l / 8) % 4,
-    // c = l % 8) of each of the wave's 4 directions
-    auto split_raw = [&](int ks) {
-        char *st = lds + (ks & 1) * kSt;
-        const int side = lane >> 5, q = (lane >> 3) & 3, cp = lane & 7;
-        // the two 16 B halves (rows + 0 .. 3, + 4 .. 7) in the order h, 1 - h with h = bit 3 of the lane: each
-        // 16-lane pass then covers every bank once
-        const int h0 = (lane >> 3) & 1;
+    // split this wave's share of a stage in place: lane l takes rows 4 l .. + 4 of each side and direction. a rows:
+    // weight * scale; b rows as they are
+    auto split_raw = [&](int ks, const float (&w)[2]) {
+        const int slot = ks & (kUgRing - 1);
+        char *c = lds + slot * kSt + dir0 * kUgDir + 16 * lane;
+        float4 v4[2][2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int dl = 4 * wave + i, sb = (i >> 1) & 1;
-            char *c = st + dl * kUgDir + side * 1024 + 256 * q + 32 * cp;
-            const float4 v4[2] = {*reinterpret_cast<const float4 *>(c + 16 * h0),
-                                  *reinterpret_cast<const float4 *>(c + 16 * (1 - h0))};
-            // a rows: weight * scale; b rows: 1. Each case converts on its own, so that the common one (kind 1)
-            // keeps its loaded registers (a merge after the rare cases' rewrites would copy them)
-            const float w = side ? 1.0f : d_w[i];
-            auto convert = [&](const float4 (&x)[2], float wx) {
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract)
-#pragma clang fp contract(off)
-                    const int hh = t ? 1 - h0 : h0;
-                    const float v[4] = {x[t].x * wx, x[t].y * wx, x[t].z * wx, x[t].w * wx};
-                    bf16x4 hi, lo;
+            for (int side = 0; side < 2; ++side)
+                v4[i][side] = *reinterpret_cast<const float4 *>(c + 2 * i * kUgDir + 1024 * side);
+        if ((slow >> slot) & 1) {
+            // zeros for a padding direction, NaN for a slice's elements outside the buffer
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int64_t k = (int64_t)(k0 + ks) * kUgDirs + dir0 + 2 * i;
+                const int64_t o = k < raw.n ? offset(k) : 0;
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    const int64_t L = o + (side ? side1 : side0) + 4 * lane;
+                    float *f = reinterpret_cast<float *>(&v4[i][side]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        hi[e] = (__bf16)v[e];
-                        lo[e] = (__bf16)(v[e] - (float)hi[e]);
+                        const bool in = L + e >= 0 && L + e < numel;
+                        f[e] = k >= raw.n ? 0.0f : in ? f[e] : __builtin_nanf("");
                     }
-                    *reinterpret_cast<bf16x4 *>(c + 16 * sb + 8 * hh) = hi;
-                    *reinterpret_cast<bf16x4 *>(c + 16 * (1 - sb) + 8 * hh) = lo;
                 }
-            };
-            if (d_kind[i] == 1) {
-                convert(v4, w);
-            } else if (d_kind[i] == 0) {
-                // a padding direction: zeros
-                const float4 z[2] = {float4{0.f, 0.f, 0.f, 0.f}, float4{0.f, 0.f, 0.f, 0.f}};
-                convert(z, 1.0f);
-            } else {
-                // the slice leaves the buffer: its elements outside read as NaN
-                const int64_t L = d_off[i] + (side ? side1 : side0) + 64 * q + 8 * cp;  // the first of the 8 rows
-                float4 y[2] = {v4[0], v4[1]};
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const int64_t Lh = L + 4 * (t ? 1 - h0 : h0);
-                    float *f = reinterpret_cast<float *>(&y[t]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) f[e] = (Lh + e >= 0 && Lh + e < numel) ? f[e] : __builtin_nanf("");
-                }
-                convert(y, w);
             }
         }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                // v rounded to fp32 first, then lo = v - hi exactly (no fused multiply-subtract)
+#pragma clang fp contract(off)
+                const float4 x = v4[i][side];
+                const float v[4] = {side ? x.x : x.x * w[i], side ? x.y : x.y * w[i], side ? x.z : x.z * w[i],
+                                    side ? x.w : x.w * w[i]};
+                bf16x8 hl;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const __bf16 hi = (__bf16)v[e];
+                    hl[4 * i + e] = hi;
+                    hl[4 * (1 - i) + e] = (__bf16)(v[e] - (float)hi);
+                }
+                *reinterpret_cast<bf16x8 *>(c + 2 * i * kUgDir + 1024 * side) = hl;
+            }
     };
 
-    // lane 16 G + i addresses direction 8 (G / 2) + i / 4 (+ 16 sk + 4 e) and rows 16 (G % 2) + 4 (i % 4)
+    // lane 16 G + i addresses direction 8 (G / 2) + i / 4 (+ 4 e) and rows 16 (G % 2) + 4 (i % 4)
     // .. + 4 of a 32-row block; bit 1 of that direction (bit 3 of i) swaps hi and lo. tro[lo]
     int tro[2];
     {
         const int G = lane >> 4, i = lane & 15;
-        const int grp = 2 * (G & 1) + ((i & 3) >> 1);  // row group within the block (0 .. 3)
 #pragma unroll
         for (int lo = 0; lo < 2; ++lo)
-            tro[lo] = (8 * (G >> 1) + (i >> 2)) * kUgDir + 32 * grp + 16 * (((i >> 3) & 1) ^ lo) + 8 * (i & 1);
+            tro[lo] = (8 * (G >> 1) + (i >> 2)) * kUgDir + 64 * (G & 1) + 16 * (i & 3) + 8 * (((i >> 3) & 1) ^ lo);
     }
-    // 32 rows from row R (a multiple of 32 within the side), directions 16 sk + 8 hf + 0 .. 7
-    auto tr_frag = [&](const char *st, int side, int R, int sk, int lo) {
-        const char *b = st + tro[lo] + side * 1024 + 4 * R + 16 * sk * kUgDir;
+    // 32 rows from row R (a multiple of 32 within the side), directions 8 hf + 0 .. 7
+    auto tr_frag = [&](const char *st, int side, int R, int lo) {
+        const char *b = st + tro[lo] + side * 1024 + 4 * R;
         const bf16x4 x = lds_read_tr16(b), y = lds_read_tr16(b + 4 * kUgDir);
         return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
     };
@@ -291,58 +322,70 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accum
     for (int fb = 0; fb < 4; ++fb)
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) acc[fb][tb] = f32x16{};
-    // fragments of 16 directions, double buffered: those of the next step are read while this step's run
-    bf16x8 ah[2][4], al[2][4], bh[2][2], bl[2][2];
-    auto fetch = [&](int buf, const char *st, int sk) {
-#pragma unroll
-        for (int fb = 0; fb < 4; ++fb) {
-            ah[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 0);
-            al[buf][fb] = tr_frag(st, 0, wn0 + 32 * fb, sk, 1);
-        }
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-            bh[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 0);
-            bl[buf][tb] = tr_frag(st, 1, wm0 + 32 * tb, sk, 1);
-        }
-    };
     // the three products as three passes over the 8 accumulators: dependent products 8 apart
-    auto products = [&](int buf) {
+    auto products = [&](int slot) {
+        const char *st = lds + slot * kSt;
+        bf16x8 ah[4], al[4], bh[2], bl[2];
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) bh[tb] = tr_frag(st, 1, wm0 + 32 * tb, 0);
+#pragma unroll
+        for (int fb = 0; fb < 4; ++fb) ah[fb] = tr_frag(st, 0, wn0 + 32 * fb, 0);
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) bl[tb] = tr_frag(st, 1, wm0 + 32 * tb, 1);
+#pragma unroll
+        for (int fb = 0; fb < 4; ++fb) al[fb] = tr_frag(st, 0, wn0 + 32 * fb, 1);
 #pragma unroll
         for (int pr = 0; pr < 3; ++pr)
 #pragma unroll
             for (int fb = 0; fb < 4; ++fb)
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb)
-                    acc[fb][tb] = mfma32x32x16(pr == 2 ? al[buf][fb] : ah[buf][fb], pr == 1 ? bl[buf][tb] : bh[buf][tb],
-                                               acc[fb][tb]);
+                    acc[fb][tb] = mfma32x32x16(pr == 2 ? al[fb] : ah[fb], pr == 1 ? bl[tb] : bh[tb], acc[fb][tb]);
     };
-    // (a direction's copies number 2 or 8, so stage 0 lands and is split before stage 1 is issued: every later wait
-    // is for all copies in flight)
+    // this wave's copies of stage ks landed: those of at most two later stages (4 or more each) may still fly
+    auto landed = [&](int ks) {
+        vm_wait_groups<4, 2>(nk - 1 - ks < 2 ? nk - 1 - ks : 2);
+        asm volatile("" ::: "memory");
+    };
+    const bool split_first = wave >= 4;
     if (nk > 0) {
-        issue_raw(0);
+        float w0[2];
+        own(0);
         vm_wait<0>();
         asm volatile("" ::: "memory");
-        split_raw(0);
+        take(0);
+        issue(0, w0);
+        if (nk > 1) issue(1, wt[0]);
+        if (nk > 2) issue(2, wt[1]);
+        landed(0);
+        split_raw(0, w0);
         __syncthreads();
-        if (nk > 1) issue_raw(1);
-        fetch(0, lds, 0);
     }
 #pragma unroll 1
     for (int ks = 0; ks < nk; ++ks) {
-        const char *st = lds + (ks & 1) * kSt;
-        fetch(1, st, 1);
-        products(0);
-        // this wave splits its part of stage ks + 1 once its copies landed (nothing was issued after them), under the
-        // tail of this stage's products and with no fragments held
-        products(1);
-        if (ks + 1 < nk) {
-            vm_wait<0>();
-            asm volatile("" ::: "memory");
-            split_raw(ks + 1);
-            __syncthreads();  // stage ks + 1 split; every wave has read its fragments of stage ks
-            if (ks + 2 < nk) issue_raw(ks + 2);
-            fetch(0, lds + ((ks + 1) & 1) * kSt, 0);
+        if (ks + 3 < nk) {
+            // the next 32 stages' offsets are copied 16 stages before they are taken
+            if (((ks + 3) & 31) == 16 && ks + 19 < nk) own(ks + 19);
+            if (((ks + 3) & 31) == 0) take(ks + 3);
+            issue(ks + 3, wt[2]);  // into the slot of stage ks - 1, which every wave has left
         }
+        if (split_first && ks + 1 < nk) {
+            landed(ks + 1);
+            split_raw(ks + 1, wt[0]);
+        }
+        __builtin_amdgcn_s_setprio(1);  // the matrix cores before the other wave's conversions
+        products(ks & (kUgRing - 1));
+        __builtin_amdgcn_s_setprio(0);
+        if (!split_first && ks + 1 < nk) {
+            landed(ks + 1);
+            split_raw(ks + 1, wt[0]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            wt[0][i] = wt[1][i];
+            wt[1][i] = wt[2][i];
+        }
+        __syncthreads();  // stage ks + 1 split; every wave has read its fragments of stage ks
     }
     // lane (j, hf), register 4 g + e of block (fb, tb): row o = wn0 + 32 fb + 8 g + 4 hf + e, column
     // i = wm0 + 32 tb + j; the 32 lanes of a half-wave write 128 contiguous bytes of one row (a partial tile:
@@ -418,8 +461,7 @@ __global__ __launch_bounds__(256) void update_small_kernel(UpdateSmall s, int64_
 // thread adds up to four entries' products; the chunks' sums go to part [chunk][entry] and are summed in order by
 // update_small_reduce_kernel. One workgroup per entry (update_small_kernel) draws a and b again for each of the 256
 // entries of a gate, 13 times the normals: 131,072 directions of the model's 6 small parameters, 148 + 6 us
-// against 923; below
-// kSmallPairs its single launch is the shorter.
+// against 923; below kSmallPairs its single launch is the shorter.
 constexpr int kSmallWidth = 512, kSmallEntries = 1024, kSmallDirs = 16;
 constexpr int64_t kSmallPairs = 4096;
 __global__ __launch_bounds__(256) void update_small_partial_kernel(UpdateSmall s, int64_t pairs, int64_t chunk,
