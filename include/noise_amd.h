@@ -582,9 +582,9 @@ typedef struct {
     int64_t rows, cols;
 } noise_update_param_t;
 
-/* Bytes of workspace noise_update_gradients needs for these parameters at this chunk of directions: the split-bf16
- * tables, then room for the GEMM's partial tiles on a 256-CU device (a workspace that holds only the tables is
- * accepted: the GEMM then runs whole tiles only, with the same results up to summation order). */
+/* Bytes of workspace noise_update_gradients needs for these parameters at this chunk of directions: a slab of
+ * (rows + cols) fp32 per direction for every matrix, then room for the GEMM's partial tiles on a 256-CU device (a
+ * workspace that holds only the slabs is accepted: the GEMM then runs whole tiles only, with the same results up to summation order). */
 int64_t noise_update_workspace_bytes(const noise_update_param_t *params, int nparams, int64_t pairs,
                                      int64_t chunk);
 
@@ -594,11 +594,11 @@ int64_t noise_update_workspace_bytes(const noise_update_param_t *params, int npa
  * grad = scale * sum_d weight[d] a_d for 1-D parameters. The reference's p.grad is scale = -1/len(fitness).
  * Parameters with both sides multiples of 256 run as split-bf16x3 MFMA GEMMs over chunks of `chunk`
  * directions (rounded up to 256), accumulated in order; others (<= 65536 entries) are summed directly.
- * The matrices' slices are regenerated from the Philox counter in-kernel (through the split tables), or, when
+ * The matrices' slices are regenerated from the Philox counter into the workspace's slabs, or, when
  * `buffer` is non-NULL, read from that materialised draw (fp32 [numel], noise_normal_fill of the same draw):
  * cheaper once pairs * sum(rows + cols) exceeds numel, since every buffer element then serves several
- * directions. With a buffer of at most 2^30 elements the GEMM copies the slices straight from it and splits
- * them itself (the workspace's table area is then unused; the results are the same bits). An element of a
+ * directions. With a buffer of at most 2^30 elements the GEMM copies the slices straight from it (the
+ * workspace's slabs are then used only for the small parameters' partial sums; the results are the same bits). An element of a
  * slice outside [0, numel) reads as NaN. */
 int noise_update_gradients(const noise_update_param_t *params, int nparams, int64_t pairs, const float *weight,
                            float scale, int64_t chunk, int64_t numel, uint64_t seed, uint64_t offset,
