@@ -767,7 +767,7 @@ int pop_block_impl(const char *fn, const noise_population_t *pop, noise_view_t y
         NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
         if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
         split_tail_launch(a, mix != 0, xout, workspace, (hipStream_t)stream);
-        split_norm_launch(a, xout, (int)nnext, split3 != 0, (hipStream_t)stream);
+        split_norm_launch(a, static_cast<const float *>(workspace), (int)nnext, split3 != 0, (hipStream_t)stream);
         return launch_status(fn);
     }
     const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
@@ -832,7 +832,7 @@ int pop_block_qkv_impl(const char *fn, const noise_population_t *pop, noise_view
         NOISE_TRY_SPLIT(split_check(fn, a, xout, workspace, workspace_bytes));
         if (jit) NOISE_TRY_SPLIT(block_jitter(fn, a, jit));
         split_tail_launch(a, mix != 0, xout, workspace, (hipStream_t)stream);
-        split_qkv_launch(a, ve ? 1 : 0, (hipStream_t)stream);
+        split_qkv_launch(a, static_cast<const float *>(workspace), true, ve ? 1 : 0, (hipStream_t)stream);
         return launch_status(fn);
     }
     const dim3 grid((unsigned)(pop->members * (pop->tokens / kBlkTok)));
@@ -989,6 +989,6 @@ extern "C" int noise_rows_qkv(const noise_population_t *pop, const float *x, con
                         0, nullptr, nullptr, out);
     a.q.ve_rows = (const __bf16 *)ve_rows;
     a.q.gate_w = gate_w;
-    split_qkv_launch(a, ve_rows ? 2 : 0, (hipStream_t)stream);
+    split_qkv_launch(a, a.xout, false, ve_rows ? 2 : 0, (hipStream_t)stream);
     return launch_status(fn);
 }

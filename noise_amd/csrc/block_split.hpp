@@ -7,13 +7,14 @@
 //   split_qkv_kernel               the next block's gates, q, k, v from norm(x_out), a part of the 24 heads
 //   (split_norm_kernel             the last block: the head's rows from norm(x_out))
 //
-// x_mid (fp32) and hid (bf16, in the order the second product reads it) pass through a workspace. A workgroup still
-// holds 128 tokens of one member in 8 waves of 16 with the same lanes, products in the same order and the same
-// reductions as block_kernel, and every workgroup that needs a row's norm forms it from the whole row: the results are
-// block_kernel's bit for bit, so a loss does not depend on how many members are evaluated together. What it costs is
-// the rows read again by each part and the launches; what it gives is CUs: 16 tiles (8 members x 256 tokens) take 83 us
-// per block against 187 on 16 workgroups (split_rows 10 and 23, split_fc 20, split_qkv 22 to 30). The launches are bound
-// by what a CU can load (about 62 GB/s, 384 to 640 KiB per workgroup) and their own start.
+// x_mid (fp32), hid (bf16) and x_out for the last launch pass through a workspace, in the order the lanes hold them: a
+// wave's load or store is then 1 KiB in one piece instead of 16 rows of 64 B. A workgroup still holds 128 tokens of one
+// member in 8 waves of 16 with the same lanes, products in the same order and the same reductions as block_kernel, and
+// every workgroup that needs a row's norm forms it from the whole row: the results are block_kernel's bit for bit, so a
+// loss does not depend on how many members are evaluated together. What it costs is the rows read again by each part
+// and the launches; what it gives is CUs: 16 tiles (8 members x 256 tokens) take 67 us per block against 187 on 16
+// workgroups (split_rows 10 and 17, split_fc 15, split_qkv 25; with rows in memory order 10, 23, 20 and 30). The
+// launches are bound by what a CU can load (384 to 640 KiB per workgroup) and their own start (4 us when empty).
 #pragma once
 #include "common.hpp"
 #include "mfma.hpp"
@@ -29,17 +30,18 @@ constexpr int kSplitLds = kSplitRing + kHidden * 4;  // and mlp.c_proj's b
 struct SplitRowsArgs {
     int members, tokens, dir_div, parts;
     const float *sign;
-    const __bf16 *x;                  // operand rows: y (strided), or hid [rows][2048] in operand order
+    const __bf16 *x;                  // operand: y's rows (strided), or WIDE: hid in lane order
     int64_t xs_m, xs_t;
     const __bf16 *w;                  // [512][K]
-    const float *res;                 // fp32 rows the products accumulate onto
+    const float *res;                 // fp32 rows the products accumulate onto (WIDE: mid)
     int64_t rs_m, rs_t;
     const float *a, *b;               // rank-1 rows (b: WIDE only) or NULL
     int64_t a_stride, b_stride;
     const float *dots;                // !WIDE: partial sums of y . b_o [rows][ndots]
     int ndots;
     const __bf16 *jit;                // WIDE: bf16 rows of 512 added to the product, or NULL
-    float *out;                       // [rows][512]
+    float *mid;                       // lane order: x_mid out, or WIDE: x_mid in, x_out out
+    float *out;                       // WIDE: [rows][512]
     int mix;
     const float *lam_r, *lam_x, *eps_r, *eps_x;
     int64_t eps_stride;
@@ -47,8 +49,11 @@ struct SplitRowsArgs {
     int64_t x0_m, x0_t;
 };
 
-// 16 NB output features of 128 tokens: the weights' rows stream through LDS in chunks of 1024 / NB columns (32 KiB: [column
-// tiles of 64][16 NB rows][128 B]), four buffers; a wave's operand fragments come from global memory a chunk ahead.
+// lane order of 16 rows from row 16 G: [G][block of 16 features][lane][4] fp32, [G][step of 32 units][lane][8] bf16
+__device__ __forceinline__ int64_t lane_block(int64_t row, int blocks) { return (row >> 4) * blocks * 64; }
+
+// 16 NB output features of 128 tokens: the weights' rows stream through LDS in chunks of 1024 / NB columns (32 KiB:
+// [column tiles of 64][16 NB rows][128 B]), four buffers; a wave's operand fragments come from global memory a chunk ahead.
 // WIDE: K = 2048 with hid . b_proj from the fragments; else K = 512 with y . b_o from the attention's partial sums.
 template <int NB, bool WIDE>
 __global__ __launch_bounds__(kBlkThreads, 1) void split_rows_kernel(SplitRowsArgs p) {
@@ -87,16 +92,19 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_rows_kernel(SplitRowsArg
     if constexpr (WIDE) {
         if (p.a) lds_dma16_at(p.b + dir * p.b_stride + 256 * wave, (unsigned)(16 * lane), lbase + kSplitRing + 1024 * wave);
     }
-    const __bf16 *xr = p.x + m * p.xs_m + (int64_t)tok * p.xs_t + 8 * g;
+    constexpr int XS = WIDE ? 512 : 32;  // elements from one k step to the next
+    const __bf16 *xr = WIDE ? p.x + (lane_block(row, kHidden / 32) + lane) * 8
+                            : p.x + m * p.xs_m + (int64_t)tok * p.xs_t + 8 * g;
     bf16x8 xf[2][JS];
 #pragma unroll
-    for (int j = 0; j < JS; ++j) xf[0][j] = load_bf16x8(xr + 32 * j);
+    for (int j = 0; j < JS; ++j) xf[0][j] = load_bf16x8(xr + XS * j);
+    float *mid = p.mid + (lane_block(row, kModel / 16) + 64 * NB * part + lane) * 4;
     f32x4 out[NB];
     {
-        const float *rr = p.res + m * p.rs_m + (int64_t)tok * p.rs_t + f0 + 4 * g;
+        const float *rr = WIDE ? mid : p.res + m * p.rs_m + (int64_t)tok * p.rs_t + f0 + 4 * g;
 #pragma unroll
         for (int ob = 0; ob < NB; ++ob) {
-            const float4 v = ld4(rr + 16 * ob);
+            const float4 v = ld4(rr + (WIDE ? 256 : 16) * ob);
             out[ob] = f32x4{v.x, v.y, v.z, v.w};
         }
     }
@@ -117,7 +125,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_rows_kernel(SplitRowsArg
         if (!kAll && c + 3 < NC) issue(c + 3);  // into the buffer of chunk c - 1, which every wave has left
         if (c + 1 < NC) {
 #pragma unroll
-            for (int j = 0; j < JS; ++j) xf[(c + 1) & 1][j] = load_bf16x8(xr + KC * (c + 1) + 32 * j);
+            for (int j = 0; j < JS; ++j) xf[(c + 1) & 1][j] = load_bf16x8(xr + XS * (JS * (c + 1) + j));
         }
         const char *buf = lds + (c & 3) * 32768;
         auto frag = [&](int f) {  // fragment f = NB j + ob: rows 16 ob .. + 16, k block j of the chunk
@@ -167,7 +175,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_rows_kernel(SplitRowsArg
     const float *ar = p.a ? p.a + dir * p.a_stride + f0 + 4 * g : nullptr;
     const float *zr = WIDE && p.mix ? p.x0 + m * p.x0_m + (int64_t)tok * p.x0_t + f0 + 4 * g : nullptr;
     const __bf16 *jr = WIDE && p.jit ? p.jit + row * kModel + f0 + 4 * g : nullptr;
-    float *dst = p.out + row * kModel + f0 + 4 * g;
+    float *dst = WIDE ? p.out + row * kModel + f0 + 4 * g : nullptr;
 #pragma unroll
     for (int ob = 0; ob < NB; ++ob) {
         const float4 a4 = ar ? ld4(ar + 16 * ob) : float4{0.f, 0.f, 0.f, 0.f};
@@ -184,16 +192,19 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_rows_kernel(SplitRowsArg
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = rl * v[r] + ml * f4get(z, r);
         }
-        st4(dst + 16 * ob, float4{v[0], v[1], v[2], v[3]});
+        st4(mid + 256 * ob, float4{v[0], v[1], v[2], v[3]});
+        if constexpr (WIDE) st4(dst + 16 * ob, float4{v[0], v[1], v[2], v[3]});
     }
 }
 
-// fp32 rows [rows][512] as block_kernel holds them (block ob, register r: feature 16 ob + 4 g + r) and 1 / rms
-__device__ __forceinline__ float split_load_rows(const float *x, int64_t row, int g, f32x4 (&out)[32]) {
-    const float *xr = x + row * kModel + 4 * g;
+// fp32 rows ([rows][512], or LANES: in lane order) as block_kernel holds them (block ob, register r: feature
+// 16 ob + 4 g + r) and 1 / rms
+template <bool LANES>
+__device__ __forceinline__ float split_load_rows(const float *x, int64_t row, int lane, f32x4 (&out)[32]) {
+    const float *xr = LANES ? x + (lane_block(row, kModel / 16) + lane) * 4 : x + row * kModel + 4 * (lane >> 4);
 #pragma unroll
     for (int ob = 0; ob < 32; ++ob) {
-        const float4 v = ld4(xr + 16 * ob);
+        const float4 v = ld4(xr + (LANES ? 256 : 16) * ob);
         out[ob] = f32x4{v.x, v.y, v.z, v.w};
     }
     float ssq = 0.f;
@@ -231,12 +242,12 @@ __device__ __forceinline__ void split_pack(const f32x4 (&out)[32], float rstd, b
 struct SplitFcArgs {
     int members, tokens, dir_div, parts;
     const float *sign;
-    const float *x;                   // x_mid [rows][512]
+    const float *x;                   // x_mid in lane order
     const __bf16 *w;                  // c_fc [2048][512], columns permuted
     const float *a, *b;               // rank-1 a [dirs][2048], b [dirs][512] or NULL
     int64_t a_stride, b_stride;
     const __bf16 *jit;                // bf16 [rows][2048] added before ReLU^2, or NULL
-    __bf16 *hid;                      // [rows][64 steps][4 lane groups][8]
+    __bf16 *hid;                      // in lane order
 };
 
 // 2048 / parts hidden units of 128 tokens, in chunks of 64 (64 KiB: [8 column tiles][64 rows][128 B], two buffers)
@@ -264,13 +275,13 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_fc_kernel(SplitFcArgs p)
     issue(0);
     if (nc > 1) issue(1);
     f32x4 out[32];
-    const float rstd = split_load_rows(p.x, row, g, out);
+    const float rstd = split_load_rows<true>(p.x, row, lane, out);
     const float corr = p.a ? sgn * (rstd * split_dot(p.b + dir * p.b_stride, g, out)) : 0.f;
     bf16x8 xf[16];
     split_pack(out, rstd, xf);
     vm_wait<0>();
     __syncthreads();
-    __bf16 *dst = p.hid + row * kHidden + 8 * g;
+    __bf16 *dst = p.hid + (lane_block(row, kHidden / 32) + lane) * 8;
     for (int c = 0; c < nc; ++c) {
         const char *buf = lds + (c & 1) * 65536;
 #pragma unroll
@@ -319,7 +330,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_fc_kernel(SplitFcArgs p)
                 hb[r] = (__bf16)(v0 * v0);
                 hb[4 + r] = (__bf16)(v1 * v1);
             }
-            store_bf16x8(dst + u, hb);
+            store_bf16x8(dst + 16 * u, hb);
         }
         if (c + 1 < nc) {
             __syncthreads();  // every wave is done with buffer c & 1
@@ -333,7 +344,8 @@ __global__ __launch_bounds__(kBlkThreads, 1) void split_fc_kernel(SplitFcArgs p)
 
 struct SplitQkvArgs {
     QkvRowsArgs q;
-    const float *x;                   // x_out [rows][512]
+    const float *x;                   // x_out
+    int lanes;                        // its order: 1 lane order, 0 [rows][512]
     const float *nb[3];
     int64_t nb_stride[3];
     int parts, heads;                 // heads per part (24 / parts)
@@ -360,7 +372,8 @@ __global__ __launch_bounds__(kQThreads, 1) void split_qkv_kernel(SplitQkvArgs p)
     bf16x8 xf[16];
     {
         f32x4 out[32];
-        const float rstd = split_load_rows(p.x, L.row, g, out);
+        const float rstd = p.lanes ? split_load_rows<true>(p.x, L.row, lane, out)
+                                   : split_load_rows<false>(p.x, L.row, lane, out);
         float dq[3] = {0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 3; ++k)
@@ -376,7 +389,7 @@ __global__ __launch_bounds__(kQThreads, 1) void split_qkv_kernel(SplitQkvArgs p)
 
 struct SplitNormArgs {
     int members, tokens, dir_div, split3;
-    const float *x;
+    const float *x;                   // in lane order
     const float *nb;                  // the head's b rows or NULL
     int64_t nb_stride;
     float *ndots;
@@ -389,7 +402,7 @@ __global__ __launch_bounds__(256) void split_norm_kernel(SplitNormArgs p) {
     const int64_t row = (int64_t)blockIdx.x * 64 + 16 * (tid >> 6) + tl;  // (tokens are whole 128s)
     const int dir = (int)(row / p.tokens) / p.dir_div;
     f32x4 out[32];
-    const float rstd = split_load_rows(p.x, row, g, out);
+    const float rstd = split_load_rows<true>(p.x, row, lane, out);
     if (p.ndots) {
         const float d = p.nb ? split_dot(p.nb + dir * p.nb_stride, g, out) : 0.f;
         if (g == 0) p.ndots[row] = rstd * d;
@@ -420,8 +433,8 @@ int split_parts(int64_t tiles) {
     while (p > 2 && tiles * p > 256) p /= 2;
     return p;
 }
-// up to this many token tiles the split launches are the faster ones: per block 83 against 187 us at 16 tiles, 125 at 64,
-// 179 at 96, 193 at 128
+// up to this many token tiles the split launches are the faster ones: per block 67 against 187 us at 16 tiles, 120 at
+// 64, 176 at 96, 208 at 128
 constexpr int64_t kSplitTiles = 96;
 int64_t split_bytes(int64_t rows) { return rows * (kModel * 4 + kHidden * 2); }
 
@@ -436,7 +449,7 @@ void split_rows_launch(const SplitRowsArgs &a, int64_t tiles, hipStream_t s) {
     }
 }
 
-// x_mid, hid and x_out of the block's arguments; xout: fp32 [rows][512]
+// x_mid, hid and x_out of the block's arguments; xout: fp32 [rows][512]; x_out in lane order at the workspace's start
 void split_tail_launch(const BlockArgs &a, bool mix, float *xout, void *workspace, hipStream_t s) {
     const int64_t rows = (int64_t)a.members * a.tokens, tiles = rows / kBlkTok;
     float *xmid = static_cast<float *>(workspace);
@@ -447,15 +460,14 @@ void split_tail_launch(const BlockArgs &a, bool mix, float *xout, void *workspac
     r.x = a.y; r.xs_m = a.ys_m; r.xs_t = a.ys_t; r.w = a.wo;
     r.res = a.xres; r.rs_m = a.xr_m; r.rs_t = a.xr_t;
     r.a = a.ao; r.a_stride = a.ao_stride; r.dots = a.odots; r.ndots = a.odots_n;
-    r.out = xmid;
+    r.mid = xmid;
     split_rows_launch<false>(r, tiles, s);
     SplitFcArgs f{};
     f.members = a.members; f.tokens = a.tokens; f.dir_div = a.dir_div; f.sign = a.sign; f.parts = r.parts;
     f.x = xmid; f.w = a.wfc; f.a = a.afc; f.b = a.bfc; f.a_stride = a.afc_stride; f.b_stride = a.bfc_stride;
     f.jit = a.jfc; f.hid = hid;
     hipLaunchKernelGGL(split_fc_kernel, dim3((unsigned)part_grid(tiles, f.parts)), dim3(kBlkThreads), 0, s, f);
-    r.x = hid; r.xs_m = (int64_t)a.tokens * kHidden; r.xs_t = kHidden; r.w = a.wpj;
-    r.res = xmid; r.rs_m = (int64_t)a.tokens * kModel; r.rs_t = kModel;
+    r.x = hid; r.w = a.wpj; r.res = nullptr;
     r.a = a.apj; r.a_stride = a.apj_stride; r.b = a.bpj; r.b_stride = a.bpj_stride; r.dots = nullptr; r.ndots = 0;
     r.jit = a.jmlp_st ? a.jmlp : nullptr;
     r.out = xout;
@@ -464,10 +476,11 @@ void split_tail_launch(const BlockArgs &a, bool mix, float *xout, void *workspac
     split_rows_launch<true>(r, tiles, s);
 }
 
-void split_qkv_launch(const BlockArgs &a, int ve, hipStream_t s) {
+// x: fp32 rows, lanes: in lane order
+void split_qkv_launch(const BlockArgs &a, const float *x, bool lanes, int ve, hipStream_t s) {
     const int64_t tiles = (int64_t)a.members * a.tokens / kBlkTok;
     SplitQkvArgs q;
-    q.q = a.q; q.x = a.xout;
+    q.q = a.q; q.x = x; q.lanes = lanes;
     for (int k = 0; k < 3; ++k) {
         q.nb[k] = a.nb[k];
         q.nb_stride[k] = a.nb_stride[k];
