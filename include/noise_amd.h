@@ -118,6 +118,8 @@ int noise_orthogonal_draws(void *out, int out_bf16, int64_t n, int64_t bt, int64
  * NOISE_ATTN_V_TRANSPOSED, element (b, t, h, d) at b*vs_b + h*vs_h + d*vs_x + t. head_dim must be 64.
  * Natural V runs the ring kernel at any seq, transposed V at a seq in whole 256-query tiles; the rest the general one.
  * NOISE_ATTN_OUT_FP32 (natural V): o is fp32 (strides in its elements, multiples of 4) holding the bf16 results.
+ * NOISE_ATTN_Q_FP32 (with NOISE_ATTN_OUT_FP32): q is fp32 (strides in its elements, multiples of 4), rounded to bf16 as
+ * it is read.
  * NOISE_ATTN_QK_NORMED: the caller guarantees every q and k row has RMS <= 1, as RMSNorm outputs do (the
  * reference normalises both, utils/model.py:94); scores are then bounded and the softmax runs with a
  * fixed shift instead of a running maximum (same result; rows that break the promise by less than a
@@ -128,6 +130,7 @@ int noise_orthogonal_draws(void *out, int out_bf16, int64_t n, int64_t bt, int64
 #define NOISE_ATTN_V_TRANSPOSED 1
 #define NOISE_ATTN_QK_NORMED 2
 #define NOISE_ATTN_OUT_FP32 4
+#define NOISE_ATTN_Q_FP32 8
 
 /* Up to three fp32 tensors [batch, tokens, heads, 64] (element (b, t, h, d) of tensor i at src[i] + b*s_b[i] + t*s_t[i] +
  * h*s_h[i] + d) rounded to bf16 [batch][tokens][heads][64] in one launch: noise_attention_fwd's operands. */

@@ -8,7 +8,7 @@ from pathlib import Path
 import torch
 
 from .abi import (SIGNATURES, LINEAR_AUTOCAST, ROUNDING_FUSED, ROUNDING_EAGER, ATTN_V_TRANSPOSED,  # noqa: F401
-                  ATTN_QK_NORMED, ATTN_OUT_FP32, CastHeads, View, Rank1, Population, UpdateParam, SliceGroups, SLICE_GROUPS_MAX, BlockJitter,
+                  ATTN_QK_NORMED, ATTN_OUT_FP32, ATTN_Q_FP32, CastHeads, View, Rank1, Population, UpdateParam, SliceGroups, SLICE_GROUPS_MAX, BlockJitter,
                   RandintSet, RANDINT_SETS_MAX, Weight, WEIGHTS_MAX, WEIGHT_BF16, WEIGHT_FP32, WEIGHT_FP32_ROUNDED, bind)
 
 # the in-tree build (noise_amd/build.py); no other library is ever loaded

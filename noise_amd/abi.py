@@ -91,6 +91,7 @@ ROUNDING_EAGER = 1
 ATTN_V_TRANSPOSED = 1
 ATTN_QK_NORMED = 2
 ATTN_OUT_FP32 = 4
+ATTN_Q_FP32 = 8
 
 
 class View(ctypes.Structure):

@@ -307,7 +307,10 @@ __device__ __forceinline__ int key_sigma(int i) { return (i & ~12) | ((i & 4) <<
 // the slot of tile t - 1, which B finished reading before that barrier.
 // VNAT: V in its natural layout [.., token, dim] (the drop-in's), copied as K is, with the 16 B chunks of row R
 // swizzled by 2 (R % 4) instead, and each V^T fragment put together from two transposing LDS reads.
-template <bool BOUNDED, bool VNAT, bool OF32 = false>
+// QF32: fp32 queries, rounded as they are read. Each is read once, so casting them beforehand as K and V are (which
+// every query tile reads again) only adds a write and a read: 5 x 8 heads x 1111 tokens, the cast 10.4 -> 8.1 us, this
+// kernel 22 -> 23, the call 30.9 -> 29.1
+template <bool BOUNDED, bool VNAT, bool OF32 = false, bool QF32 = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_vt_kernel(AttnArgs a) {
     constexpr int QT = kVtQT, NS = 4;
     constexpr int QB = 1, NW = QT / 32, QW = 32, CPW = 4;  // waves, queries per wave, copies per A wave
@@ -346,7 +349,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int q = q0w + 32 * qb + j;
-            qf[qb][s] = load_bf16x8(Qb + (int64_t)(VNAT && q > last ? last : q) * a.qs_t + 16 * s + 8 * hf);
+            const int64_t at = (int64_t)(VNAT && q > last ? last : q) * a.qs_t + 16 * s + 8 * hf;
+            if constexpr (QF32) {
+                const float *qp = reinterpret_cast<const float *>(a.q) + b * a.qs_b + h * a.qs_h + at;
+                const float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
+                qf[qb][s] = bf16x8{(__bf16)x.x, (__bf16)x.y, (__bf16)x.z, (__bf16)x.w,
+                                   (__bf16)y.x, (__bf16)y.y, (__bf16)y.z, (__bf16)y.w};
+            } else {
+                qf[qb][s] = load_bf16x8(Qb + at);
+            }
         }
     // the query fragments land before any tile copy is issued: the compiler's own wait for them inside the
     // tile loop would otherwise be a vmcnt that also drains the copies in flight
@@ -796,7 +807,8 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
                                    int64_t dot_vec_stride, int64_t dot_div, float *dot_out,
                                    noise_stream_t stream) {
     clear_error();
-    NOISE_CHECK_ARG((flags & ~(NOISE_ATTN_V_TRANSPOSED | NOISE_ATTN_QK_NORMED | NOISE_ATTN_OUT_FP32)) == 0,
+    NOISE_CHECK_ARG((flags & ~(NOISE_ATTN_V_TRANSPOSED | NOISE_ATTN_QK_NORMED | NOISE_ATTN_OUT_FP32 |
+                               NOISE_ATTN_Q_FP32)) == 0,
                     "noise_attention_fwd: unknown flags 0x%x", flags);
     const bool v_transposed = flags & NOISE_ATTN_V_TRANSPOSED;
     NOISE_CHECK_ARG(head_dim == kD, "noise_attention_fwd: head_dim must be 64, got %lld", (long long)head_dim);
@@ -806,9 +818,10 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     NOISE_CHECK_ARG(q && k && v && o, "noise_attention_fwd: NULL tensor pointer");
     NOISE_CHECK_ARG(aligned(q, 16) && aligned(k, 16) && aligned(o, 8) && aligned(v, v_transposed ? 2 : 16),
                     "noise_attention_fwd: q, k (16 B), o (8 B) and v must be aligned");
-    NOISE_CHECK_ARG(qs_t % 8 == 0 && ks_t % 8 == 0 && qs_b % 8 == 0 && qs_h % 8 == 0 && ks_b % 8 == 0 &&
+    const int qa = flags & NOISE_ATTN_Q_FP32 ? 4 : 8;
+    NOISE_CHECK_ARG(qs_t % qa == 0 && ks_t % 8 == 0 && qs_b % qa == 0 && qs_h % qa == 0 && ks_b % 8 == 0 &&
                         ks_h % 8 == 0 && os_t % 4 == 0 && os_b % 4 == 0 && os_h % 4 == 0,
-                    "noise_attention_fwd: q/k strides must be multiples of 8 elements, o strides of 4");
+                    "noise_attention_fwd: q/k strides must be multiples of 8 elements (4 for fp32 q), o strides of 4");
     if (v_transposed) {
         NOISE_CHECK_ARG(vs_x % 8 == 0 && vs_b % 8 == 0 && vs_h % 8 == 0 && aligned(v, 16),
                         "noise_attention_fwd: transposed v needs 16 B alignment and strides multiple of 8");
@@ -826,6 +839,8 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     const bool out_fp32 = flags & NOISE_ATTN_OUT_FP32;
     NOISE_CHECK_ARG(!out_fp32 || (vt_path && !v_transposed && aligned(o, 16)),
                     "noise_attention_fwd: fp32 output needs natural v, row strides below 2^25 and o 16 B aligned");
+    const bool q_fp32 = flags & NOISE_ATTN_Q_FP32;
+    NOISE_CHECK_ARG(!q_fp32 || out_fp32, "noise_attention_fwd: fp32 queries are served with fp32 output");
     const int64_t qtile = vt_path ? kVtQT : kBQ;
     int64_t qtiles = (seq + qtile - 1) / qtile;
     NOISE_CHECK_ARG(bh * qtiles < (1ll << 31), "noise_attention_fwd: too many workgroups");
@@ -849,7 +864,9 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     dim3 grid((unsigned)(bh * qtiles));
     if (vt_path) {
         const bool bounded = flags & NOISE_ATTN_QK_NORMED;
-        auto kernel = out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
+        auto kernel = q_fp32 ? (bounded ? attention_vt_kernel<true, true, true, true>
+                                        : attention_vt_kernel<false, true, true, true>)
+                      : out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
                       : v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
                                    : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>);
         hipLaunchKernelGGL(kernel, grid, dim3(512), 0, (hipStream_t)stream, a);

@@ -12,7 +12,7 @@ import torch
 from torch import nn
 
 from . import _lib
-from ._lib import ATTN_OUT_FP32, ATTN_QK_NORMED, ATTN_V_TRANSPOSED
+from ._lib import ATTN_OUT_FP32, ATTN_Q_FP32, ATTN_QK_NORMED, ATTN_V_TRANSPOSED
 
 BF16 = torch.bfloat16
 N_LAYER, N_HEAD, HEAD_DIM, N_EMBD, VOCAB, SEQ = 8, 8, 64, 512, 4096, 2048
@@ -168,7 +168,15 @@ def attention(q, k, v, window):
     B, T, H, D = q.shape
     stream = _lib.stream_ptr(q.device)
     ops, cast, n = [q, k, v], None, 0
-    for i, t in enumerate(ops):
+    flags = 0
+    for i in (1, 2, 0):
+        t = ops[i]
+        if i == 0 and t.dtype == torch.float32 and max(ops[1].stride(1), ops[2].stride(1)) < 1 << 25:
+            flags = ATTN_OUT_FP32
+            s = t.stride()
+            if D == HEAD_DIM and s[3] == 1 and not (s[0] | s[1] | s[2]) % 4 and not t.data_ptr() % 16:
+                flags |= ATTN_Q_FP32   # 16 B aligned rows are rounded by the kernel as it reads them
+                break
         if t.dtype == torch.float32 and D == HEAD_DIM and t.stride(-1) == 1:
             # fp32 operands are rounded together, in one launch
             if cast is None:
@@ -185,11 +193,10 @@ def attention(q, k, v, window):
     qb, kb, vb = ops
     ks, vs = kb.stride(), vb.stride()
     # V in its own layout: the ring kernel reads V^T fragments from natural V tiles with transposing LDS reads
-    fp32 = q.dtype == torch.float32 and max(ks[1], vs[1]) < 1 << 25
-    out = torch.empty(B, T, H, D, dtype=torch.float32 if fp32 else BF16, device=q.device)
+    out = torch.empty(B, T, H, D, dtype=torch.float32 if flags else BF16, device=q.device)
     qs, os = qb.stride(), out.stride()
     _lib.call('noise_attention_fwd', qb.data_ptr(), kb.data_ptr(), vb.data_ptr(), out.data_ptr(), B, H, T, D,
-              qs[0], qs[2], qs[1], ks[0], ks[2], ks[1], vs[0], vs[2], vs[1], ATTN_OUT_FP32 if fp32 else 0,
+              qs[0], qs[2], qs[1], ks[0], ks[2], ks[1], vs[0], vs[2], vs[1], flags,
               os[0], os[2], os[1], int(window), 1.0 / math.sqrt(D), None, 0, 1, None, stream)
     return out if out.dtype == q.dtype else out.to(q.dtype)
 

@@ -60,3 +60,35 @@ def test_rows_past_the_end_are_not_written(flags):
     assert (out[:, T:] == 9).all() and (dots[B * T * H:] == 9).all()
     expect = (out[:, :T].float() * vec.view(B, 1, H, 64)).sum(-1)
     assert torch.allclose(dots[:B * T * H].view(B, T, H), expect, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize('T', [1, 100, 257])
+@pytest.mark.parametrize('flags', [12, 14])
+def test_fp32_queries(T, flags):
+    """Queries rounded by the kernel: the bits of bf16 queries, in any strides of whole 16 B; odd ones and a bf16 output
+    are refused by the kernel's entry and served by the drop-in."""
+    from noise_amd import _lib
+    from noise_amd.model import attention
+    g = torch.Generator(DEV).manual_seed(T)
+    B, H = 2, 3
+    wide = torch.nn.functional.rms_norm(torch.randn(B, H, T + 1, 68, device=DEV, generator=g), (68,))
+    k, v = (torch.nn.functional.rms_norm(torch.randn(B, T, H, 64, device=DEV, generator=g), (64,)).bfloat16()
+            for _ in range(2))
+
+    def call(q, flags, dtype):
+        out = torch.full((B, T + 3, H, 64), 9.0, device=DEV, dtype=dtype)
+        s = [x for t in (q, k, v) for x in (t.stride(0), t.stride(2), t.stride(1))]
+        _lib.call('noise_attention_fwd', q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, T, 64, *s, flags,
+                  out.stride(0), out.stride(2), out.stride(1), 77, 0.125, None, 0, 1, None, _lib.stream_ptr(DEV))
+        assert (out[:, T:] == 9).all()
+        return out[:, :T]
+
+    q = wide[:, :, :T, :64].transpose(1, 2)   # [B, T, H, 64], rows of 68
+    assert torch.equal(call(q, flags, torch.float32), call(q.bfloat16().contiguous(), flags & ~8, torch.float32))
+    with pytest.raises(RuntimeError):
+        call(q, flags & ~4, torch.bfloat16)
+    odd = torch.randn(B, T, H, 65, device=DEV, generator=g)[..., :64]
+    with pytest.raises(RuntimeError):
+        call(odd, flags, torch.float32)
+    for t in (q, odd):
+        assert torch.equal(attention(t, k, v, 77), attention(t.bfloat16().contiguous(), k, v, 77).float())
