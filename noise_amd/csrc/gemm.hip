@@ -1072,7 +1072,9 @@ constexpr int kH3Step = 2 * kH3Part;          // hi then lo
 #define HEAD3_AHEAD 4
 #endif
 
-// XF32: x is fp32 [T][512], its rows split here, their norm applied to the logits (the head_loss drop-in, unperturbed)
+// XF32: x is fp32 [T][512], its rows split here, their norm applied to the logits (the head_loss drop-in, unperturbed).
+// Normalising first reads x twice: 67 us against 53 for 3,000 rows. The errors against 64 bits are the same either way
+// (120,000 rows: rms 3.11e-6, largest of 3,000 1.2e-5).
 template <bool PERT, bool XF32 = false>
 __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
     __shared__ __attribute__((aligned(16))) char lds[2 * kH3Step];
