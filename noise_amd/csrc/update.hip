@@ -20,6 +20,7 @@
 
 #include "common.hpp"
 #include "philox.hpp"
+#include "slice_copy.hpp"
 #include "tile.hpp"
 
 namespace noise {
@@ -140,7 +141,7 @@ struct UpdateRaw {
     int64_t d0, n;             // the chunk's first direction and its directions (zeros fill the last stage)
     const float *weight;
     float scale;
-    const float *buf;          // fp32 [numel], numel <= 2^30 (lane offsets are 32-bit byte offsets); NULL: the slabs
+    const float *buf;          // fp32 [numel]; NULL: the slabs
     int64_t numel;
 };
 constexpr int kUgDirs = 16;          // directions per stage
@@ -218,7 +219,13 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accum
     // leaves the buffer
     float wt[3][2] = {};  // of stages ks + 1 .. ks + 3
     unsigned slow = 0;
-    auto offset = [&](int64_t k) { return raw.buf ? s.offsets[p][raw.d0 + k] : k * (rows + cols); };
+    // (wave-uniform, and read out of its vector registers here: a load left to its first use in the slow branch makes
+    // the compiler wait for every copy in flight where the branches meet, 31.0 -> 36.3 ms for 131,072 pairs)
+    auto offset = [&](int64_t k) {
+        const int64_t o = raw.buf ? s.offsets[p][raw.d0 + k] : k * (rows + cols);
+        return (int64_t)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(o >> 32)) << 32) |
+                         (unsigned)__builtin_amdgcn_readfirstlane((int)o));
+    };
     auto issue = [&](int ks, float (&w)[2]) {
         const int slot = ks & (kUgRing - 1), at = 2 * (ks & 31);
         const unsigned st = lbase + slot * kSt + dir0 * kUgDir;
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accum
                              st + 2 * i * kUgDir + 1024);
             }
         } else {
-            // 4 B copies with every lane's element clamped into the buffer (a padding direction reads element 0)
+            // 4 B copies with every lane's element clamped into the buffer (a padding direction reads from element 0)
             slow |= 1u << slot;
 #pragma unroll 1
             for (int i = 0; i < 2; ++i) {
@@ -242,9 +249,9 @@ __global__ __launch_bounds__(512) void update_gemm_kernel(UpdateSet s, int accum
                 const int64_t o = k < raw.n ? offset(k) : 0;
 #pragma unroll 1
                 for (int q = 0; q < 8; ++q) {
-                    int64_t L = k < raw.n ? o + (q >= 4 ? side1 : side0) + 64 * (q & 3) + lane : 0;
-                    L = L < 0 ? 0 : (L < numel ? L : numel - 1);
-                    lds_dma4_at(buf, (unsigned)(4 * L), st + 2 * i * kUgDir + 256 * q);
+                    const int64_t first = k < raw.n ? o + (q >= 4 ? side1 : side0) + 64 * (q & 3) : 0;
+                    const int64_t base = slice_base(first, numel);
+                    lds_dma4_at(buf + base, slice_lane(first, lane, base, numel), st + 2 * i * kUgDir + 256 * q);
                 }
             }
 #pragma unroll

@@ -44,3 +44,30 @@ def test_long_chunks(pairs):
     assert torch.equal(nan, torch.isnan(g_regen['q']))
     assert torch.equal(torch.nan_to_num(g_buf['q'], nan=0.0), torch.nan_to_num(g_regen['q'], nan=0.0))
     assert nan[:40].all() and not nan[40:, :188].any()
+
+
+def test_a_slab_of_more_than_2_to_the_30_elements():
+    """The last direction of a chunk whose regenerated slices pass 4 GiB, alone in its stage: its copies' byte offsets
+    do not fit 32 bits. Its weight outweighs the others', so that another direction's slice in its place shows."""
+    from noise_amd.eggroll import Eggroll
+    pairs, rows, cols = 16385, 65280, 256
+    assert (pairs - 1) * (rows + cols) == 2 ** 30 and pairs % 16 == 1
+    p = torch.nn.Module()
+    p.wide = torch.nn.Parameter(torch.zeros(rows, cols))
+    es = Eggroll(p.cuda(), pairs)
+    offsets = es.offsets(3)
+    losses = torch.randn(2 * pairs, device='cuda', generator=torch.Generator('cuda').manual_seed(1))
+    losses[-1] += 1e4
+    one = es.update(losses, offsets, chunk=pairs, materialise=False)['wide']
+    three = es.update(losses, offsets, chunk=8192, materialise=False)['wide']
+    score = (losses[1::2] - losses[0::2]).double()
+    w = (score / (score.std() + 1e-8)) / pairs
+    pick = torch.tensor([0, 1, 255, 256, 40000, rows - 1], device='cuda')
+    d = torch.arange(pairs, device='cuda')
+    a = torch.cat([es.buffer.gather(offsets['wide'] + r, 1, rows=d) for r in pick.tolist()], 1).double()
+    b = es.buffer.gather(offsets['wide'] + rows, cols, rows=d).double()
+    ref = -(a * w[:, None]).T.contiguous() @ b
+    mag = (a * w[:, None]).abs().T.contiguous() @ b.abs()
+    bound = (3 * 2.0 ** -16 + 3 * pairs * 2.0 ** -24 + 2.0 ** -21) * mag
+    for g in (one, three):
+        assert ((g[pick].double() - ref).abs() <= bound).all()
