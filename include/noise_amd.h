@@ -356,8 +356,7 @@ int noise_pop_block_qkv(const noise_population_t *pop, noise_view_t y, const voi
 
 /* DUST's jitter on a population block (block_forward, run.py:102-117, for the block a rerun enters at): bf16 rows
  * [members * tokens][2048] added to mlp.c_fc's product before ReLU^2 (fc) and [members * tokens][512] added to
- * mlp.c_proj's product (mlp), either may be NULL (not both); without mlp rows, zero_row is 512 zero bf16 values
- * (16 B aligned) the kernel reads instead. The attention-output and attn.c_proj jitter go in before the call
+ * mlp.c_proj's product (mlp), either may be NULL (not both); zero_row is no longer read and may be NULL. The attention-output and attn.c_proj jitter go in before the call
  * (noise_add_bf16 on y, noise_block_entry's residual). */
 typedef struct {
     const void *fc;

@@ -147,7 +147,7 @@ class CastHeads(ctypes.Structure):
 
 
 class BlockJitter(ctypes.Structure):
-    """noise_block_jitter_t: bf16 jitter rows added to mlp.c_fc's and mlp.c_proj's products (NULL: none)."""
+    """noise_block_jitter_t: bf16 jitter rows added to mlp.c_fc's and mlp.c_proj's products (NULL: none); zero_row is not read."""
     _fields_ = [('fc', ctypes.c_void_p), ('mlp', ctypes.c_void_p), ('zero_row', ctypes.c_void_p)]
 
 

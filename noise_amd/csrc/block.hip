@@ -104,9 +104,13 @@ struct BlockArgs {
     float *ndots;                          // [rows][NNEXT]
     QkvRowsArgs q;                         // the next block's q/k/v (QKV): its x is h, its dots come from the epilogue
     const __bf16 *jfc;                     // JIT: mlp.c_fc jitter bf16 [m * T][2048] (added before ReLU^2) or NULL
-    const __bf16 *jmlp;                    // JIT: mlp.c_proj jitter bf16, row r at r * jmlp_st (added to its product)
-    int64_t jmlp_st;                       //   512, or 0 with one zero row when the block has no mlp.c_proj jitter
+    const __bf16 *jmlp;                    // JIT: mlp.c_proj jitter bf16 [m * T][512] (added to its product) or NULL
 };
+
+// The row a jittered block without mlp.c_proj jitter reads: zeros of the library's own image, never written and in place
+// on every device before any stream runs. (Loads under a condition instead made the jittered kernels spill 97 to 106
+// registers; this way they keep their 241 to 256 and spill none.)
+__device__ __attribute__((aligned(16))) __bf16 kNoJitter[kModel];
 
 // sum over the four lanes holding one token's features (l % 16 + 16 g)
 __device__ __forceinline__ float token_sum(float v) { return sum_lanes_16_32(v); }
@@ -431,7 +435,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void block_kernel(BlockArgs p) {
     {
         const float *apj = reinterpret_cast<const float *>(lds + kVApj) + 4 * g;
         const float *zr = MIX ? p.x0 + m * p.x0_m + (int64_t)tok * p.x0_t + 4 * g : nullptr;
-        const __bf16 *jr = kJit ? p.jmlp + row * p.jmlp_st + 4 * g : nullptr;
+        const __bf16 *jr = kJit ? (p.jmlp ? p.jmlp + row * kModel : kNoJitter) + 4 * g : nullptr;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             float4 zv[8];
@@ -720,15 +724,7 @@ int block_jitter(const char *fn, BlockArgs &a, const noise_block_jitter_t *jit) 
                     "%s: a jittered block takes no rank-1 or mixing-scalar noise", fn);
     NOISE_CHECK_ARG((!jit->fc || aligned(jit->fc, 16)) && (!jit->mlp || aligned(jit->mlp, 16)),
                     "%s: jitter rows must be 16 B aligned", fn);
-    // no mlp.c_proj jitter: every row reads one zero row (the kernel's epilogue loads unconditionally)
     a.jmlp = (const __bf16 *)jit->mlp;
-    a.jmlp_st = kModel;
-    if (!a.jmlp) {
-        NOISE_CHECK_ARG(jit->zero_row && aligned(jit->zero_row, 16), "%s: without mlp jitter a 512-element zero row "
-                        "(bf16, 16 B aligned) must be given", fn);
-        a.jmlp = (const __bf16 *)jit->zero_row;
-        a.jmlp_st = 0;
-    }
     a.jfc = (const __bf16 *)jit->fc;   // each workgroup copies only its own token rows of it
     return NOISE_OK;
 }

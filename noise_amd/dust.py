@@ -105,7 +105,7 @@ def block_forward_eager(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, 
     Returns x_out fp32 [B, T, 512]: bf16 products with fp32 accumulation, bf16 attention, fp32 residual stream, as the
     reference's autocast. Four launches on the population kernels, one sequence per member: the weights' bf16 copies,
     norm with gates and q/k/v, attention, and the rest of the block (with few sequences shared out over the CUs)."""
-    from .eggroll import _split_workspace, _zero_row_bf16
+    from .eggroll import _split_workspace
     dev = x.device
     B, T, C = x.shape
     if C != 512 or T % 256:
@@ -160,7 +160,7 @@ def block_forward_eager(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, 
         _lib.call('noise_add_bf16', y.data_ptr(), o.data_ptr(), y.numel(), stream)
     js = None
     if fc is not None or mlp is not None:
-        js = ctypes.byref(_lib.BlockJitter(_lib.ptr(fc), _lib.ptr(mlp), _zero_row_bf16(dev).data_ptr()))
+        js = ctypes.byref(_lib.BlockJitter(_lib.ptr(fc), _lib.ptr(mlp), None))
     split = _split_workspace(B, T, dev)
     _lib.call('noise_block_tail', pop, _lib.View(y.data_ptr(), T * C, C), ws['proj'].data_ptr(),
               _lib.View(xs.data_ptr(), T * C, C), ws['fc'].data_ptr(), ws['out'].data_ptr(), out.data_ptr(), js,

@@ -235,18 +235,6 @@ def _block(name, split, args, stream, jit=None, label='block'):
         _call(name + '_split', *args, jit, split.data_ptr(), split.numel(), stream, label=label)
 
 
-_ZERO_ROWS = {}
-
-
-def _zero_b(dev, width):
-    """A single zero row with stride 0: the b of an unperturbed matrix whose dot slot must still exist."""
-    key = (dev, width)
-    if key not in _ZERO_ROWS:
-        _ZERO_ROWS[key] = torch.zeros(width, dtype=F32, device=dev)
-    z = _ZERO_ROWS[key]
-    return _lib.Rank1(None, z.data_ptr(), 0, 0)
-
-
 def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffers=None, per_token=False,
                        rounding=_lib.ROUNDING_FUSED, fuse_qkv=True):
     """Per-member mean cross-entropy [m] of the perturbed models (eggroll.py:66-103 semantics).
@@ -316,16 +304,25 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
         pre = f'transformer.h.{i}.'
         return [nz(pre + 'attn.c_q.weight'), nz(pre + 'attn.c_k.weight'), nz(pre + 'attn.c_v.weight')]
 
-    def dot_vecs(pairs, width):
+    zero_b = None
+
+    def dot_vecs(pairs):
+        nonlocal zero_b
         arr = (_lib.Rank1 * len(pairs))()
         for k, pr in enumerate(pairs):
-            arr[k] = _rank1(pr) if pr is not None else _zero_b(dev, width)
+            if pr is None:
+                # an unperturbed matrix whose dot slot must still exist: one zero row, of this call's stream and kept to its end
+                if zero_b is None:
+                    zero_b = torch.zeros(E, dtype=F32, device=dev)
+                arr[k] = _lib.Rank1(None, zero_b.data_ptr(), 0, 0)
+            else:
+                arr[k] = _rank1(pr)
         return arr
 
     # q/k/v dots of block 0
     n0 = qkv_noise(0)
     if any(v is not None for v in n0):
-        _call('noise_member_dots', popp, _view(B.h0, sm_e, E), E, dot_vecs(n0, E), 3, B.d_qkv.data_ptr(), stream)
+        _call('noise_member_dots', popp, _view(B.h0, sm_e, E), E, dot_vecs(n0), 3, B.d_qkv.data_ptr(), stream)
 
     qkv_out = (ctypes.c_void_p * 3)(*(B.qkv[i].data_ptr() for i in range(3)))
     split = _split_workspace(m, T, dev) if fuse_qkv and rounding == _lib.ROUNDING_FUSED else None
@@ -384,12 +381,12 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
                 nn = qkv_noise(i + 1)
                 if not fuse_qkv:
                     want = any(v is not None for v in nn)
-                    nxt, nnext, ndots = (dot_vecs(nn, E), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
+                    nxt, nnext, ndots = (dot_vecs(nn), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
                     hout, split3 = B.h, 0
                 mixargs = (1, W.lam_r(i + 1), W.lam_x(i + 1), eps_ptr(eps_r, i + 1), eps_ptr(eps_x, i + 1), eps_stride)
             else:
                 nh = nz('lm_head.weight')
-                nxt, nnext, ndots = (dot_vecs([nh], E), 1, B.d_head.data_ptr()) if nh is not None else (None, 0, None)
+                nxt, nnext, ndots = (dot_vecs([nh]), 1, B.d_head.data_ptr()) if nh is not None else (None, 0, None)
                 hout, split3 = (B.h3, 1) if W.fp32_head else (B.h, 0)
                 mixargs = (0, None, None, None, None, 0)
             if not last and fuse_qkv:
@@ -428,14 +425,14 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
         if not last:
             nn = qkv_noise(i + 1)
             want = any(v is not None for v in nn)
-            nxt, nnext, ndots = (dot_vecs(nn, E), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
+            nxt, nnext, ndots = (dot_vecs(nn), 3, B.d_qkv.data_ptr()) if want else (None, 0, None)
             _call('noise_pop_residual', popp, _view(B.act, T * 4 * E, 4 * E), blk['mp'].data_ptr(), 4 * E,
                   ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, resid_view, B.resid.data_ptr(),
                   1, W.lam_r(i + 1), W.lam_x(i + 1), eps_ptr(eps_r, i + 1), eps_ptr(eps_x, i + 1),
                   eps_stride, x0_view, B.h.data_ptr(), 0, nxt, nnext, ndots, stream, label='mlp.c_proj')
         else:
             nh = nz('lm_head.weight')
-            nxt, nnext, ndots = (dot_vecs([nh], E), 1, B.d_head.data_ptr()) if nh is not None else (None, 0, None)
+            nxt, nnext, ndots = (dot_vecs([nh]), 1, B.d_head.data_ptr()) if nh is not None else (None, 0, None)
             hout = B.h3 if W.fp32_head else B.h
             _call('noise_pop_residual', popp, _view(B.act, T * 4 * E, 4 * E), blk['mp'].data_ptr(), 4 * E,
                   ctypes.byref(mp_r1), B.d_mp.data_ptr(), 16, 16, resid_view, None, 0, None, None,
@@ -453,16 +450,6 @@ def population_forward(W, noise, sign, idx, targets, dir_div=1, rope=None, buffe
     out = torch.empty(m, dtype=F32, device=dev)
     _call('noise_member_mean', B.loss_tok.data_ptr(), m, T, out.data_ptr(), stream)
     return out
-
-
-_ZERO_BF16 = {}
-
-
-def _zero_row_bf16(dev):
-    """512 zero bf16 values on dev (the mlp.c_proj jitter row a jittered block reads when it has none)."""
-    if dev not in _ZERO_BF16:
-        _ZERO_BF16[dev] = torch.zeros(N_EMBD, dtype=BF16, device=dev)
-    return _ZERO_BF16[dev]
 
 
 def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=None, jitter=None):
@@ -538,8 +525,7 @@ def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=No
             if 'o' in jit:
                 _call('noise_add_bf16', B.y.data_ptr(), jit['o'].data_ptr(), B.y.numel(), stream)
             if 'fc' in jit or 'mlp' in jit:
-                js = _lib.BlockJitter(_lib.ptr(jit.get('fc')), _lib.ptr(jit.get('mlp')),
-                                      _zero_row_bf16(dev).data_ptr())
+                js = _lib.BlockJitter(_lib.ptr(jit.get('fc')), _lib.ptr(jit.get('mlp')), None)
         yv, wo, wfc, wmp = _view(B.y, T * E, E), blk['o'].data_ptr(), blk['fc_blk'].data_ptr(), blk['mp_blk'].data_ptr()
         plain = (popp, yv, wo, ctypes.byref(none), B.d_attn.data_ptr(), N_HEAD, xres, wfc, ctypes.byref(none), wmp,
                  ctypes.byref(none))

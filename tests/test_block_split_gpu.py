@@ -154,3 +154,73 @@ def test_block_forward_against_the_tiled_kernels(B, T, layer, site):
     rel = float((got - ref).norm() / (ref - x).norm())
     print(B, T, layer, site, rel, flush=True)
     assert rel <= 4.8e-3
+
+
+def _block_inputs(B, T, seed):
+    g = torch.Generator(DEV).manual_seed(seed)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    w = dict(q=r(512, 512) * .044, k=r(512, 512) * .044, v=r(512, 512) * .044, proj=r(512, 512) * .044,
+             fc=r(2048, 512) * .044, out=r(512, 2048) * .022, gate=None)
+    return r(B, T, 512), w, (r(B, T, 2048) * .1).bfloat16()
+
+
+@pytest.mark.parametrize('B,T', [(1, 256), (49, 256)])
+def test_c_fc_jitter_alone_is_the_one_with_zero_rows(B, T):
+    """Without mlp.c_proj jitter the block adds zeros of its own, in the split and in the one-launch form: the bits of
+    jitter rows that hold zeros, +0 and -0 products included."""
+    from noise_amd.dust import block_forward
+    from noise_amd.model import rotary_tables
+    x, w, fc = _block_inputs(B, T, B)
+    w['out'][::2] = 0
+    x[..., ::3] = -0.0
+    cos, sin = (t.to(DEV) for t in rotary_tables(T))
+    got = block_forward(x, w, None, cos, sin, 128, fc=fc)
+    ref = block_forward(x, w, None, cos, sin, 128, fc=fc, mlp=torch.zeros(B, T, 512, dtype=torch.bfloat16, device=DEV))
+    assert torch.equal(_bits(got), _bits(ref))
+
+
+def test_jitter_on_two_streams():
+    """A call whose stream is far behind holds nothing that a call on another stream reads: results are the same bits."""
+    from noise_amd.dust import block_forward
+    from noise_amd.model import rotary_tables
+    x, w, fc = _block_inputs(50, 256, 3)
+    cos, sin = (t.to(DEV) for t in rotary_tables(256))
+    behind, ahead = torch.cuda.Stream(DEV), torch.cuda.Stream(DEV)
+    torch.full((1 << 22,), float('nan'), device=DEV)   # blocks freed here and taken again hold no zeros
+    torch.cuda.synchronize()
+    outs = []
+    for stream in (behind, ahead):
+        with torch.cuda.stream(stream):
+            torch.full((1 << 16,), float('nan'), device=DEV)
+            if stream is behind:
+                torch.cuda._sleep(20_000_000)
+            outs.append(block_forward(x, w, None, cos, sin, 128, fc=fc))
+    torch.cuda.synchronize()
+    ref = block_forward(x, w, None, cos, sin, 128, fc=fc)
+    for out in outs:
+        assert torch.equal(_bits(out), _bits(ref))
+
+
+@pytest.mark.parametrize('fuse_qkv', [True, False])
+def test_one_perturbed_matrix_of_q_k_and_v(fuse_qkv):
+    """The dot slots of unperturbed matrices beside a perturbed one hold dots with zeros of the call's own: losses are those
+    of rank-1 terms that are zero, on any stream."""
+    from noise_amd.eggroll import Eggroll, Weights, _pair_signs, population_forward
+    from noise_amd.model import make_model
+    model = make_model('cpu', 0).to(DEV)
+    model.lm_head.weight.mul_(30)
+    es = Eggroll(model, 3)
+    tokens = torch.randint(0, 4096, (257,), device=DEV, generator=torch.Generator(DEV).manual_seed(0))
+    W, sign = Weights(es.params), _pair_signs(3, 0.02, DEV)
+    names = [f'transformer.h.{i}.attn.c_{x}.weight' for i in (0, 5) for x in 'kqv']
+    offsets = es.offsets(0)
+    noise = es.noise_tables({n: offsets[n] for n in names}, torch.arange(3, device=DEV))
+    forward = lambda n: population_forward(W, n, sign, tokens[:-1], tokens[1:], dir_div=2, fuse_qkv=fuse_qkv)
+    ref = forward({n: v if '.c_k.' in n else (torch.zeros_like(v[0]), v[1]) for n, v in noise.items()})
+    alone = {n: v for n, v in noise.items() if '.c_k.' in n}
+    assert torch.equal(forward(alone), ref)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream(DEV)):
+        other = forward(alone)
+    torch.cuda.synchronize()
+    assert torch.equal(other, ref)
