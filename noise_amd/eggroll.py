@@ -68,7 +68,8 @@ def _rope_tables(T, dev):
     key = (T, dev.type, dev.index)
     if key not in _ROPE:
         cos, sin = rotary_tables(T)
-        _ROPE[key] = (cos.to(dev).bfloat16().contiguous(), sin.to(dev).bfloat16().contiguous())
+        # rounded on the host: the copies are complete when .to returns, so other streams may read them
+        _ROPE[key] = (cos.bfloat16().to(dev), sin.bfloat16().to(dev))
     return _ROPE[key]
 
 

@@ -81,3 +81,16 @@ def test_noise_tables_are_the_noise():
     for n, v in ref.items():
         for a, b in zip(v if isinstance(v, tuple) else (v,), tables[n] if isinstance(v, tuple) else (tables[n],)):
             assert torch.equal(a, b), n
+
+
+def test_rotary_tables_are_complete_when_cached():
+    """The rotary tables are shared by every stream: nothing that fills them is left on the first caller's stream."""
+    from noise_amd.eggroll import _rope_tables
+    from noise_amd.model import rotary_tables
+    stream = torch.cuda.Stream(DEV)
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(2_000_000)
+        cos, sin = _rope_tables(1003, DEV)   # (no other test's length)
+        assert stream.query()
+    for got, ref in zip((cos, sin), rotary_tables(1003)):
+        assert got.dtype == torch.bfloat16 and got.is_contiguous() and torch.equal(got.cpu(), ref.bfloat16())
