@@ -59,8 +59,13 @@ struct OperandArgs {
     __bf16 *xb, *wb;          // [rows][kp] (NULL: x is used as it is), [n_out + b_rows][kp]
     float *dots;              // [rows] x . bf16(b[dir]), or NULL
     int x_fp32, w_fp32, x_vec, w_vec, b_vec;
-    int64_t x_blocks;
+    int64_t x_blocks;         // workgroups of x's rows
+    int64_t first;            // this launch's first workgroup
 };
+
+// A launch has fewer than 2^32 threads (one of more is cut short without an error): a call of more workgroups than this
+// goes in several launches.
+constexpr int64_t kLaunchGroups = 1 << 23;
 
 // One wave per row: x rows first, then W's, then b's. Reads each tensor once and writes its bf16 form once;
 // bound by those bytes (24,000 x 512 fp32: 49 MB in, 25 MB out).
@@ -71,8 +76,9 @@ __global__ __launch_bounds__(256) void lowrank_operands_kernel(OperandArgs p) {
     const float *br = nullptr;
     float *dot = nullptr;
     bool fp32, vec;
-    if (blockIdx.x < p.x_blocks) {
-        const int64_t r = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t block = p.first + blockIdx.x;
+    if (block < p.x_blocks) {
+        const int64_t r = block * 4 + wave;
         if (r >= p.rows) return;
         const int64_t m = r / p.tokens, t = r - m * p.tokens;
         fp32 = p.x_fp32;
@@ -84,7 +90,7 @@ __global__ __launch_bounds__(256) void lowrank_operands_kernel(OperandArgs p) {
             dot = p.dots + r;
         }
     } else {
-        const int64_t r = ((int64_t)blockIdx.x - p.x_blocks) * 4 + wave;
+        const int64_t r = (block - p.x_blocks) * 4 + wave;
         if (r >= p.n_out + p.b_rows) return;
         const bool is_w = r < p.n_out;
         fp32 = is_w ? p.w_fp32 : true;
@@ -221,6 +227,7 @@ struct NarrowArgs {
     int64_t a_stride, b_stride;
     const float *sign;
     float *y;
+    unsigned first;           // this launch's first tile
 };
 
 // 32 rows x 8 outputs per workgroup, eight lanes per row: each lane takes 4 of every 32 k for the eight products
@@ -230,8 +237,10 @@ constexpr int kNarrowK = 256;
 template <bool XF, bool WF>
 __global__ __launch_bounds__(256) void lowrank_narrow_kernel(NarrowArgs p) {
     __shared__ __attribute__((aligned(16))) float ws[8][kNarrowK];
-    const int tid = threadIdx.x, l = tid & 7, groups = (p.n_out + 7) / 8, o0 = (int)(blockIdx.x % groups) * 8;
-    const int64_t row = (int64_t)(blockIdx.x / groups) * 32 + (tid >> 3);
+    const int tid = threadIdx.x, l = tid & 7, groups = (p.n_out + 7) / 8;
+    const unsigned tile = p.first + blockIdx.x;
+    const int o0 = (int)(tile % groups) * 8;
+    const int64_t row = (int64_t)(tile / groups) * 32 + (tid >> 3);
     const bool live = row < p.rows;
     const int64_t m = live ? row / p.tokens : 0, t = live ? row - m * p.tokens : 0, dir = m / p.dir_div;
     const char *xr = static_cast<const char *>(p.x) + (m * p.xs_m + t * p.xs_t) * (XF ? 4 : 2);
@@ -312,12 +321,15 @@ int narrow_launch(const noise_population_t *pop, noise_view_t x, bool xf, int64_
     p.sign = pop->sign; p.y = y;
     const int64_t tiles = (p.rows + 31) / 32 * ((n_out + 7) / 8);
     NOISE_CHECK_ARG(tiles <= INT32_MAX, "%s: output too large", fn);
-    const dim3 grid((unsigned)tiles);
     hipStream_t st = (hipStream_t)stream;
-    if (xf && wf) hipLaunchKernelGGL((lowrank_narrow_kernel<true, true>), grid, dim3(256), 0, st, p);
-    else if (xf) hipLaunchKernelGGL((lowrank_narrow_kernel<true, false>), grid, dim3(256), 0, st, p);
-    else if (wf) hipLaunchKernelGGL((lowrank_narrow_kernel<false, true>), grid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((lowrank_narrow_kernel<false, false>), grid, dim3(256), 0, st, p);
+    for (int64_t first = 0; first < tiles; first += kLaunchGroups) {
+        const dim3 grid((unsigned)(tiles - first < kLaunchGroups ? tiles - first : kLaunchGroups));
+        p.first = (unsigned)first;
+        if (xf && wf) hipLaunchKernelGGL((lowrank_narrow_kernel<true, true>), grid, dim3(256), 0, st, p);
+        else if (xf) hipLaunchKernelGGL((lowrank_narrow_kernel<true, false>), grid, dim3(256), 0, st, p);
+        else if (wf) hipLaunchKernelGGL((lowrank_narrow_kernel<false, true>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((lowrank_narrow_kernel<false, false>), grid, dim3(256), 0, st, p);
+    }
     return launch_status(fn);
 }
 
@@ -361,9 +373,12 @@ extern "C" int noise_lowrank_operands(const noise_population_t *pop, noise_view_
     p.w_vec = rows_vec(w, w_fp32, n_in, 0, 0);
     p.b_vec = b && rows_vec(b, true, n_in, b_stride, 0);
     p.x_blocks = xb || dots ? (p.rows + 3) / 4 : 0;
-    const int64_t grid = p.x_blocks + (n_out + b_rows + 3) / 4;
-    NOISE_CHECK_ARG(grid <= INT32_MAX, "%s: too many rows", fn);
-    hipLaunchKernelGGL(lowrank_operands_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, p);
+    const int64_t blocks = p.x_blocks + (n_out + b_rows + 3) / 4;
+    NOISE_CHECK_ARG(blocks <= INT32_MAX, "%s: too many rows", fn);
+    for (p.first = 0; p.first < blocks; p.first += kLaunchGroups) {
+        const int64_t n = blocks - p.first < kLaunchGroups ? blocks - p.first : kLaunchGroups;
+        hipLaunchKernelGGL(lowrank_operands_kernel, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream, p);
+    }
     return launch_status(fn);
 }
 
@@ -396,7 +411,7 @@ extern "C" int noise_lowrank_product(const noise_population_t *pop, const void *
     const int64_t big = ((N + 255) / 256) * ((rows + 255) / 256);
     if (big >= 256) {
         p.tiles_n = (int)((N + 255) / 256);
-        NOISE_CHECK_ARG(big <= INT32_MAX, "%s: too many tiles", fn);
+        NOISE_CHECK_ARG(big < kLaunchGroups, "%s: too many tiles", fn);
         p.tiles_t = (int)((rows + 255) / 256);
         hipLaunchKernelGGL((lowrank_product_kernel<8, 256, 256>), dim3((unsigned)big), dim3(512), 0, st, p);
     } else {

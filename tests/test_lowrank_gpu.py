@@ -69,3 +69,15 @@ def test_lowrank_views():
     check(x, w.t().contiguous().t(), a.bfloat16(), b.half(), sign, 1)
     check(x.transpose(1, 2)[:1].expand(6, 512, 40), torch.randn(18, 40, device=DEV), torch.randn(6, 18, device=DEV),
           torch.randn(6, 40, device=DEV), sign, 1)             # shared, no unit inner stride, outputs off the groups of 4
+
+
+@pytest.mark.parametrize('m,n_in,n_out', [(65537, 32, 18), (2 ** 19 + 1, 32, 1), (2 ** 19 + 1, 8, 7)])
+def test_more_rows_than_one_launch_has_waves(m, n_in, n_out):
+    """1024 rows per member, past 2^26 rows for the operands' wave per row and 2^29 for the narrow form's eight lanes per row:
+    a launch has fewer than 2^32 threads. A member's rows are one row repeated, so its outputs are that row's."""
+    from noise_amd.eggroll import lowrank
+    print(m, n_in, n_out, flush=True)
+    x, w, a, b, sign = inputs(m, 1, n_in, n_out, 2, torch.bfloat16, n_out)
+    few = lowrank(x, w, a, b, sign, dir_div=2)
+    got = lowrank(x.expand(m, 1024, n_in), w, a, b, sign, dir_div=2)
+    assert torch.equal(got[:, 0], few[:, 0]) and torch.equal(got.amin(1), few[:, 0]) and torch.equal(got.amax(1), few[:, 0])
