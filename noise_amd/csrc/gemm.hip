@@ -1075,6 +1075,9 @@ constexpr int kH3Step = 2 * kH3Part;          // hi then lo
 // XF32: x is fp32 [T][512], its rows split here, their norm applied to the logits (the head_loss drop-in, unperturbed).
 // Normalising first reads x twice: 67 us against 53 for 3,000 rows. The errors against 64 bits are the same either way
 // (120,000 rows: rms 3.11e-6, largest of 3,000 1.2e-5).
+// Raw values enter the products times 2^-60, exactly: finite rows whose squares pass fp32 norm to zeros (scale 0), and
+// their products, unlike inf * 0, must stay finite for that. A lo half is exact down to values of 1e-15.
+constexpr float kRawScale = 0x1p-60f;
 template <bool PERT, bool XF32 = false>
 __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
     __shared__ __attribute__((aligned(16))) char lds[2 * kH3Step];
@@ -1120,12 +1123,13 @@ __global__ __launch_bounds__(kH3Threads, 1) void head3_kernel(HeadArgs p) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float f = e < 4 ? f4get(u, e) : f4get(v, e - 4);
+                const float s = f * kRawScale;
                 ss += f * f;
-                xh[kb][e] = (__bf16)f;
-                xl[kb][e] = (__bf16)(f - (float)xh[kb][e]);
+                xh[kb][e] = (__bf16)s;
+                xl[kb][e] = (__bf16)(s - (float)xh[kb][e]);
             }
         }
-        scale = rsqrtf(sum_lanes_16_32(ss) * (1.0f / 512.0f) + kEps);
+        scale = rsqrtf(sum_lanes_16_32(ss) * (1.0f / 512.0f) + kEps) * (1.0f / kRawScale);
     } else {
         const __bf16 *xr = p.x + m * p.xs_m + (int64_t)tok * p.xs_t + 8 * g;
 #pragma unroll

@@ -2,6 +2,7 @@
 and off the tiles (the last tile ragged) and with every kernel that serves it. The sums of 128
 vocabulary rows are added in order whoever forms them, so a split loss has the unsplit one's bits."""
 import ctypes
+import math
 
 import pytest
 import torch
@@ -74,3 +75,25 @@ def test_split_equals_unsplit(K, m, T, pert, eager):
     assert (m * T > 100000) == (need == 0) or need > 0
     assert torch.equal(out[0].isnan(), out[1].isnan())
     assert torch.equal(out[0].nan_to_num(), out[1].nan_to_num())
+
+
+@pytest.mark.parametrize('rows', [40, 33000])
+def test_rows_whose_squares_overflow(rows):
+    """Finite rows whose sum of squares passes fp32 norm to zeros (x rsqrt(inf), utils/model.py:46-47 in fp32), whatever
+    their products with the weights come to; an infinity or a NaN among the values makes the loss NaN."""
+    from noise_amd.dust import head_loss
+    g = torch.Generator(DEV).manual_seed(rows)
+    x, w = torch.randn(rows, 512, device=DEV, generator=g), torch.randn(4096, 512, device=DEV, generator=g)
+    y = torch.randint(0, 4096, (rows,), device=DEV, generator=g)
+    plain = head_loss(x, w, y, 4096)
+    big = torch.finfo(torch.float32).max
+    x[3], x[7], x[17], x[21] = big, 1e30 * x[7], -big * torch.rand(512, device=DEV, generator=g), 3e19 * x[21]
+    x[5, 9], x[6, 1] = float('inf'), float('nan')
+    x[8, 500] = big
+    got = head_loss(x, w, y, 4096)
+    zeros, bad = [3, 7, 17, 21, 8], [5, 6]
+    assert ((got[zeros] - math.log(4096)).abs() <= 1e-5).all()
+    assert got[bad].isnan().all()
+    keep = torch.ones(rows, dtype=torch.bool, device=DEV)
+    keep[zeros + bad] = False
+    assert torch.equal(got[keep], plain[keep])
