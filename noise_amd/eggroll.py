@@ -20,7 +20,7 @@ import torch
 from . import _lib
 from ._lib import ATTN_QK_NORMED, ATTN_V_TRANSPOSED
 from .model import rotary_tables, window_sizes, has_ve, N_EMBD, N_HEAD, HEAD_DIM, VOCAB
-from .noise import DeviceGenerator, OrthogonalDraws
+from .noise import GATHER_ROWS, DeviceGenerator, OrthogonalDraws
 
 BF16 = torch.bfloat16
 F32 = torch.float32
@@ -760,6 +760,14 @@ class Eggroll:
         names = list(offsets)
         widths = [-(-sum(self.params[n].shape) // 256) * 256 for n in names]
         if not names:
+            return out
+        if directions.numel() > GATHER_ROWS and not any(self.params[n].dim() == 2 and sum(self.params[n].shape) % 256 == 0
+                                                        for n in names):
+            # more directions than a launch for several parameters serves: one launch (or more) for each of the small ones
+            for n in names:
+                p = self.params[n]
+                rows = self.buffer.gather(offsets[n], sum(p.shape), rows=directions)
+                out[n] = tuple(rows.split(list(p.shape), dim=1)) if p.dim() == 2 else rows
             return out
         table = self.buffer.gather_many([offsets[n] for n in names], widths, directions)
         # every column view in one call: a, b (or eps) and the columns after a narrower slice

@@ -13,6 +13,8 @@ import torch
 
 from . import _lib
 
+GATHER_ROWS = 65535  # rows of one gather launch (a grid's second dimension)
+
 
 def draw_layout(numel, device=None):
     """(threads, offset increment) of a torch draw of `numel` values on `device`."""
@@ -50,8 +52,8 @@ class Draw:
             rows = rows.to(device=self.device, dtype=torch.int64).contiguous()
         nrows = offsets.numel() if rows is None else rows.numel()
         out = torch.empty(nrows, width, device=self.device, dtype=torch.float32)
-        for start in range(0, nrows, 65535):
-            n = min(65535, nrows - start)
+        for start in range(0, nrows, GATHER_ROWS):
+            n = min(GATHER_ROWS, nrows - start)
             sub_rows = None if rows is None else rows[start:start + n]
             sub_offsets = offsets[start:start + n] if rows is None else offsets
             _lib.call('noise_gather_slices', _lib.ptr(out[start:start + n]), n, width, _lib.ptr(sub_offsets),
@@ -66,8 +68,8 @@ class Draw:
         of 256."""
         rows = rows.to(device=self.device, dtype=torch.int64).contiguous()
         nrows = rows.numel()
-        if nrows > 65535:
-            raise ValueError('gather_many: at most 65535 rows per call')
+        if nrows > GATHER_ROWS:
+            raise ValueError(f'gather_many: at most {GATHER_ROWS} rows per call')
         offsets = [o if o.dtype == torch.int64 and o.device == self.device and o.is_contiguous() else
                    o.to(device=self.device, dtype=torch.int64).contiguous() for o in offsets]
         total = int(sum(widths))

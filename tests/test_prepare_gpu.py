@@ -94,3 +94,19 @@ def test_rotary_tables_are_complete_when_cached():
         assert stream.query()
     for got, ref in zip((cos, sin), rotary_tables(1003)):
         assert got.dtype == torch.bfloat16 and got.is_contiguous() and torch.equal(got.cpu(), ref.bfloat16())
+
+
+def test_small_parameters_of_any_number_of_directions():
+    """Parameters whose slices are no whole 256s are gathered for more directions than one launch of the table serves."""
+    from noise_amd.eggroll import Eggroll
+    pairs = 65536 + 70
+    p = torch.nn.Module()
+    p.lam, p.gate, p.mat = (torch.nn.Parameter(torch.zeros(*s)) for s in ((8,), (8, 32), (256, 256)))
+    es = Eggroll(p.to(DEV), pairs)
+    offsets = es.offsets(1)
+    directions = torch.arange(pairs, device=DEV).flip(0)
+    small = {n: offsets[n] for n in ('lam', 'gate')}
+    tables, ref = es.noise_tables(small, directions), es.noise(small, directions)
+    assert torch.equal(tables['lam'], ref['lam']) and all(torch.equal(a, b) for a, b in zip(tables['gate'], ref['gate']))
+    with pytest.raises(ValueError, match='65535'):
+        es.noise_tables(offsets, directions)
