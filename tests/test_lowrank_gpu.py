@@ -81,3 +81,20 @@ def test_more_rows_than_one_launch_has_waves(m, n_in, n_out):
     few = lowrank(x, w, a, b, sign, dir_div=2)
     got = lowrank(x.expand(m, 1024, n_in), w, a, b, sign, dir_div=2)
     assert torch.equal(got[:, 0], few[:, 0]) and torch.equal(got.amin(1), few[:, 0]) and torch.equal(got.amax(1), few[:, 0])
+
+
+@pytest.mark.parametrize('n_in,n_out', [(512, 18), (1024, 1), (64, 131)])
+def test_shared_rows_are_not_copied_per_member(n_in, n_out):
+    """x broadcast over the members: the scratch memory stays within the outputs' size in whole groups of 4 twice over, and
+    the shared rows' and weights' own."""
+    from noise_amd.eggroll import lowrank
+    m, T = 256, 1024
+    x, w, a, b, sign = inputs(1, T, n_in, n_out, 1, torch.bfloat16, 5)
+    a, b, sign = (torch.randn(m, n, device=DEV) for n in (n_out, n_in, 1))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = lowrank(x.expand(m, T, n_in), w, a, b, sign[:, 0], dir_div=1)
+    used = torch.cuda.max_memory_allocated() - before
+    assert used <= 8 * m * T * -(-n_out // 4) * 4 + 16 * T * (n_in + n_out + m) + (64 << 20)
+    check(x.expand(m, T, n_in), w, a, b, sign[:, 0], 1)

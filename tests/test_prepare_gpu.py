@@ -106,7 +106,7 @@ def test_small_parameters_of_any_number_of_directions():
     offsets = es.offsets(1)
     directions = torch.arange(pairs, device=DEV).flip(0)
     small = {n: offsets[n] for n in ('lam', 'gate')}
-    tables, ref = es.noise_tables(small, directions), es.noise(small, directions)
+    tables, ref = es.noise_tables(small, directions), es.noise(offsets, directions)
     assert torch.equal(tables['lam'], ref['lam']) and all(torch.equal(a, b) for a, b in zip(tables['gate'], ref['gate']))
     with pytest.raises(ValueError, match='65535'):
         es.noise_tables(offsets, directions)
