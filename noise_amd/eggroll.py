@@ -640,12 +640,21 @@ def lowrank_eager(x, weight, a, b, sign, dir_div=1):
         xb = xb.to(BF16)
     if xb.stride(-1) != 1:
         xb = xb.contiguous()
+    narrow = n_out <= 16 and n_in <= 256 or n_in > 1 << 21
+    kp = -(-n_in // 64) * 64
+    if shared and n_out % 4 and not narrow and 2 * m * T * kp > 64 << 20:
+        # the expansion writes whole groups of 4 outputs: up to three more of zero weights, cut off again, instead of more than
+        # 64 MiB of bf16 copies of the shared rows, one per member (65 x 1024 rows of 512 -> 18: 63 us against 80; 8 MiB of
+        # copies, 64 x 1000 rows of 64 -> 131: 71 against 54, the pads' launches)
+        more = -n_out % 4
+        w, a = (torch.nn.functional.pad(t, p) for t, p in ((w, (0, 0, 0, more)), (a, (0, more))))
+        return lowrank_eager(x, w, a, b, sign, dir_div)[..., :n_out].contiguous()
     stream = _lib.stream_ptr(dev)
     pop = _pop(m, T, sign, dir_div)
     x_fp32, w_fp32 = int(xb.dtype == F32), int(w.dtype == F32)
     xv = _lib.View(xb.data_ptr(), 0 if shared else xb.stride(0), xb.stride(1))
     y = torch.empty(m, T, n_out, dtype=F32, device=dev)
-    if n_out <= 16 and n_in <= 256 or n_in > 1 << 21:
+    if narrow:
         # one launch: two (operands, product) cost more than the products of so few outputs (and the product's copies
         # address rows of up to 2^21 elements)
         r1 = _lib.Rank1(a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0))
@@ -659,7 +668,6 @@ def lowrank_eager(x, weight, a, b, sign, dir_div=1):
         one, rows, extra = _pop(1, T, None, 1), T, dirs
     else:
         one, rows, extra = pop, m * T, 0
-    kp = -(-n_in // 64) * 64
     flat = extra or m == 1 or (not shared and xb.stride(0) == T * xb.stride(1))
     direct = (not x_fp32 and kp == n_in and flat and xb.stride(1) % 8 == 0 and xb.stride(1) <= 1 << 21
               and xb.data_ptr() % 16 == 0)
