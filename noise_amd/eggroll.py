@@ -782,7 +782,7 @@ class Eggroll:
         sizes = []
         for n, w in zip(names, widths):
             shape = self.params[n].shape
-            sizes += [*shape, w - sum(shape)]
+            sizes += [*(shape if len(shape) == 2 else (sum(shape),)), w - sum(shape)]
         views = iter(table.split(sizes, dim=1))
         for n in names:
             out[n] = (next(views), next(views)) if self.params[n].dim() == 2 else next(views)

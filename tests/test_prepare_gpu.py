@@ -110,3 +110,15 @@ def test_small_parameters_of_any_number_of_directions():
     assert torch.equal(tables['lam'], ref['lam']) and all(torch.equal(a, b) for a, b in zip(tables['gate'], ref['gate']))
     with pytest.raises(ValueError, match='65535'):
         es.noise_tables(offsets, directions)
+
+
+def test_parameters_that_are_neither_vectors_nor_matrices():
+    """Their slice is one row per direction (eggroll.py:127-128), and the parameters after them keep their columns."""
+    from noise_amd.eggroll import Eggroll
+    p = torch.nn.Module()
+    p.cube, p.lam, p.mat = (torch.nn.Parameter(torch.zeros(*s)) for s in ((2, 3, 4), (8,), (8, 32)))
+    es = Eggroll(p.to(DEV), 5)
+    offsets, directions = es.offsets(0), torch.arange(5, device=DEV)
+    tables, ref = es.noise_tables(offsets, directions), es.noise(offsets, directions)
+    assert torch.equal(tables['cube'], ref['cube']) and torch.equal(tables['lam'], ref['lam'])
+    assert all(torch.equal(a, b) for a, b in zip(tables['mat'], ref['mat']))
