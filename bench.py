@@ -41,6 +41,7 @@ def visible_pairs(T, window):
 def kernel_flops_per_launch(name, label, members, T):
     """Algorithmic FLOPs one launch performs (dense products; rank-1 terms not counted)."""
     rows = members * T
+    name = name.removesuffix('_split')  # the same products, shared out over more workgroups
     if name == 'noise_pop_qkv':
         return 2 * 512 * 1536 * rows
     if name == 'noise_pop_fc':

@@ -18,3 +18,10 @@ def test_dominant_kernel_traffic_is_at_least_its_algorithmic_bytes():
     # the block kernel with the next q/k/v moves at least y (1 KiB) + the residual (2 KiB) in and the residual
     # (2 KiB) + q, k, v (3 KiB) out per member-token: 8 KiB x 1024 x 2048
     assert bench.profiled_traffic('noise_pop_block_qkv[block]') >= 8 * 1024 * 1024 * 2048
+
+
+def test_split_block_launches_count_as_the_blocks_they_are():
+    # up to 96 token tiles a block is noise_pop_block[_qkv]_split; without FLOPs it would drop out of the roofline's kernels
+    for name in ('noise_pop_block', 'noise_pop_block_qkv'):
+        flops = bench.kernel_flops_per_launch(name, 'block', 8, 256)
+        assert flops > 0 and bench.kernel_flops_per_launch(name + '_split', 'block', 8, 256) == flops
