@@ -65,7 +65,7 @@ def kernel_flops_per_launch(name, label, members, T):
 PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'profiles', 'population_forward_1024x2048.md')
 # entry point (bench label) -> the kernel name in the committed trace of the default workload (the block
 # kernels that form the next block's q/k/v: 4 of their 7 launches carry value embeddings)
-ROCPROF_NAME = {'noise_pop_qkv': 'qkv16_kernel<false>', 'noise_pop_head_ce': 'head_x_kernel<false, false>',
+ROCPROF_NAME = {'noise_pop_qkv': 'qkv16_kernel<false, false>', 'noise_pop_head_ce': 'head_x_kernel<false, false>',
                 'noise_pop_block_qkv[block]': 'block_kernel<true, 3, false, 2, 0>',
                 'noise_pop_block[block]': 'block_kernel<false, 0, false, 0, 0>'}
 
@@ -73,7 +73,7 @@ ROCPROF_NAME = {'noise_pop_qkv': 'qkv16_kernel<false>', 'noise_pop_head_ce': 'he
 def profiled_traffic(kernel):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 summary (FETCH_SIZE + WRITE_SIZE, scaled
     by the 1 GiB copy calibration), or None."""
-    name = ROCPROF_NAME.get(kernel) or ('attention_vt_kernel<true, false>' if kernel.startswith('noise_attention') else None)
+    name = ROCPROF_NAME.get(kernel) or ('attention_vt_kernel<true, false, false, false>' if kernel.startswith('noise_attention') else None)
     if not name or not os.path.exists(PROFILE):
         return None
     for line in open(PROFILE):
@@ -89,7 +89,7 @@ def profiled_traffic(kernel):
 def profiled_mfma_busy(kernel):
     """The kernel's MFMA-busy fraction from the committed counter table (SQ_VALU_MFMA_BUSY_CYCLES over the
     cycles it ran, on its own clock), or None."""
-    name = ROCPROF_NAME.get(kernel) or ('attention_vt_kernel<true, false>' if kernel.startswith('noise_attention') else None)
+    name = ROCPROF_NAME.get(kernel) or ('attention_vt_kernel<true, false, false, false>' if kernel.startswith('noise_attention') else None)
     if not name or not os.path.exists(PROFILE):
         return None
     col = None
