@@ -269,7 +269,7 @@ int noise_pop_fc(const noise_population_t *pop, noise_view_t x, const void *w, c
  * a[m / dir_div] (dots = x . b from noise_member_dots; r1 NULL or r1->a NULL: plain linear). bf16 x and
  * w [N][K]; y with strides ys_m, ys_t: bf16 (y_fp32 = 0), fp32 (1), or fp32 in autocast's form (2: the
  * product and the dot rounded to bf16 before the fp32 sum, as eggroll.py:58 runs under autocast).
- * N multiple of 256, K of 64. */
+ * N multiple of 256, K of 64. (The Python layer uses the plain fp32 product; its lowrank is noise_lowrank_*.) */
 int noise_pop_linear(const noise_population_t *pop, noise_view_t x, const void *w, int64_t K, int64_t N,
                      const noise_rank1_t *r1, const float *dots, void *y, int y_fp32, int64_t ys_m, int64_t ys_t,
                      noise_stream_t stream);
@@ -460,7 +460,7 @@ int noise_lowrank_embed(float *out, const float *w, int64_t vocab, int64_t width
  * (y_fp32 = 0) or fp32 (1; 2: the dot rounded to bf16 first, autocast's form) [m][T][width], base fp32
  * [T][width], width a multiple of 4. With x shared the dot x[t] . b depends on the direction only: dots
  * [T][dots_stride >= directions]. An HBM-write stream: the shared x W^T and x B^T are computed once
- * (noise_pop_linear). */
+ * (noise_lowrank_product). */
 int noise_rank1_expand(const noise_population_t *pop, const float *base, int64_t width, const float *dots,
                        int64_t dots_stride, const noise_rank1_t *r1, void *y, int y_fp32, noise_stream_t stream);
 
@@ -468,7 +468,8 @@ int noise_rank1_expand(const noise_population_t *pop, const float *base, int64_t
  * sign[m] * bf16(x[m, t, :] . bf16(b[m/dir_div, :])) * a[m/dir_div, o], fp32 accumulation, y fp32
  * [members][tokens][n_out]. x bf16 through the strided view (element (m, t, k) at x + m*sm + t*st + k),
  * w bf16 [n_out][n_in]. One launch with no workspace, on the vector units: for a few outputs, e.g. the
- * value-embedding gate linear('attn.ve_gate.weight', h[..., :32]) (eggroll.py:88 via :80). */
+ * value-embedding gate linear('attn.ve_gate.weight', h[..., :32]) (eggroll.py:88 via :80). The bf16 form of
+ * noise_lowrank_narrow, kept for its callers. */
 int noise_lowrank_rows(const noise_population_t *pop, noise_view_t x, int64_t n_in, const void *w, int64_t n_out,
                        const noise_rank1_t *r1, float *y, noise_stream_t stream);
 

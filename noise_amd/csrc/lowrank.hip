@@ -7,8 +7,8 @@
 //   narrow     a few outputs of a short contraction (the value-embedding gate's [8, 32] weight on h[..., :32],
 //              eggroll.py:88): one launch on the caller's tensors as they are
 //
-// The MFMA path replaced one thread per output element with a serial dot: 24 x 1000 rows, 512 -> 2048, fp32
-// inputs, 93.9 ms -> the figures at the kernels below.
+// 24 x 1000 rows, 512 -> 2048, fp32 inputs: 20 us for the operands and 94 for the product; one thread per output element
+// with a serial dot, which served this shape before, took 93.9 ms. 16 x 256 rows, 32 -> 8: the narrow kernel 4.1 us.
 #include "common.hpp"
 #include "mfma.hpp"
 #include "tile.hpp"

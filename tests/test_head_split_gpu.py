@@ -28,9 +28,10 @@ def _targets(rows, g):
 
 @pytest.mark.parametrize('rows', [1, 15, 16, 127, 128, 129, 300, 3000, 33000])
 def test_fp32_rows_against_64_bits(rows):
-    """The head_loss drop-in: fp32 rows split in the kernel, normed in the logits. A term h w of a logit loses at most 3 x 2^-18
-    of itself (lo lo, and the rounding of both lo halves), the loss takes at most two logits' errors, and the fp32
-    sums and the exponentials add 1e-5."""
+    """The head_loss drop-in: fp32 rows split in the kernel, normed in the logits. bf16 rounds by at most 2^-8 of a value, so a
+    term h w of a logit loses at most 3 x 2^-16 of itself (lo lo, and the rounding of both lo halves); the 512 terms' losses
+    have either sign, and a quarter of the sum of their bounds is allowed. The loss takes at most two logits' errors, and
+    the fp32 sums and the exponentials add 1e-5."""
     from noise_amd.dust import head_loss
     print(rows, flush=True)
     g = torch.Generator(DEV).manual_seed(rows)

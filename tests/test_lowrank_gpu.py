@@ -9,10 +9,10 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device('cuda', 0)
 
 
-def check(x, w, a, b, sign, div):
+def check(x, w, a, b, sign, div, got=None):
     from noise_amd.eggroll import lowrank
     m = x.shape[0]
-    got = lowrank(x, w, a, b, sign, dir_div=div)
+    got = lowrank(x, w, a, b, sign, dir_div=div) if got is None else got
     bf = lambda t: t.bfloat16().float()
     d = torch.arange(m, device=DEV) // div
     xr, wr, br, ar = bf(x), bf(w), bf(b)[d], a.float()[d]
@@ -98,3 +98,45 @@ def test_shared_rows_are_not_copied_per_member(n_in, n_out):
     used = torch.cuda.max_memory_allocated() - before
     assert used <= 8 * m * T * -(-n_out // 4) * 4 + 16 * T * (n_in + n_out + m) + (64 << 20)
     check(x.expand(m, T, n_in), w, a, b, sign[:, 0], 1)
+
+
+@pytest.mark.parametrize('m,T,n_in,n_out', [(3, 70, 32, 8), (2, 33, 300, 19)])
+def test_the_bf16_c_entry(m, T, n_in, n_out):
+    """noise_lowrank_rows is the drop-in's narrow form on bf16 tensors, at any number of outputs: held to the same bound."""
+    import ctypes
+    from noise_amd import _lib
+    x, w, a, b, sign = inputs(m, T, n_in, n_out, 2, torch.bfloat16, 7)
+    wb, y = w.bfloat16(), torch.empty(m, T, n_out, device=DEV)
+    pop = _lib.Population(m, T, sign.data_ptr(), 2)
+    r1 = _lib.Rank1(a.data_ptr(), b.data_ptr(), n_out, n_in)
+    _lib.call('noise_lowrank_rows', ctypes.byref(pop), _lib.View(x.data_ptr(), T * n_in, n_in), n_in, wb.data_ptr(), n_out,
+              ctypes.byref(r1), y.data_ptr(), _lib.stream_ptr(DEV))
+    check(x, wb, a, b, sign, 2, y)
+
+
+@pytest.mark.parametrize('form', [0, 1, 2])
+@pytest.mark.parametrize('K,N', [(512, 256), (192, 512)])
+def test_the_tiled_c_entry(form, K, N):
+    """noise_pop_linear with its rank-1 term, as bf16 (0), fp32 (1) and autocast's fp32 (2). The fp32 sum of the terms rounds
+    by 2^-20 of their sizes; form 0 rounds the result once more, and form 2 the product and the dot (one bf16 ulp each)."""
+    import ctypes
+    from noise_amd import _lib
+    m, T = 3, 512
+    x, w, a, b, sign = inputs(m, T, K, N, 2, torch.bfloat16, 9)
+    wb, bb = w.bfloat16(), b.bfloat16().float()
+    d = torch.arange(m, device=DEV) // 2
+    dots = (x.float() * bb[d][:, None, :]).sum(-1)
+    y = torch.empty(m, T, N, device=DEV, dtype=torch.bfloat16 if form == 0 else torch.float32)
+    pop = _lib.Population(m, T, sign.data_ptr(), 2)
+    r1 = _lib.Rank1(a.data_ptr(), bb.data_ptr(), N, K)
+    _lib.call('noise_pop_linear', ctypes.byref(pop), _lib.View(x.data_ptr(), T * K, K), wb.data_ptr(), K, N, ctypes.byref(r1),
+              dots.data_ptr(), y.data_ptr(), form, T * N, N, _lib.stream_ptr(DEV))
+    if form == 2:
+        check(x, wb, a, b, sign, 2, y)
+        return
+    xd, wd = x.double(), wb.double()
+    term = (sign[:, None] * dots).double()[..., None] * a.double()[d][:, None, :]
+    ref = torch.stack([xd[i] @ wd.t() for i in range(m)]) + term
+    size = torch.stack([xd[i].abs() @ wd.abs().t() for i in range(m)]) + term.abs()
+    bound = size * 2.0 ** -20 + (ref.abs() * 2.0 ** -7 if form == 0 else 0)
+    assert ((y.double() - ref).abs() <= bound).all()
