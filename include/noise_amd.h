@@ -356,13 +356,18 @@ int noise_pop_block_qkv(const noise_population_t *pop, noise_view_t y, const voi
 
 /* DUST's jitter on a population block (block_forward, run.py:102-117, for the block a rerun enters at): bf16 rows
  * [members * tokens][2048] added to mlp.c_fc's product before ReLU^2 (fc) and [members * tokens][512] added to
- * mlp.c_proj's product (mlp), either may be NULL (not both); zero_row is no longer read and may be NULL. The attention-output and attn.c_proj jitter go in before the call
+ * mlp.c_proj's product (mlp), either may be NULL (not both); without mlp rows, zero_row is 512 zero bf16 values
+ * (16 B aligned) the kernel reads instead. The attention-output and attn.c_proj jitter go in before the call
  * (noise_add_bf16 on y, noise_block_entry's residual). */
 typedef struct {
     const void *fc;
     const void *mlp;
     const void *zero_row;
 } noise_block_jitter_t;
+
+/* *row: 512 zero bf16 values (16 B aligned) in the current device's memory for noise_block_jitter_t's zero_row. They are
+ * the library's own, never written, and may be read on any stream and under capture. */
+int noise_zero_row(const void **row);
 
 /* noise_pop_block / noise_pop_block_qkv for an unperturbed block with jitter (no rank-1 or mixing-scalar noise,
  * no next-matrix dots; no counterpart in the reference beyond block_forward's jitter arguments): the last block

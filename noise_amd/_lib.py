@@ -57,3 +57,11 @@ def head_workspace(members, tokens, K, vocab, device):
     if need < 0:
         raise RuntimeError(lib().noise_last_error().decode(errors='replace'))
     return (torch.empty(need, dtype=torch.uint8, device=device) if need else None), need
+
+
+def zero_row(device):
+    """Address of 512 zero bf16 values on `device` that any stream may read (noise_zero_row)."""
+    row = ctypes.c_void_p()
+    with torch.cuda.device(device):
+        call('noise_zero_row', ctypes.byref(row))
+    return row.value

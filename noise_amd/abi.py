@@ -44,6 +44,7 @@ SIGNATURES = {
     'noise_pop_block_qkv_split': [_p, 'View', _p, _p, _p, _i64, 'View', _p, _p, _p, _p, _p, _i32, _p, _p, _p, _p, _i64,
                                   'View', _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p],
     'noise_block_weight_layout': [_p, _p, _i64, _i64, _p],
+    'noise_zero_row': [_p],
     'noise_weights_prepare': [_p, _i32, _p],
     'noise_mlp_proj_layout': [_p, _p, _i64, _p],
     'noise_pop_linear': [_p, 'View', _p, _i64, _i64, _p, _p, _p, _i32, _i64, _i64, _p],
@@ -147,7 +148,7 @@ class CastHeads(ctypes.Structure):
 
 
 class BlockJitter(ctypes.Structure):
-    """noise_block_jitter_t: bf16 jitter rows added to mlp.c_fc's and mlp.c_proj's products (NULL: none); zero_row is not read."""
+    """noise_block_jitter_t: bf16 jitter rows added to mlp.c_fc's and mlp.c_proj's products (NULL: none)."""
     _fields_ = [('fc', ctypes.c_void_p), ('mlp', ctypes.c_void_p), ('zero_row', ctypes.c_void_p)]
 
 

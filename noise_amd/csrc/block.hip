@@ -104,13 +104,13 @@ struct BlockArgs {
     float *ndots;                          // [rows][NNEXT]
     QkvRowsArgs q;                         // the next block's q/k/v (QKV): its x is h, its dots come from the epilogue
     const __bf16 *jfc;                     // JIT: mlp.c_fc jitter bf16 [m * T][2048] (added before ReLU^2) or NULL
-    const __bf16 *jmlp;                    // JIT: mlp.c_proj jitter bf16 [m * T][512] (added to its product) or NULL
+    const __bf16 *jmlp;                    // JIT: mlp.c_proj jitter bf16, row r at r * jmlp_st (added to its product)
+    int64_t jmlp_st;                       //   512, or 0 with one zero row when the block has no mlp.c_proj jitter
 };
 
-// The row a jittered block without mlp.c_proj jitter reads: zeros of the library's own image, never written and in place
-// on every device before any stream runs. (Loads under a condition instead made the jittered kernels spill 97 to 106
-// registers; this way they keep their 241 to 256 and spill none.)
-__device__ __attribute__((aligned(16))) __bf16 kNoJitter[kModel];
+// noise_zero_row's zeros: part of the library's image, never written and in place on every device before any stream
+// runs, so that every stream may read them
+__device__ __attribute__((aligned(16))) __bf16 kZeroRow[kModel];
 
 // sum over the four lanes holding one token's features (l % 16 + 16 g)
 __device__ __forceinline__ float token_sum(float v) { return sum_lanes_16_32(v); }
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(kBlkThreads, 1) void block_kernel(BlockArgs p) {
     {
         const float *apj = reinterpret_cast<const float *>(lds + kVApj) + 4 * g;
         const float *zr = MIX ? p.x0 + m * p.x0_m + (int64_t)tok * p.x0_t + 4 * g : nullptr;
-        const __bf16 *jr = kJit ? (p.jmlp ? p.jmlp + row * kModel : kNoJitter) + 4 * g : nullptr;
+        const __bf16 *jr = kJit ? p.jmlp + row * p.jmlp_st + 4 * g : nullptr;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             float4 zv[8];
@@ -724,7 +724,16 @@ int block_jitter(const char *fn, BlockArgs &a, const noise_block_jitter_t *jit) 
                     "%s: a jittered block takes no rank-1 or mixing-scalar noise", fn);
     NOISE_CHECK_ARG((!jit->fc || aligned(jit->fc, 16)) && (!jit->mlp || aligned(jit->mlp, 16)),
                     "%s: jitter rows must be 16 B aligned", fn);
+    // no mlp.c_proj jitter: every row reads one zero row (the kernel's epilogue loads unconditionally: under a condition
+    // the jittered kernels spill 97 to 106 registers instead of none)
     a.jmlp = (const __bf16 *)jit->mlp;
+    a.jmlp_st = kModel;
+    if (!a.jmlp) {
+        NOISE_CHECK_ARG(jit->zero_row && aligned(jit->zero_row, 16), "%s: without mlp jitter a 512-element zero row "
+                        "(bf16, 16 B aligned) must be given", fn);
+        a.jmlp = (const __bf16 *)jit->zero_row;
+        a.jmlp_st = 0;
+    }
     a.jfc = (const __bf16 *)jit->fc;   // each workgroup copies only its own token rows of it
     return NOISE_OK;
 }
@@ -858,6 +867,19 @@ extern "C" int noise_pop_block(const noise_population_t *pop, noise_view_t y, co
     return pop_block_impl("noise_pop_block", pop, y, w_o, r_o, o_dots, o_dots_n, xres, w_fc, r_fc, w_proj, r_proj,
                           xout, mix, lam_r, lam_x, eps_r, eps_x, eps_stride, x0, hout, split3, next, nnext, next_dots,
                           nullptr, stream);
+}
+
+extern "C" int noise_zero_row(const void **row) {
+    clear_error();
+    NOISE_CHECK_ARG(row, "noise_zero_row: row must not be NULL");
+    void *at = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&at, HIP_SYMBOL(kZeroRow));
+    if (e != hipSuccess) {
+        set_error("noise_zero_row: hipGetSymbolAddress: %s", hipGetErrorString(e));
+        return (int)e;
+    }
+    *row = at;
+    return NOISE_OK;
 }
 
 extern "C" int noise_pop_block_jit(const noise_population_t *pop, noise_view_t y, const void *w_o, noise_view_t xres,

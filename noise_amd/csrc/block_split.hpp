@@ -469,7 +469,7 @@ void split_tail_launch(const BlockArgs &a, bool mix, float *xout, void *workspac
     hipLaunchKernelGGL(split_fc_kernel, dim3((unsigned)part_grid(tiles, f.parts)), dim3(kBlkThreads), 0, s, f);
     r.x = hid; r.w = a.wpj; r.res = nullptr;
     r.a = a.apj; r.a_stride = a.apj_stride; r.b = a.bpj; r.b_stride = a.bpj_stride; r.dots = nullptr; r.ndots = 0;
-    r.jit = a.jmlp;
+    r.jit = a.jmlp_st ? a.jmlp : nullptr;  // (not the zero row)
     r.out = xout;
     r.mix = mix; r.lam_r = a.lam_r; r.lam_x = a.lam_x; r.eps_r = a.eps_r; r.eps_x = a.eps_x; r.eps_stride = a.eps_stride;
     r.x0 = a.x0; r.x0_m = a.x0_m; r.x0_t = a.x0_t;

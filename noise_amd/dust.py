@@ -160,7 +160,8 @@ def block_forward_eager(x, w, ve, cos, sin, window, o=None, attn=None, fc=None, 
         _lib.call('noise_add_bf16', y.data_ptr(), o.data_ptr(), y.numel(), stream)
     js = None
     if fc is not None or mlp is not None:
-        js = ctypes.byref(_lib.BlockJitter(_lib.ptr(fc), _lib.ptr(mlp), None))
+        zero = None if mlp is not None else _lib.zero_row(dev)
+        js = ctypes.byref(_lib.BlockJitter(_lib.ptr(fc), _lib.ptr(mlp), zero))
     split = _split_workspace(B, T, dev)
     _lib.call('noise_block_tail', pop, _lib.View(y.data_ptr(), T * C, C), ws['proj'].data_ptr(),
               _lib.View(xs.data_ptr(), T * C, C), ws['fc'].data_ptr(), ws['out'].data_ptr(), out.data_ptr(), js,

@@ -526,7 +526,8 @@ def blocks_forward(W, first, x_in, h_in, x0, idx, targets, rope=None, buffers=No
             if 'o' in jit:
                 _call('noise_add_bf16', B.y.data_ptr(), jit['o'].data_ptr(), B.y.numel(), stream)
             if 'fc' in jit or 'mlp' in jit:
-                js = _lib.BlockJitter(_lib.ptr(jit.get('fc')), _lib.ptr(jit.get('mlp')), None)
+                js = _lib.BlockJitter(_lib.ptr(jit.get('fc')), _lib.ptr(jit.get('mlp')),
+                                      None if 'mlp' in jit else _lib.zero_row(dev))
         yv, wo, wfc, wmp = _view(B.y, T * E, E), blk['o'].data_ptr(), blk['fc_blk'].data_ptr(), blk['mp_blk'].data_ptr()
         plain = (popp, yv, wo, ctypes.byref(none), B.d_attn.data_ptr(), N_HEAD, xres, wfc, ctypes.byref(none), wmp,
                  ctypes.byref(none))
