@@ -55,7 +55,12 @@ struct AttnArgs {
     float *dot;
     int64_t ds_b;
     int ddiv;
+    int first;                          // this launch's first workgroup
 };
+
+// A launch has fewer than 2^32 threads (one of more is cut short without an error): a call of more workgroups than this
+// goes in several launches. (A multiple of 8, so that a workgroup's XCD does not depend on its launch.)
+constexpr int64_t kLaunchGroups = 1 << 22;
 
 template <bool VT>
 __device__ __forceinline__ void load_tile_regs(const AttnArgs &a, const __bf16 *Kb, const __bf16 *Vb, int k0,
@@ -108,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void attention_fwd_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) __bf16 sV[2][kD][kLds];
 
     // workgroup -> (batch*head, query tile)
-    int wg = blockIdx.x;
+    int wg = a.first + blockIdx.x;
     int bh, qt;
     if (a.xcd_grouped) {
         int xcd = wg & 7, slot = wg >> 3;
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     constexpr int QB = 1, NW = QT / 32, QW = 32, CPW = 4;  // waves, queries per wave, copies per A wave
     __shared__ __attribute__((aligned(16))) char lds[NS * kStage];
 
-    int wg = blockIdx.x;
+    int wg = a.first + blockIdx.x;
     int bh, qt;
     if (a.tile_major) {
         // query tile descending, then head: with bh_total % 8 == 0 head bh still runs on XCD bh % 8
@@ -712,9 +717,10 @@ struct CastArgs {
     __bf16 *dst[3];
     int wide[3];       // 16 B aligned rows
     int64_t tokens, heads, chunks;
+    int64_t first;     // this launch's first workgroup
 };
 __global__ __launch_bounds__(256) void cast_heads_kernel(CastArgs p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = (p.first + blockIdx.x) * 256 + threadIdx.x;
     if (i >= p.chunks) return;
     const int k = blockIdx.y;
     const int64_t row = i >> 3, bt = row / p.heads, h = row - bt * p.heads, b = bt / p.tokens, t = bt - b * p.tokens;
@@ -794,8 +800,11 @@ extern "C" int noise_cast_heads(const noise_cast_heads_t *cast, int64_t batch, i
         p.s_b[i] = cast->s_b[i]; p.s_t[i] = cast->s_t[i]; p.s_h[i] = cast->s_h[i];
         p.wide[i] = aligned(cast->src[i], 16) && p.s_b[i] % 4 == 0 && p.s_t[i] % 4 == 0 && p.s_h[i] % 4 == 0;
     }
-    hipLaunchKernelGGL(cast_heads_kernel, dim3((unsigned)((p.chunks + 255) / 256), (unsigned)cast->count), dim3(256), 0,
-                       (hipStream_t)stream, p);
+    const int64_t groups = (p.chunks + 255) / 256;
+    for (p.first = 0; p.first < groups; p.first += kLaunchGroups) {
+        const int64_t n = groups - p.first < kLaunchGroups ? groups - p.first : kLaunchGroups;
+        hipLaunchKernelGGL(cast_heads_kernel, dim3((unsigned)n, (unsigned)cast->count), dim3(256), 0, (hipStream_t)stream, p);
+    }
     return launch_status(fn);
 }
 
@@ -861,18 +870,17 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     a.dvec = dot_vec; a.dot = dot_out; a.ds_b = dot_vec_stride; a.ddiv = (int)dot_div;
     // rows of RMS <= 1 (rounded to bf16): |q . k| <= D (1 + 2^-8)^2 < 1.0079 D
     a.shift = kD * fabsf(scale) * kLog2e * 1.0079f;
-    dim3 grid((unsigned)(bh * qtiles));
-    if (vt_path) {
-        const bool bounded = flags & NOISE_ATTN_QK_NORMED;
-        auto kernel = q_fp32 ? (bounded ? attention_vt_kernel<true, true, true, true>
-                                        : attention_vt_kernel<false, true, true, true>)
-                      : out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
-                      : v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
-                                   : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>);
-        hipLaunchKernelGGL(kernel, grid, dim3(512), 0, (hipStream_t)stream, a);
-    } else if (v_transposed)
-        hipLaunchKernelGGL(attention_fwd_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL(attention_fwd_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, a);
+    hipStream_t st = (hipStream_t)stream;
+    const bool bounded = flags & NOISE_ATTN_QK_NORMED;
+    auto ring = q_fp32 ? (bounded ? attention_vt_kernel<true, true, true, true> : attention_vt_kernel<false, true, true, true>)
+                : out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
+                : v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
+                               : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>);
+    auto kernel = vt_path ? ring : v_transposed ? attention_fwd_kernel<true> : attention_fwd_kernel<false>;
+    for (int64_t first = 0; first < bh * qtiles; first += kLaunchGroups) {
+        const int64_t n = bh * qtiles - first;
+        a.first = (int)first;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(n < kLaunchGroups ? n : kLaunchGroups)), dim3(vt_path ? 512 : 256), 0, st, a);
+    }
     return launch_status("noise_attention_fwd");
 }

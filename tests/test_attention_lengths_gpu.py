@@ -92,3 +92,40 @@ def test_fp32_queries(T, flags):
         call(odd, flags, torch.float32)
     for t in (q, odd):
         assert torch.equal(attention(t, k, v, 77), attention(t.bfloat16().contiguous(), k, v, 77).float())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_more_workgroups_than_one_launch(dtype):
+    """2^23 heads and more, of one workgroup of 512 threads each: a launch has fewer than 2^32 threads. A lone token's output
+    is its v, a second token's the softmax of two scores."""
+    from noise_amd.model import attention
+    B, H = 2 ** 20 + 1, 8
+    print(B, H, dtype, flush=True)
+    g = torch.Generator(DEV).manual_seed(3)
+    q, k, v = (torch.randn(B, 1, H, 64, device=DEV, generator=g).to(dtype) for _ in range(3))
+    assert torch.equal(attention(q, k, v, 5), v.bfloat16().to(dtype))
+    few = (torch.randn(B // 64, 2, H, 64, device=DEV, generator=g).to(dtype) for _ in range(3))
+    q, k, v = (t.repeat(64, 1, 1, 1) for t in few)
+    n = B // 64
+    want = attention(q[:n], k[:n], v[:n], 5)
+    rel_ok(want[:64], fp32_reference_gpu(*(t[:64].bfloat16() for t in (q, k, v)), 5))
+    out = attention(q, k, v, 5)
+    assert out.view(64, n, 2, H, 64).eq(want).all()
+
+
+def test_more_rows_than_one_cast_launch():
+    """2^29 rows and more, eight threads each. Every batch of the source is the same rows."""
+    import ctypes
+    from noise_amd import _lib
+    batch, H = 2 ** 26 + 1, 8
+    print(batch, H, flush=True)
+    src = torch.randn(1, 1, H, 64, device=DEV)
+    dst = torch.empty(batch, H, 64, device=DEV, dtype=torch.bfloat16)
+    dst[-4096:] = 9
+    cast = _lib.CastHeads()
+    cast.count, cast.src[0], cast.dst[0], cast.s_h[0] = 1, src.data_ptr(), dst.data_ptr(), 64
+    _lib.call('noise_cast_heads', ctypes.byref(cast), batch, 1, H, _lib.stream_ptr(DEV))
+    for part in (dst[:4096], dst[batch // 2:][:4096], dst[-4096:]):
+        assert part.eq(src[0].bfloat16()).all()
+    del dst, part
+    torch.cuda.empty_cache()
