@@ -1,5 +1,7 @@
 // Row-wise kernels of the population forward: embedding entry, member dot products, loss reduction and
 // the split-bf16x3 operands of the fp32 head. One 64-lane wave per 512-wide row, 8 elements per lane.
+#include <algorithm>
+
 #include "common.hpp"
 #include "mfma.hpp"
 #include "tile.hpp"
@@ -393,6 +395,7 @@ __global__ __launch_bounds__(256) void lowrank_embed_kernel(float *out, const fl
 // members, reading each direction's a row (L2-resident) once for all of that direction's members, one
 // direction ahead. Each store instruction covers 1 KiB (fp32) of one output row, lane after lane: stores
 // whose lanes leave gaps (32 B per lane as two 16 B halves) measured 20% slower on this HBM-write stream.
+// Few tokens leave fewer tiles than CUs, so the directions are shared out too: blockIdx.y takes `dirs_per` of them.
 constexpr int kExpRows = 4, kExpCols = 1024;
 // DD: members per direction as a constant (2: antithetic pairs), or 0 to take dir_div at run time; FULL: every
 // tile has all its rows and every direction all its members (no guards between the stores)
@@ -402,7 +405,7 @@ __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y,
                                                            const float *__restrict__ dots, int64_t dots_stride,
                                                            const float *__restrict__ a, int64_t a_stride,
                                                            const float *__restrict__ sign, int members, int dir_div,
-                                                           int tokens, int width) {
+                                                           int tokens, int width, int dirs_per) {
     const int dd = DD ? DD : dir_div;
     const int col_tiles = (width + kExpCols - 1) / kExpCols;
     const int t0 = (blockIdx.x / col_tiles) * kExpRows;
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y,
 #pragma unroll
     for (int r = 0; r < kExpRows; ++r)
         bv[r] = r < rows ? ld4(base + (int64_t)(t0 + r) * width + n) : float4{0.f, 0.f, 0.f, 0.f};
-    const int dirs = (members + dd - 1) / dd;
+    const int first = blockIdx.y * dirs_per, dirs = min(first + dirs_per, (members + dd - 1) / dd);
     const int64_t mstride = (int64_t)tokens * width;
     float4 av[2];
     float dv[2][kExpRows];
@@ -438,8 +441,8 @@ __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y,
             }
         }
     };
-    fetch(0, 0);
-    for (int d0 = 0; d0 < dirs; d0 += 2) {
+    fetch(first, 0);
+    for (int d0 = first; d0 < dirs; d0 += 2) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int d = d0 + u;
@@ -492,14 +495,17 @@ extern "C" int noise_rank1_expand(const noise_population_t *pop, const float *ba
                     "%s: alignment", fn);
     const int64_t tiles = (pop->tokens + kExpRows - 1) / kExpRows * ((width + kExpCols - 1) / kExpCols);
     NOISE_CHECK_ARG(tiles <= INT32_MAX, "%s: too many tiles", fn);
-    const dim3 grid((unsigned)tiles), block(256);
+    // below a tile per CU, parts of the directions (none empty) until 1024 workgroups are in the launch: lowrank of 4000
+    // members on 2 shared rows, 1024 -> 16, 867 us with one workgroup and 27 with 1000
+    const int64_t parts = tiles < 256 ? std::min<int64_t>(dirs, 1024 / tiles) : 1, per = (dirs + parts - 1) / parts;
+    const dim3 grid((unsigned)tiles, (unsigned)((dirs + per - 1) / per)), block(256);
     const int rd = y_fp32 == 2;
     const int m = (int)pop->members, dd = (int)pop->dir_div, T = (int)pop->tokens, W = (int)width;
     hipStream_t st = (hipStream_t)stream;
     const bool full = T % kExpRows == 0 && m % dd == 0;
 #define NOISE_EXPAND(DD, F, FULL)                                                                                    \
     hipLaunchKernelGGL((rank1_expand_kernel<DD, F, FULL>), grid, block, 0, st, y, rd, base, dots, dots_stride, r1->a, \
-                       r1->a_stride, pop->sign, m, dd, T, W)
+                       r1->a_stride, pop->sign, m, dd, T, W, (int)per)
     if (dd == 2 && y_fp32 && full) NOISE_EXPAND(2, true, true);
     else if (dd == 2 && y_fp32) NOISE_EXPAND(2, true, false);
     else if (dd == 2 && full) NOISE_EXPAND(2, false, true);

@@ -71,6 +71,34 @@ def test_lowrank_views():
           torch.randn(6, 40, device=DEV), sign, 1)             # shared, no unit inner stride, outputs off the groups of 4
 
 
+@pytest.mark.parametrize('m,T,n_in,n_out,div', [(1301, 2, 320, 20, 1), (1301, 5, 512, 4, 2), (1027, 3, 64, 1040, 3), (9, 1, 300, 8, 2),
+                                                (2049, 129, 128, 32, 2)])
+def test_shared_rows_of_few_tokens(m, T, n_in, n_out, div):
+    """Few token tiles: the expansion's directions are shared out over workgroups, the last of them with fewer."""
+    x, w, a, b, sign = inputs(m, T, n_in, n_out, div, torch.bfloat16, m + T)
+    check(x[:1].expand(m, T, n_in), w, a, b, sign, div)
+
+
+def test_shared_rows_of_few_tokens_take_no_longer_than_copies():
+    """4,000 members on two shared rows: one workgroup that walks all of them took 20 times the call on copied rows."""
+    from noise_amd.eggroll import lowrank
+    x, w, a, b, sign = inputs(4000, 2, 1024, 16, 2, torch.bfloat16, 1)
+
+    def ms(v):
+        times = []
+        for _ in range(7):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(20):
+                lowrank(v, w, a, b, sign, dir_div=2)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return sorted(times)[3]
+
+    assert ms(x[:1].expand(4000, 2, 1024)) <= 4 * ms(x)
+
+
 @pytest.mark.parametrize('m,n_in,n_out', [(65537, 32, 18), (2 ** 19 + 1, 32, 1), (2 ** 19 + 1, 8, 7)])
 def test_more_rows_than_one_launch_has_waves(m, n_in, n_out):
     """1024 rows per member, past 2^26 rows for the operands' wave per row and 2^29 for the narrow form's eight lanes per row:
