@@ -315,8 +315,10 @@ __device__ __forceinline__ int key_sigma(int i) { return (i & ~12) | ((i & 4) <<
 // QF32: fp32 queries, rounded as they are read. Each is read once, so casting them beforehand as K and V are (which
 // every query tile reads again) only adds a write and a read: 5 x 8 heads x 1111 tokens, the cast 10.4 -> 8.1 us, this
 // kernel 22 -> 23, the call 30.9 -> 29.1
-template <bool BOUNDED, bool VNAT, bool OF32 = false, bool QF32 = false>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_vt_kernel(AttnArgs a) {
+// RAGGED: any length (with VNAT); else lengths in whole 256-query tiles, without the clamps (24 x 8 heads x 2048 tokens, window
+// 64: 43.3 us with them, 41.9 without; a window of 16, 45.0 and 43.7)
+template <bool BOUNDED, bool VNAT, bool OF32, bool QF32, bool RAGGED>
+__device__ __forceinline__ void attention_ring(const AttnArgs &a) {
     constexpr int QT = kVtQT, NS = 4;
     constexpr int QB = 1, NW = QT / 32, QW = 32, CPW = 4;  // waves, queries per wave, copies per A wave
     __shared__ __attribute__((aligned(16))) char lds[NS * kStage];
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int j = lane & 31, hf = lane >> 5;
     const int T = a.seq, W = a.window;
     const int q0w = qt * QT + wave * QW;
-    // VNAT takes any length: rows past the last token are the last token's (queries there are not stored, and keys there
+    // RAGGED: rows past the last token are the last token's (queries there are not stored, and keys there
     // are visible to no query before them)
     const int last = T - 1;
 
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int q = q0w + 32 * qb + j;
-            const int64_t at = (int64_t)(VNAT && q > last ? last : q) * a.qs_t + 16 * s + 8 * hf;
+            const int64_t at = (int64_t)(RAGGED && q > last ? last : q) * a.qs_t + 16 * s + 8 * hf;
             if constexpr (QF32) {
                 const float *qp = reinterpret_cast<const float *>(a.q) + b * a.qs_b + h * a.qs_h + at;
                 const float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const unsigned voff = (unsigned)((lane >> 3) * a.vs_x * 2 + vchunk * 16);
     const unsigned lb = lds_addr(lds);
     auto issue = [&](int k0, unsigned st) {  // st: LDS byte address of the stage
-        if (VNAT && k0 + kBKV > T) {
+        if (RAGGED && k0 + kBKV > T) {
             // the tile that holds the last token: each lane's row is clamped (row strides below 2^25 elements)
 #pragma unroll
             for (int i = 0; i < CPW; ++i) {
@@ -442,12 +444,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
 
     const int wg_q_lo = qt * QT;
-    const int wg_q_hi = VNAT ? min(wg_q_lo + QT - 1, last) : wg_q_lo + QT - 1;
+    const int wg_q_hi = RAGGED ? min(wg_q_lo + QT - 1, last) : wg_q_lo + QT - 1;
     const int kv_first = max(0, wg_q_lo - W) / kBKV;
     const int kv_last = wg_q_hi / kBKV;
     const int nt = kv_last - kv_first + 1;
     // (a wave whose queries all lie past the last token has no active tile)
-    const int wq_lo = q0w, wq_hi = VNAT ? (q0w > last ? -1 : min(q0w + QW - 1, last)) : q0w + QW - 1;
+    const int wq_lo = q0w, wq_hi = RAGGED ? (q0w > last ? -1 : min(q0w + QW - 1, last)) : q0w + QW - 1;
     const float c2 = a.scale_log2, shift = a.shift;
 
     f32x16 sc[2][QB];
@@ -660,13 +662,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
             for (int it = 0; it < 8; ++it) {
                 const int r = 4 * it + (lane >> 4), ch = lane & 15;
-                if (q0w + r <= last)
+                if (!RAGGED || q0w + r <= last)
                     *reinterpret_cast<float4 *>(ob + (int64_t)(q0w + r) * a.os_t + 4 * ch) =
                         *reinterpret_cast<const float4 *>(stg + r * 256 + ((ch ^ (r & 15)) << 4));
             }
         } else {
             __bf16 *orow = a.o + b * a.os_b + h * a.os_h + (int64_t)q * a.os_t;
-            const bool live = !VNAT || q <= last;
+            const bool live = !RAGGED || q <= last;
             // with 16 B aligned output rows the wave's 32 x 64 block is staged in LDS (the K / V ring, free once
             // both groups are past their last tile) and stored as whole 128 B row segments: in the MFMA layout
             // one 8 B store would touch 32 rows
@@ -695,19 +697,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
                 for (int it = 0; it < 4; ++it) {
                     const int c = it * 64 + lane, r = c >> 3, ch = c & 7;
-                    if (!VNAT || q0w + 32 * qb + r <= last)
+                    if (!RAGGED || q0w + 32 * qb + r <= last)
                         store_bf16x8(ob + (int64_t)r * a.os_t + ch * 8, load_bf16x8(stg + r * kOP + ch * 8));
                 }
             }
         }
         if (a.dot) {
             dsum += swap_halves(dsum);
-            if (hf == 0 && (!VNAT || q <= last)) a.dot[((int64_t)b * T + q) * a.heads + h] = dsum;
+            if (hf == 0 && (!RAGGED || q <= last)) a.dot[((int64_t)b * T + q) * a.heads + h] = dsum;
         }
     }
 }
 
+template <bool BOUNDED, bool VNAT, bool OF32 = false, bool QF32 = false>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_vt_kernel(AttnArgs a) {
+    attention_ring<BOUNDED, VNAT, OF32, QF32, false>(a);
+}
 
+template <bool BOUNDED, bool OF32 = false, bool QF32 = false>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_ragged_kernel(AttnArgs a) {
+    attention_ring<BOUNDED, true, OF32, QF32, true>(a);
+}
 
 // Up to three fp32 tensors [b, t, h, 64] (unit inner stride) -> bf16 [b][t][h][64] contiguous, 8 dims per thread.
 // grid = (chunks / 256, tensors)
@@ -872,10 +882,14 @@ extern "C" int noise_attention_fwd(const void *q, const void *k, const void *v, 
     a.shift = kD * fabsf(scale) * kLog2e * 1.0079f;
     hipStream_t st = (hipStream_t)stream;
     const bool bounded = flags & NOISE_ATTN_QK_NORMED;
-    auto ring = q_fp32 ? (bounded ? attention_vt_kernel<true, true, true, true> : attention_vt_kernel<false, true, true, true>)
-                : out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
-                : v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
-                               : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>);
+    auto ring = v_transposed ? (bounded ? attention_vt_kernel<true, false> : attention_vt_kernel<false, false>)
+                : seq % kVtQT == 0
+                    ? (q_fp32 ? (bounded ? attention_vt_kernel<true, true, true, true> : attention_vt_kernel<false, true, true, true>)
+                       : out_fp32 ? (bounded ? attention_vt_kernel<true, true, true> : attention_vt_kernel<false, true, true>)
+                                  : (bounded ? attention_vt_kernel<true, true> : attention_vt_kernel<false, true>))
+                    : (q_fp32 ? (bounded ? attention_ragged_kernel<true, true, true> : attention_ragged_kernel<false, true, true>)
+                       : out_fp32 ? (bounded ? attention_ragged_kernel<true, true> : attention_ragged_kernel<false, true>)
+                                  : (bounded ? attention_ragged_kernel<true> : attention_ragged_kernel<false>));
     auto kernel = vt_path ? ring : v_transposed ? attention_fwd_kernel<true> : attention_fwd_kernel<false>;
     for (int64_t first = 0; first < bh * qtiles; first += kLaunchGroups) {
         const int64_t n = bh * qtiles - first;

@@ -129,3 +129,15 @@ def test_more_rows_than_one_cast_launch():
         assert part.eq(src[0].bfloat16()).all()
     del dst, part
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize('T', [256, 512, 768])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_whole_tiles(T, dtype):
+    """Lengths in whole 256-query tiles, without the clamps, give the bits of the same tokens with one more behind them."""
+    from noise_amd.model import attention
+    test_lengths(T, dtype)
+    g = torch.Generator(DEV).manual_seed(T)
+    for window in (0, 100, 4096):
+        q, k, v = (torch.randn(2, T + 1, 3, 64, device=DEV, generator=g).to(dtype) for _ in range(3))
+        assert torch.equal(attention(q[:, :T], k[:, :T], v[:, :T], window), attention(q, k, v, window)[:, :T])
