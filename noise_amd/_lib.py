@@ -3,6 +3,7 @@
 There is no fallback: if the library is missing or does not load, every op raises.
 """
 import ctypes
+import functools
 from pathlib import Path
 
 import torch
@@ -59,8 +60,10 @@ def head_workspace(members, tokens, K, vocab, device):
     return (torch.empty(need, dtype=torch.uint8, device=device) if need else None), need
 
 
+@functools.lru_cache(maxsize=None)
 def zero_row(device):
-    """Address of 512 zero bf16 values on `device` that any stream may read (noise_zero_row)."""
+    """Address of 512 zero bf16 values on `device` that any stream may read (noise_zero_row). It is part of the loaded
+    library, the same for the life of the process."""
     row = ctypes.c_void_p()
     with torch.cuda.device(device):
         call('noise_zero_row', ctypes.byref(row))

@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256) void lowrank_embed_kernel(float *out, const fl
 // Few tokens leave fewer tiles than CUs, so the directions are shared out too: blockIdx.y takes `dirs_per` of them.
 constexpr int kExpRows = 4, kExpCols = 1024;
 // DD: members per direction as a constant (2: antithetic pairs), or 0 to take dir_div at run time; FULL: every
-// tile has all its rows and every direction all its members (no guards between the stores)
+// tile has all its rows and every direction all its members (no guards between the stores), in one part
 template <int DD, bool F32, bool FULL>
 __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y, int round_dot,
                                                            const float *__restrict__ base,
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256) void rank1_expand_kernel(void *__restrict__ y,
 #pragma unroll
     for (int r = 0; r < kExpRows; ++r)
         bv[r] = r < rows ? ld4(base + (int64_t)(t0 + r) * width + n) : float4{0.f, 0.f, 0.f, 0.f};
-    const int first = blockIdx.y * dirs_per, dirs = min(first + dirs_per, (members + dd - 1) / dd);
+    const int first = FULL ? 0 : blockIdx.y * dirs_per, all = (members + dd - 1) / dd, dirs = FULL ? all : min(first + dirs_per, all);
     const int64_t mstride = (int64_t)tokens * width;
     float4 av[2];
     float dv[2][kExpRows];
@@ -502,7 +502,7 @@ extern "C" int noise_rank1_expand(const noise_population_t *pop, const float *ba
     const int rd = y_fp32 == 2;
     const int m = (int)pop->members, dd = (int)pop->dir_div, T = (int)pop->tokens, W = (int)width;
     hipStream_t st = (hipStream_t)stream;
-    const bool full = T % kExpRows == 0 && m % dd == 0;
+    const bool full = grid.y == 1 && T % kExpRows == 0 && m % dd == 0;
 #define NOISE_EXPAND(DD, F, FULL)                                                                                    \
     hipLaunchKernelGGL((rank1_expand_kernel<DD, F, FULL>), grid, block, 0, st, y, rd, base, dots, dots_stride, r1->a, \
                        r1->a_stride, pop->sign, m, dd, T, W, (int)per)
